@@ -758,6 +758,15 @@ __device__ __forceinline__ double rsq(double x) {
  * kernel evaluates the same form and branch from the same FP64 symbols, so the
  * basis is consistent; other grids keep the reference's arithmetic, whose
  * register footprint matters in the FP32 inner kernels.                     */
+/* 3 Lq - |S|^2 as |d|^2, d = (Lz - Ly, Lx - Lz, Ly - Lx): near L parallel to (1, 1, 1)
+ * the difference loses up to 6 digits (FCC 96), by other amounts in every
+ * kernel that sums in another order, and the basis has to be the same in all
+ * of them; the sum of squares is accurate to a few ulp in any order          */
+__device__ __forceinline__ double pi_d2_general(double2 lx, double2 ly, double2 lz) {
+    const double2 d1 = csub(lz, ly), d2 = csub(lx, lz), d3 = csub(ly, lx);
+    return d1.x * d1.x + d1.y * d1.y + d2.x * d2.x + d2.y * d2.y + d3.x * d3.x + d3.y * d3.y;
+}
+
 template <bool FAST = false, bool GUARD = false>
 __device__ __forceinline__ void pi_basis(const GridDev& g, double2 lx, double2 ly, double2 lz,
                                          double2 p1[3], double2 p2[3]) {
@@ -778,9 +787,8 @@ __device__ __forceinline__ void pi_basis(const GridDev& g, double2 lx, double2 l
         }
     } else if (g.general) {
         const double2 Ls = cadd(cadd(lx, ly), lz);
-        const double Lp = Ls.x * Ls.x + Ls.y * Ls.y;
-        const double i1 = rsq<FAST>(3.0 * Lq * Lq - Lq * Lp);
-        const double i2 = rsq<FAST>(3.0 * Lq - Lp);
+        const double i2 = rsq<FAST>(pi_d2_general(lx, ly, lz));
+        const double i1 = i2 * rsq<FAST>(Lq);
         const double2 lxs = cmulc(lx, Ls), lys = cmulc(ly, Ls), lzs = cmulc(lz, Ls);
         p1[0] = make_double2((Lq - lxs.x) * i1, -lxs.y * i1);
         p1[1] = make_double2((Lq - lys.x) * i1, -lys.y * i1);
@@ -818,9 +826,8 @@ __device__ __forceinline__ void pi_norms_general(double2 lx, double2 ly, double2
                                                  double& i1, double& i2) {
     Lq = lx.x * lx.x + lx.y * lx.y + ly.x * ly.x + ly.y * ly.y + lz.x * lz.x + lz.y * lz.y;
     Ls = cadd(cadd(lx, ly), lz);
-    const double Lp = Ls.x * Ls.x + Ls.y * Ls.y;
-    i1 = rsq<FAST>(3.0 * Lq * Lq - Lq * Lp);
-    i2 = rsq<FAST>(3.0 * Lq - Lp);
+    i2 = rsq<FAST>(pi_d2_general(lx, ly, lz));
+    i1 = i2 * rsq<FAST>(Lq);
 }
 template <bool FAST>
 __device__ __forceinline__ void pi_expand_general(double2 lx, double2 ly, double2 lz, double2 x1, double2 x2,

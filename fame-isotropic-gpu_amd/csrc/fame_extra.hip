@@ -273,9 +273,21 @@ extern "C" fame_status fame_time_qbq_passes(fame_ctx* c, int prec, int reps, dou
     const KAxis ko = c->kout(prec, 0, nullptr, LIST_EPS);
     ki.x = x; ki.pikind = 0;
     kf.y = y; kf.pikind = 0;
+    /* the plane path has one kernel between the inner ones, timed as entry 2 */
+    const bool pln = c->plane[prec == 8 ? 0 : 1];
+    KLine kl, kc2;
+    KPlane kp;
+    if (pln) { kl = c->kline(prec, 0, nullptr); kc2 = c->kline(prec, 0, nullptr, true); kp = c->kplane(prec, 0, nullptr); kl.x = x; kc2.xs = y; }
     for (int which = 0; which < 6; ++which) {
+        if (pln && (which == 1 || which == 3)) { us6[which] = 0.0; continue; }
         for (int rep = -1; rep < reps; ++rep) {
             if (rep == 0) HIPCHK(hipEventRecord(e0, c->stream));
+            if (pln && which != 5) {
+                if (which == 0) HIPCHK(c->launch_line(kl, 1, LINE_EX_PLAIN, prec, nk));
+                else if (which == 2) HIPCHK(c->launch_plane(kp, prec, nk));
+                else HIPCHK(c->launch_line(kc2, 0, LINE_CO_PLAIN, prec, nk));
+                continue;
+            }
             switch (which) {
                 case 0: HIPCHK(fame_launch_inner(ki, 1, prec, nk, c->stream)); break;
                 case 1: HIPCHK(fame_launch_mid(kmi, +1, prec, nk, c->stream)); break;
@@ -332,7 +344,17 @@ extern "C" fame_status fame_time_cg_passes(fame_ctx* c, int prec, int reps, doub
     KInner kc = c->kin(prec, 0, c->active, LIST_FWD);
     kc.x = pv; kc.y = r; kc.pikind = 0;
     kc.cg_r = r; kc.cgsc = c->cgsc; kc.partials = c->partials2;
-    const int nbi = c->nblk_in[prec == 8 ? 0 : 1];
+    const int nbi = c->inner_blocks(prec);
+    const bool pln = c->plane[prec == 8 ? 0 : 1];
+    KLine kl, kc2;
+    KPlane kp;
+    if (pln) {
+        kl = c->kline(prec, 0, c->active); kp = c->kplane(prec, 0, c->active);
+        kl.x = pv; kl.r = r; kl.xs = x; kl.cgsc = c->cgsc;
+        kc2 = c->kline(prec, 0, c->active, true);
+        kc2.r = r; kc2.cgsc = c->cgsc; kc2.rpart = c->partials2 + 3; kc2.rstep = 6;
+        kp.pap = c->pap_part;
+    }
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
@@ -345,8 +367,15 @@ extern "C" fame_status fame_time_cg_passes(fame_ctx* c, int prec, int reps, doub
         HIPCHK(fame_cg_begin(x, r, pv, b, c->partials, NBLK_VEC, st, st, nk, prec, nullptr, c->stream));
         HIPCHK(fame_cg_init_scal2(c->cgsc, c->partials, NBLK_VEC, 0.0, 0.0, 1 << 30, nk, c->active, nullptr, c->stream));
         CHK(c->cg_step_rc(prec, pv, r, x, 0, nk, npap));
+        if (pln && (which == 1 || which == 4)) { us8[which] = 0.0; continue; }
         for (int rep = -1; rep < reps; ++rep) {
             if (rep == 0) HIPCHK(hipEventRecord(e0, c->stream));
+            if (pln && (which == 0 || which == 2 || which == 5)) {
+                if (which == 0) HIPCHK(c->launch_line(kl, 1, LINE_EX_CG, prec, nk));
+                else if (which == 2) HIPCHK(c->launch_plane(kp, prec, nk));
+                else HIPCHK(c->launch_line(kc2, 0, LINE_CO_CG, prec, nk));
+                continue;
+            }
             switch (which) {
                 case 0: HIPCHK(fame_launch_inner(ki, 1, prec, nk, c->stream)); break;
                 case 1: HIPCHK(fame_launch_mid(kmi, +1, prec, nk, c->stream)); break;

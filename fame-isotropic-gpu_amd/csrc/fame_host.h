@@ -9,6 +9,9 @@
 #include "fame_hip.h"
 #include "fame_kernels.h"
 
+/* contraction and expansion modes of the plane path (fame_plane.hpp) */
+enum { LINE_EX_PLAIN = 0, LINE_EX_CG = 1, LINE_EX_FX = 2, LINE_CO_PLAIN = 0, LINE_CO_CG = 1, LINE_CO_RES = 2 };
+
 #define NBLK_VEC 1024   /* blocks per problem of the vector/reduction kernels */
 #define CG_GRAPH_ITERS 4   /* CG iterations per captured graph (fewer launch gaps between them) */
 
@@ -23,6 +26,8 @@ struct AxisPlan {
     fame::LinePlanDev lists[2][NLIST];   /* [0] FP64, [1] FP32; LIST_* stage lists */
     int cap[2] = {0, 0};                 /* elements a 256-thread block transforms at once */
     std::vector<void*> bufs;
+    const PlaneStage* pst[2] = {nullptr, nullptr};  /* passes of the plane kernels: nst, then nst reversed */
+    const void* afrag[2] = {nullptr, nullptr};   /* direct DFT: A operand fragments of the plane kernels */
     fame_status build(int n, int engine);
     ~AxisPlan();
 };
@@ -44,6 +49,16 @@ struct fame_ctx {
     /* permittivity, kernel layout */
     double* invB64 = nullptr; float* invB32 = nullptr; double* eps_int = nullptr; double* eps_ref = nullptr;
     bool have_eps = false;
+    /* plane path (fame_plane.hpp), per precision index: whether the grid has it,
+     * whether the solver takes it, the inner tiles (engine, lines per block) of
+     * its expanding and contracting kernels, the launch templates, its tables */
+    bool plane_ok[2] = {false, false}, plane[2] = {false, false};
+    PassTile ltile[2], ctile[2];
+    int PP = 0, CS = 0;           /* plane pitch and component stride (na PP)  */
+    PlaneAxis laxis[2][2];        /* inner axis [precision][engine], n = 0 when not available */
+    KPlane kpl[2];
+    void *invBp[2] = {nullptr, nullptr}, *ltw[2] = {nullptr, nullptr}, *mtw[2] = {nullptr, nullptr}, *eatab = nullptr;
+    LineTab* ltab = nullptr;
     /* wave vectors */
     int nk = 0;
     std::vector<fame::ProbDev> prob_h;
@@ -109,6 +124,13 @@ struct fame_ctx {
     fame_status cg_step_ap(int prec, void* p, void* r, void* x, void* Ap, int p0, int nprob);
     fame_status cg_step_rc(int prec, void* p, void* r, void* x, int p0, int nprob, int npap);
 
+    bool line_tile_ok(int prec, int eng, int L) const;
+    fame_status plane_setup();
+    KLine kline(int prec, int p0, const int* act, bool contract = false) const;
+    KPlane kplane(int prec, int p0, const int* act) const;
+    hipError_t launch_line(const KLine& k, int expand, int mode, int prec, int nprob);
+    hipError_t launch_plane(const KPlane& k, int prec, int nprob);
+    int inner_blocks(int prec) const;   /* blocks per problem whose sums the contracting pass leaves */
     KInner kin(int prec, int p0, const int* act, int list) const;
     KAxis kmid(int prec, int p0, const int* act, int list) const;
     KAxis kout(int prec, int p0, const int* act, int list) const;

@@ -81,6 +81,73 @@ struct KInner {
     int cgdots;
 };
 
+/* one axis of the plane kernels (fame_plane.hpp): Stockham passes, or a direct
+ * DFT on the matrix cores */
+struct PlaneStage {
+    int R, Ns, nb, tstep;        /* radix, radices before it, butterflies per line, twiddle step */
+    unsigned mNs;
+};
+struct PlaneAxis {
+    int n, eng, nst;
+    unsigned mnl;                /* udiv magic for / lines                      */
+    int ntab;                    /* entries of W, kept in LDS                   */
+    const void* W;               /* Stockham: exp(-2 pi i m / n), n entries; direct DFT: its
+                                    (cos, -sin) fragments [tile][K step][64]    */
+    /* device arrays: the passes of the inverse transform, and of the forward one
+     * (the radices in reverse order)                                          */
+    const PlaneStage* st;
+    const PlaneStage* sf;
+};
+
+/* constants of one line (b, c) of a wave vector: the symbols of the two outer
+ * axes, exp(i pi phi / na) of the inner phase, the symbols' sum, squared norm and
+ * squared distance                                                            */
+struct LineTab { double2 b, c, e, s; double q, d; };
+
+/* the inner-axis kernels of the plane path */
+struct KLine {
+    fame::GridDev g;
+    const fame::ProbDev* prob;
+    const int* active;
+    PlaneAxis a;
+    const LineTab* lt;           /* nb nc per problem                           */
+    const void* tw;              /* inner twiddle factors, inner_tw_per_line(na) per line */
+    const void* ea;              /* exp(i pi a / na), na complex doubles        */
+    void* f;                     /* field, plane layout [component][a][PP]      */
+    size_t fstride, xstride;
+    int PP, cs;                  /* plane pitch and component stride (na PP)    */
+    int L, P;                    /* lines per block, LDS line pitch             */
+    unsigned mLs;                /* udiv magic of the field accesses: / (L / 2) in FP32, / L in FP64 */
+    /* reduced vectors: mode f of the first half at [f - off], of the second at
+     * [half + f - off] (padded vectors: off 0, half N; the reference's layout at
+     * Gamma: off 1, half N - 1)                                              */
+    const void* x;
+    int half, off;
+    const double* sig;           /* expand, plain: x scaled by sig[f] (optional) */
+    void* r;                     /* CG residual; contract CO_RES: r32           */
+    void* xs;                    /* CG solution; contract: y, or x32 of CO_RES  */
+    const CgScal* cgsc;
+    const void* fx32;
+    const void* fp32;
+    const void* rb;
+    void* p32;
+    double* rpart;               /* contract: block sums of <r, r>, every rstep doubles */
+    int rstep;
+};
+struct KPlane {
+    fame::GridDev g;
+    const int* active;
+    void* f;
+    size_t fstride;
+    int PP;
+    const void* invB;            /* 1 / (N eps), plane layout                   */
+    const void* tw;              /* middle twiddles, nb nc per problem          */
+    double* pap;                 /* optional <v, eps^-1 v / N> per block, [problem][component][a] */
+    PlaneAxis b, c;
+    unsigned mnb;
+    int nprob, nt;
+};
+
 struct KAxis {
     fame::GridDev g;
     const fame::ProbDev* prob;
@@ -119,6 +186,24 @@ size_t fame_line_lds(const fame::LinePlanDev& pl, int prec, int nl, int P, int e
 hipError_t fame_launch_inner(const KInner& a, int expand, int prec, int nprob, hipStream_t s);
 hipError_t fame_launch_mid(const KAxis& a, int dir, int prec, int nprob, hipStream_t s);
 hipError_t fame_launch_outer(const KAxis& a, int mode, int prec, int nprob, hipStream_t s);
+/* dynamic LDS of one block that leaves a second one room on the CU (160 KiB,
+ * with the kernels' static LDS) */
+#define FAME_LDS_HALF (80 * 1024 - 256)
+/* LDS bytes of the plane path's kernels */
+inline size_t fame_plane_lds(int nb, int nc, int ntab, int prec) {
+    return (size_t)(prec == 8 ? 16 : 8) * ((size_t)ntab + (((size_t)nc * (nb | 1) + 1) & ~(size_t)1));
+}
+inline size_t fame_line_lds2(int na, int ntab, int L, int P, int prec) {
+    return 16 * (size_t)na + sizeof(LineTab) * L + (prec == 8 ? 16 : 8) * ((size_t)ntab + (size_t)L * inner_tw_per_line(na) + 3 * (size_t)L * P);
+}
+hipError_t fame_launch_line32(const KLine& k, int expand, int mode, int nprob, hipStream_t s);
+hipError_t fame_launch_line64(const KLine& k, int expand, int mode, int nprob, hipStream_t s);
+hipError_t fame_launch_plane32(const KPlane& k, int nprob, hipStream_t s);
+hipError_t fame_launch_plane64(const KPlane& k, int nprob, hipStream_t s);
+hipError_t fame_prepare_plane32(int eb, int ec, size_t lds);
+hipError_t fame_prepare_plane64(int eb, int ec, size_t lds);
+hipError_t fame_launch_line_tab(const fame::GridDev& g, const fame::ProbDev* prob, LineTab* lt, void* tw64, void* tw32,
+                                void* mid64, void* mid32, int nprob, hipStream_t s);
 hipError_t fame_launch_xz_transpose(const void* in, void* out, int nx, int ny, int nz, int dir, size_t stride,
                                     int ncomp, int nprob, int prec, hipStream_t s);
 hipError_t fame_launch_pack(const void* in, void* out, int N, int Nd, int dir, int prec, hipStream_t s);

@@ -339,10 +339,17 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         for (int pi = 0; pi < 2; ++pi)
             for (int a = 0; a < 3; ++a)
                 same = same && k->tile[a][pi].eng == c->tile[a][pi].eng && k->tile[a][pi].L == c->tile[a][pi].L;
+        for (int pi = 0; pi < 2; ++pi)
+            same = same && k->plane[pi] == c->plane[pi] && k->ltile[pi].eng == c->ltile[pi].eng && k->ltile[pi].L == c->ltile[pi].L &&
+                   k->ctile[pi].L == c->ctile[pi].L && k->kpl[pi].nt == c->kpl[pi].nt;
         if (!same) {
             for (int pi = 0; pi < 2; ++pi) {
                 for (int a = 0; a < 3; ++a) k->tile[a][pi] = c->tile[a][pi];
                 k->nblk_in[pi] = c->nblk_in[pi];
+                k->plane[pi] = c->plane[pi];
+                k->ltile[pi] = c->ltile[pi];
+                k->ctile[pi] = c->ctile[pi];
+                k->kpl[pi].nt = c->kpl[pi].nt;
             }
             k->drop_graphs();
         }

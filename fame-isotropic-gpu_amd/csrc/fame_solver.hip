@@ -214,6 +214,38 @@ fame_status AxisPlan::build(int n_, int engine) {
         CHK(upload(ch, prec, &base.chirp));
         CHK(upload(bm, prec, &base.bm));
         CHK(upload(bp, prec, &base.bp));
+        if (mfma) {
+            /* lane l of K step ks, tile w: row q = 16 w + l % 16, t = 4 ks + l / 16 + 1 */
+            const int m = (n - 1) / 2, Q = n / 2 + 1, nqt = (Q + 15) / 16, nks = std::max(1, (m + 3) / 4);
+            std::vector<cld> af((size_t)nqt * nks * 64, cld(0, 0));
+            for (int w = 0; w < nqt; ++w)
+                for (int ks = 0; ks < nks; ++ks)
+                    for (int l = 0; l < 64; ++l) {
+                        const int q = 16 * w + l % 16, t = 4 * ks + l / 16 + 1;
+                        if (q < Q && t <= m) af[((size_t)w * nks + ks) * 64 + l] = W[(size_t)q * t % n];
+                    }
+            CHK(upload(af, prec, &afrag[pi]));
+        }
+        if (!mfma && !blue) {
+            std::vector<PlaneStage> ps(2 * rads.size());
+            int Ns = 1, Nf = 1;
+            for (size_t i = 0; i < rads.size(); ++i) {
+                auto fill = [&](PlaneStage& t, int R, int ns) {
+                    t.R = R; t.Ns = ns; t.nb = n / R; t.tstep = n / (ns * R); t.mNs = fame_magic32(ns);
+                };
+                /* the inverse transform ends and the forward one begins with
+                 * the largest radix: the column pass between them runs both
+                 * butterflies on one LDS round trip                        */
+                const int Ri = rads[rads.size() - 1 - i];
+                fill(ps[i], Ri, Ns); Ns *= Ri;
+                fill(ps[rads.size() + i], rads[i], Nf); Nf *= rads[i];
+            }
+            void* d = nullptr;
+            HIPCHK(hipMalloc(&d, sizeof(PlaneStage) * std::max<size_t>(ps.size(), 1)));
+            bufs.push_back(d);
+            HIPCHK(hipMemcpy(d, ps.data(), sizeof(PlaneStage) * ps.size(), hipMemcpyHostToDevice));
+            pst[pi] = (const PlaneStage*)d;
+        }
         bool ok = true;
         for (int l = 0; l < NLIST && mfma; ++l) {
             LinePlanDev& d = lists[pi][l];
@@ -305,6 +337,120 @@ fame_ctx::~fame_ctx() {
     for (void* p : big) if (p) (void)hipFree(p);
 }
 
+/* lines per block of the plane path's inner kernels: FP32 moves pairs of lines,
+ * and a block's lines, constants and tables stay within 64 KiB of LDS */
+bool fame_ctx::line_tile_ok(int prec, int eng, int L) const {
+    const int pi = prec == 8 ? 0 : 1;
+    if (!plane_ok[pi] || eng < 0 || eng > 1 || laxis[pi][eng].n == 0 || L < 1 || L > MAX_LINES_INNER) return false;
+    if (prec == 4 && (L & 1)) return false;
+    return fame_line_lds2(g.na, laxis[pi][eng].ntab, L, g.na | 1, prec) <= 63 * 1024;
+}
+
+/* an axis of the plane path: its Stockham passes, or the direct DFT */
+static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q) {
+    std::memset(q, 0, sizeof(*q));
+    if (p.n < 2 || (eng == ENG_STOCKHAM ? p.blue != 0 : p.n < 8)) return false;
+    const LinePlanDev& d = p.lists[pi][LIST_FWD];
+    const int m = (p.n - 1) / 2, nqt = (p.n / 2 + 16) / 16;
+    q->eng = eng;
+    q->W = eng == ENG_MFMA ? p.afrag[pi] : d.W;
+    q->ntab = eng == ENG_MFMA ? nqt * ((m + 3) / 4) * 64 : p.n;
+    q->mnl = fame_magic32(nl);
+    if (eng == ENG_STOCKHAM) { q->nst = d.nst; q->st = p.pst[pi]; q->sf = p.pst[pi] + d.nst; }
+    q->n = p.n;
+    return true;
+}
+
+/* whether the grid has the plane path, per precision: no Bluestein axis (a
+ * length with a prime factor above 13 takes the direct DFT), and a plane
+ * within the LDS of a CU */
+fame_status fame_ctx::plane_setup() {
+    PP = (g.nb * g.nc + 15) & ~15;
+    CS = g.na * PP;
+    if (g.nb < 2 || g.nc < 2 || (long long)3 * CS >= (1LL << 31)) return FAME_OK;
+    for (int pi = 0; pi < 2; ++pi) {
+        const int prec = pi == 0 ? 8 : 4;
+        KPlane& k = kpl[pi];
+        std::memset(&k, 0, sizeof(k));
+        auto engine = [&](int axis) { return (ax[axis][0].blue || eng_forced == 1) ? ENG_MFMA : ENG_STOCKHAM; };
+        if (!plane_axis(ax[AX_MID][engine(AX_MID)], engine(AX_MID), pi, g.nc, &k.b)) continue;
+        if (!plane_axis(ax[AX_OUTER][engine(AX_OUTER)], engine(AX_OUTER), pi, g.nb, &k.c)) continue;
+        const size_t lds = fame_plane_lds(g.nb, g.nc, k.b.ntab + k.c.ntab, prec);
+        if (lds > 160 * 1024 - 256) continue;
+        k.g = g;
+        k.PP = PP;
+        k.mnb = fame_magic32(g.nb);
+        k.nt = lds > FAME_LDS_HALF ? (prec == 8 ? 512 : 1024) : lds > 24 * 1024 ? 512 : 256;
+        bool any = false;
+        for (int e = 0; e < 2; ++e) {
+            if (eng_forced >= 0 && e != eng_forced && !(eng_forced == 0 && ax[AX_INNER][0].blue)) { laxis[pi][e].n = 0; continue; }
+            if (!plane_axis(ax[AX_INNER][e], e, pi, 1, &laxis[pi][e])) laxis[pi][e].n = 0;
+            any = any || laxis[pi][e].n > 0;
+        }
+        if (!any) continue;
+        plane_ok[pi] = true;
+        const int eng = laxis[pi][0].n > 0 ? 0 : 1;
+        int L = prec == 4 ? 16 : 8;
+        while (L > 1 && !line_tile_ok(prec, eng, L)) L >>= 1;
+        if (!line_tile_ok(prec, eng, L)) { plane_ok[pi] = false; continue; }
+        ltile[pi].eng = eng; ltile[pi].L = L; ltile[pi].P = g.na | 1;
+        ctile[pi] = ltile[pi];
+        HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng, lds) : fame_prepare_plane32(k.b.eng, k.c.eng, lds));
+        /* before tuning: an FP64 plane that fills a CU alone pays where one
+         * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
+         * iteration in 112 us against 134 by axis passes; SC 96, 288 blocks: 193
+         * against 180)                                                        */
+        plane[pi] = prec == 4 || lds <= FAME_LDS_HALF || 3 * g.na <= 256;
+    }
+    return FAME_OK;
+}
+
+hipError_t fame_ctx::launch_line(const KLine& k, int expand, int mode, int prec, int nprob) {
+    return prec == 8 ? fame_launch_line64(k, expand, mode, nprob, stream) : fame_launch_line32(k, expand, mode, nprob, stream);
+}
+hipError_t fame_ctx::launch_plane(const KPlane& k, int prec, int nprob) {
+    return prec == 8 ? fame_launch_plane64(k, nprob, stream) : fame_launch_plane32(k, nprob, stream);
+}
+
+/* threads per block of the plane kernel (within its launch bounds) */
+static bool plane_threads_ok(int prec, int nt) { return nt == 256 || nt == 512 || nt == 1024; }
+
+KLine fame_ctx::kline(int prec, int p0, const int* act, bool contract) const {
+    const int pi = prec == 8 ? 0 : 1;
+    const size_t es = prec == 8 ? 16 : 8, nl = (size_t)g.nb * g.nc;
+    KLine k;
+    std::memset(&k, 0, sizeof(k));
+    const PassTile& t = contract ? ctile[pi] : ltile[pi];
+    k.g = g; k.prob = prob_d + p0; k.active = act;
+    k.a = laxis[pi][t.eng];
+    k.a.mnl = fame_magic32(3 * t.L);
+    k.lt = ltab + nl * p0;
+    k.tw = (char*)ltw[pi] + es * nl * inner_tw_per_line(g.na) * p0;
+    k.ea = eatab;
+    k.PP = PP; k.cs = CS;
+    k.fstride = 3 * (size_t)CS; k.xstride = 2 * (size_t)N;
+    k.f = prec == 8 ? (char*)F64 + 16 * k.fstride * p0 : (char*)F32 + 8 * k.fstride * p0;
+    k.L = t.L; k.P = t.P;
+    k.mLs = fame_magic32(prec == 8 ? t.L : t.L / 2);
+    k.half = N; k.off = 0;
+    return k;
+}
+KPlane fame_ctx::kplane(int prec, int p0, const int* act) const {
+    const int pi = prec == 8 ? 0 : 1;
+    const size_t es = prec == 8 ? 16 : 8;
+    KPlane k = kpl[pi];
+    k.active = act;
+    k.fstride = 3 * (size_t)CS;
+    k.f = prec == 8 ? (char*)F64 + 16 * k.fstride * p0 : (char*)F32 + 8 * k.fstride * p0;
+    k.invB = invBp[pi];
+    k.tw = (char*)mtw[pi] + es * (size_t)g.nb * g.nc * p0;
+    return k;
+}
+int fame_ctx::inner_blocks(int prec) const {
+    const int pi = prec == 8 ? 0 : 1;
+    return plane[pi] ? (g.nb * g.nc + ctile[pi].L - 1) / ctile[pi].L : nblk_in[pi];
+}
+
 extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int device, fame_ctx** out) {
     if (!lat || !out || max_batch < 1) FAIL(FAME_ERR_ARG, "fame_create: null argument or max_batch < 1");
     for (int i = 0; i < 3; ++i) if (lat->grid_nums[i] < 1 || lat->grid_nums[i] > 1024) FAIL(FAME_ERR_ARG, "grid_nums out of range");
@@ -363,7 +509,8 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
             }
         }
     }
-    const size_t N = g.N, B = max_batch;
+    if ((st = c->plane_setup()) != FAME_OK) { delete c; return st; }
+    const size_t N = g.N, B = max_batch, NF = std::max((size_t)g.N, (size_t)c->CS);
     c->nblk_in[0] = (g.nb * g.nc + c->tile[AX_INNER][0].L - 1) / c->tile[AX_INNER][0].L;
     c->nblk_in[1] = (g.nb * g.nc + c->tile[AX_INNER][1].L - 1) / c->tile[AX_INNER][1].L;
 #define A(ptr, bytes) do { fame_status s_ = dalloc(c, (void**)&(ptr), (bytes)); if (s_ != FAME_OK) { delete c; return s_; } } while (0)
@@ -374,8 +521,28 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
     A(c->invB32, sizeof(float) * 3 * N);
     A(c->eps_int, sizeof(double) * 3 * N);
     A(c->eps_ref, sizeof(double) * 3 * N);
-    A(c->F64, 16 * 3 * N * B);
-    A(c->F32, 8 * 3 * N * B);
+    A(c->F64, 16 * 3 * NF * B);
+    A(c->F32, 8 * 3 * NF * B);
+    if (c->plane_ok[0] || c->plane_ok[1]) {
+        const size_t nl = (size_t)g.nb * g.nc, tpl = inner_tw_per_line(g.na);
+        A(c->ltab, sizeof(LineTab) * nl * B);
+        for (int pi = 0; pi < 2; ++pi) {
+            const size_t es = pi ? 8 : 16;
+            A(c->invBp[pi], es / 2 * 3 * (size_t)c->CS);
+            A(c->ltw[pi], es * nl * tpl * B);
+            A(c->mtw[pi], es * nl * B);
+        }
+        A(c->eatab, 16 * (size_t)g.na);
+        std::vector<double> ea(2 * (size_t)g.na);
+        for (int a = 0; a < g.na; ++a) {
+            const long double x = 3.14159265358979323846264338327950288L * a / g.na;
+            ea[2 * a] = (double)cosl(x); ea[2 * a + 1] = (double)sinl(x);
+        }
+        if (hipMemcpy(c->eatab, ea.data(), 16 * (size_t)g.na, hipMemcpyHostToDevice) != hipSuccess) {
+            delete c;
+            FAIL(FAME_ERR_HIP, "fame_create: copy of the phase table failed");
+        }
+    }
     for (int i = 0; i < 4; ++i) A(c->cg64[i], 16 * 2 * N * B);
     for (int i = 0; i < 5; ++i) A(c->cg32[i], 8 * 2 * N * B);
     for (int i = 0; i < 3; ++i) A(c->ref64[i], 16 * 2 * N * B);
@@ -446,6 +613,20 @@ extern "C" fame_status fame_set_eps(fame_ctx* c, const double* eps) {
                     size_t q = comp * N + int_index(c->g, x, y, z);
                     e[q] = v; ib[q] = 1.0 / v; ib32[q] = (float)(1.0 / v);
                 }
+    /* 1 / (N eps) in the plane layout [component][a][c][b] of pitch PP */
+    std::vector<double> pb;
+    std::vector<float> pb32;
+    if (c->plane_ok[0] || c->plane_ok[1]) {
+        pb.assign(3 * (size_t)c->CS, 0.0); pb32.assign(3 * (size_t)c->CS, 0.0f);
+        const size_t nl = (size_t)c->g.nb * c->g.nc;
+        const double sc = 1.0 / (double)N;
+        for (int comp = 0; comp < 3; ++comp)
+            for (size_t l = 0; l < nl; ++l)
+                for (int a = 0; a < c->g.na; ++a) {
+                    const size_t d = (size_t)comp * c->CS + (size_t)a * c->PP + l;
+                    pb[d] = ib[comp * N + l * c->g.na + a] * sc; pb32[d] = (float)pb[d];
+                }
+    }
     /* the context's stream may still be running kernels that read the old values */
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -455,6 +636,10 @@ extern "C" fame_status fame_set_eps(fame_ctx* c, const double* eps) {
     HIPCHK(hipMemcpyAsync(c->eps_ref, eps, sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->invB64, ib.data(), sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->invB32, ib32.data(), sizeof(float) * 3 * N, hipMemcpyHostToDevice, c->stream));
+    if (!pb.empty()) {
+        HIPCHK(hipMemcpyAsync(c->invBp[0], pb.data(), sizeof(double) * pb.size(), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(c->invBp[1], pb32.data(), sizeof(float) * pb32.size(), hipMemcpyHostToDevice, c->stream));
+    }
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_eps = true;
     ++c->eps_ver;
@@ -506,6 +691,8 @@ extern "C" fame_status fame_set_wave_vectors(fame_ctx* c, int nk, const double* 
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMemcpyAsync(c->prob_d, c->prob_h.data(), sizeof(ProbDev) * nk, hipMemcpyHostToDevice, c->stream));
     HIPCHK(fame_launch_sigma(c->g, c->prob_d, c->sig, c->sig_inv, nk, c->stream));
+    if (c->ltab)
+        HIPCHK(fame_launch_line_tab(c->g, c->prob_d, c->ltab, c->ltw[0], c->ltw[1], c->mtw[0], c->mtw[1], nk, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     ++c->k_ver;
     return FAME_OK;
@@ -547,6 +734,7 @@ KAxis fame_ctx::kout(int prec, int p0, const int* act, int list) const {
 }
 
 int fame_ctx::pap_blocks(int prec) const {
+    if (plane[pix(prec)]) return g.na;
     for (int axis = 0; axis < 3; ++axis)
         if (plan(axis, prec).lists[pix(prec)][LIST_FWD].blue) return 0;
     const int L = tile[AX_OUTER][pix(prec)].L;
@@ -557,6 +745,17 @@ int fame_ctx::pap_blocks(int prec) const {
  * with dotvec, partial sums of conj(dotvec).y go to partials2 per inner block. */
 fame_status fame_ctx::qbq(int prec, const void* x, void* y, int p0, int nprob, const int* act, const void* dotvec,
                           void* cg_r, void* cg_x, const void* cg_ap, bool cgdots) {
+    if (plane[pix(prec)] && !cg_r && !dotvec && !cgdots) {
+        KLine k = kline(prec, p0, act);
+        k.x = x;
+        HIPCHK(launch_line(k, 1, LINE_EX_PLAIN, prec, nprob));
+        HIPCHK(launch_plane(kplane(prec, p0, act), prec, nprob));
+        k = kline(prec, p0, act, true);
+        k.xs = y;
+        HIPCHK(launch_line(k, 0, LINE_CO_PLAIN, prec, nprob));
+        if (prec == 8) cnt_qbq64 += nprob; else cnt_qbq32 += nprob;
+        return FAME_OK;
+    }
     KInner ki = kin(prec, p0, act, LIST_INV);
     ki.x = x; ki.pikind = 0;
     if (cg_r) { ki.cg_r = cg_r; ki.cg_x = cg_x; ki.cgsc = cgsc; ki.cg_ap = cg_ap; ki.partials = partials2; }
@@ -576,6 +775,19 @@ fame_status fame_ctx::qbq(int prec, const void* x, void* y, int p0, int nprob, c
 fame_status fame_ctx::qbq_residual32(const void* xr, const void* b, void* x32, int p0, int nprob, const int* act,
                                      int nact) {
     const size_t es = 8 * 2 * (size_t)N;   /* FP32 complex vector bytes per problem */
+    if (plane[0]) {
+        KLine k = kline(8, p0, act);
+        k.x = xr; k.fx32 = x32; k.fp32 = (char*)cg32[1] + es * p0; k.cgsc = cgsc;
+        HIPCHK(launch_line(k, 1, LINE_EX_FX, 8, nprob));
+        HIPCHK(launch_plane(kplane(8, p0, act), 8, nprob));
+        k = kline(8, p0, act, true);
+        k.rb = b; k.xs = x32;
+        k.r = (char*)cg32[0] + es * p0; k.p32 = (char*)cg32[1] + es * p0;
+        k.rpart = partials; k.rstep = 1;
+        HIPCHK(launch_line(k, 0, LINE_CO_RES, 8, nprob));
+        cnt_qbq64 += nact;
+        return FAME_OK;
+    }
     KInner ki = kin(8, p0, act, LIST_INV);
     ki.x = xr; ki.pikind = 0;
     ki.fx32 = x32; ki.fp32 = (char*)cg32[1] + es * p0; ki.cgsc = cgsc;
@@ -654,6 +866,19 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
             break;
         case FAME_OP_QBQ:
+            if (c->plane[0]) {
+                KLine k = c->kline(8, ik, nullptr);
+                k.off = N - Nd; k.half = Nd;
+                k.x = x;
+                HIPCHK(c->launch_line(k, 1, LINE_EX_PLAIN, 8, 1));
+                HIPCHK(c->launch_plane(c->kplane(8, ik, nullptr), 8, 1));
+                k = c->kline(8, ik, nullptr, true);
+                k.off = N - Nd; k.half = Nd;
+                k.xs = y;
+                HIPCHK(c->launch_line(k, 0, LINE_CO_PLAIN, 8, 1));
+                ++c->cnt_qbq64;
+                break;
+            }
             HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
             /* the field slot used by qbq is that of problem ik */
             CHK(c->qbq(8, xin, yout, ik, 1, nullptr, nullptr));
@@ -700,7 +925,7 @@ fame_status fame_ctx::tune(int prec) {
     void* F = prec == 8 ? (void*)F64 : (void*)F32;
     void* x = prec == 8 ? cg64[1] : cg32[1];
     void* y = prec == 8 ? cg64[2] : cg32[2];
-    HIPCHK(hipMemsetAsync(F, 0, es * 3 * (size_t)N * nk, stream));
+    HIPCHK(hipMemsetAsync(F, 0, es * 3 * (size_t)std::max(N, CS) * nk, stream));
     HIPCHK(hipMemsetAsync(x, 0, es * 2 * (size_t)N * nk, stream));
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
@@ -708,7 +933,72 @@ fame_status fame_ctx::tune(int prec) {
     static const int candL_inner[] = {2, 4, 6, 8, 10, 12, 16, 20, 24, 32};
     static const int candL_axis[] = {4, 8, 16, 24, 32, 48, 64};
     fame_status st = FAME_OK;
-    for (int a = 0; a < 3 && st == FAME_OK; ++a) {
+    /* milliseconds of three launches of one pass after an untimed one */
+    auto timed = [&](auto launch, float* ms) -> bool {
+        for (int rep = -1; rep < 3; ++rep) {
+            if (rep == 0 && hipEventRecord(e0, stream) != hipSuccess) return false;
+            if (launch() != hipSuccess) return false;
+        }
+        return hipEventRecord(e1, stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+               hipEventElapsedTime(ms, e0, e1) == hipSuccess;
+    };
+    float plane_ms = 1e30f, axis_ms = 0;
+    if (plane_ok[pi]) {
+        /* the CG forms of the inner kernels, whose extra streams shift the best
+         * tile (12 lines for the plain FP32 expansion at FCC 96, 16 for the CG
+         * one), on zero vectors with zero scalars                            */
+        void* r = prec == 8 ? cg64[0] : cg32[0];
+        HIPCHK(hipMemsetAsync(r, 0, es * 2 * (size_t)N * nk, stream));
+        HIPCHK(hipMemsetAsync(y, 0, es * 2 * (size_t)N * nk, stream));
+        std::memset(sc_h, 0, sizeof(CgScal) * nk);
+        for (int i = 0; i < nk; ++i) sc_h[i].pend = 1;    /* x read and written, as inside a solve */
+        HIPCHK(hipMemcpyAsync(cgsc, sc_h, sizeof(CgScal) * nk, hipMemcpyHostToDevice, stream));
+        plane_ms = 0;
+        for (int contract = 0; contract < 2 && st == FAME_OK; ++contract) {
+            PassTile& t = contract ? ctile[pi] : ltile[pi];
+            PassTile best = t;
+            float best_ms = 1e30f;
+            static const int cand[] = {4, 8, 12, 16, 24, 32};
+            for (int eng = 0; eng < 2 && st == FAME_OK; ++eng) {
+                if (contract && eng != ltile[pi].eng) continue;
+                for (int L : cand) {
+                    if (!line_tile_ok(prec, eng, L)) continue;
+                    t.eng = eng; t.L = L;
+                    KLine k = kline(prec, 0, nullptr, contract);
+                    k.x = x; k.r = r; k.xs = y; k.cgsc = cgsc;
+                    k.rpart = partials2 + 3; k.rstep = 6;
+                    float ms = 0;
+                    if (!timed([&] { return launch_line(k, !contract, contract ? (int)LINE_CO_CG : (int)LINE_EX_CG, prec, nk); }, &ms)) {
+                        st = FAME_ERR_HIP;
+                        break;
+                    }
+                    if (ms < best_ms) { best_ms = ms; best = t; }
+                }
+            }
+            t = best;
+            plane_ms += best_ms;
+        }
+        int best_nt = kpl[pi].nt;
+        float best_ms = 1e30f;
+        for (int nt = 256; nt <= 1024 && st == FAME_OK; nt *= 2) {
+            if (!plane_threads_ok(prec, nt)) continue;
+            KPlane k = kplane(prec, 0, nullptr);
+            k.nt = nt;
+            k.pap = pap_part;
+            float ms = 0;
+            if (!timed([&] { return launch_plane(k, prec, nk); }, &ms)) { st = FAME_ERR_HIP; break; }
+            if (ms < best_ms) { best_ms = ms; best_nt = nt; }
+        }
+        kpl[pi].nt = best_nt;
+        plane_ms += best_ms;
+    }
+    /* a plane that leaves room for two blocks per CU beats the axis passes by 8% to
+     * 30% at every batch measured; one that fills the CU alone may not, so both
+     * are timed                                                               */
+    const size_t plds = plane_ok[pi] ? fame_plane_lds(g.nb, g.nc, kpl[pi].b.ntab + kpl[pi].c.ntab, prec) : 0;
+    const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF;
+    plane[pi] = plane_ok[pi];
+    for (int a = 0; a < 3 && st == FAME_OK && axis_too; ++a) {
         PassTile best = tile[a][pi];
         float best_ms = 1e30f;
         for (int eng = 0; eng < 2; ++eng) {
@@ -748,7 +1038,9 @@ fame_status fame_ctx::tune(int prec) {
             if (st != FAME_OK) break;
         }
         tile[a][pi] = best;
+        axis_ms += best_ms;
     }
+    if (axis_too && axis_ms < plane_ms) plane[pi] = false;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (st != FAME_OK) FAIL(st, std::string("autotune: HIP error: ") + hipGetErrorString(hipGetLastError()));
@@ -761,6 +1053,21 @@ fame_status fame_ctx::tune(int prec) {
 extern "C" fame_status fame_set_tiles(fame_ctx* c, int prec, const int* choice) {
     if (!c || !choice || (prec != 8 && prec != 4)) FAIL(FAME_ERR_ARG, "fame_set_tiles: bad arguments");
     const int pi = prec == 8 ? 0 : 1;
+    /* engine 2 for the middle and outer passes: the plane path, whose middle
+     * entry holds the contracting kernel's lines and outer entry the plane
+     * kernel's threads                                                        */
+    if (choice[2] == 2 && choice[4] == 2) {
+        if (!c->line_tile_ok(prec, choice[0], choice[1]) || !c->line_tile_ok(prec, choice[0], choice[3]) ||
+            !plane_threads_ok(prec, choice[5]))
+            FAIL(FAME_ERR_ARG, "fame_set_tiles: engine, lines per block or threads not available for the plane path");
+        c->plane[pi] = true;
+        c->ltile[pi].eng = c->ctile[pi].eng = choice[0];
+        c->ltile[pi].L = choice[1]; c->ctile[pi].L = choice[3];
+        c->kpl[pi].nt = choice[5];
+        c->tuned[pi] = true;
+        c->drop_graphs();
+        return FAME_OK;
+    }
     for (int a = 0; a < 3; ++a) {
         const int eng = choice[2 * a], L = choice[2 * a + 1];
         if (eng < 0 || eng > 1 || c->ax[a][eng].n == 0 || !tile_ok(c->ax[a][eng], a, prec, L, c->g))
@@ -770,6 +1077,7 @@ extern "C" fame_status fame_set_tiles(fame_ctx* c, int prec, const int* choice) 
         PassTile& t = c->tile[a][pi];
         t.eng = choice[2 * a]; t.L = choice[2 * a + 1]; t.P = c->ax[a][t.eng].M | 1;
     }
+    c->plane[pi] = false;
     c->nblk_in[pi] = (c->g.nb * c->g.nc + c->tile[AX_INNER][pi].L - 1) / c->tile[AX_INNER][pi].L;
     c->tuned[pi] = true;
     c->drop_graphs();
@@ -783,6 +1091,11 @@ extern "C" fame_status fame_autotune(fame_ctx* c, int prec, int* choice) {
     if (choice) {
         const int pi = prec == 8 ? 0 : 1;
         for (int a = 0; a < 3; ++a) { choice[2 * a] = c->tile[a][pi].eng; choice[2 * a + 1] = c->tile[a][pi].L; }
+        if (c->plane[pi]) {
+            choice[0] = c->ltile[pi].eng; choice[1] = c->ltile[pi].L;
+            choice[2] = 2; choice[3] = c->ctile[pi].L;
+            choice[4] = 2; choice[5] = c->kpl[pi].nt;
+        }
     }
     return FAME_OK;
 }
@@ -854,6 +1167,20 @@ fame_status fame_ctx::cg_step_ap(int prec, void* p, void* r, void* x, void* Ap, 
  * the last pass stores r - alpha Ap (Ap itself is never written) and sums its
  * <r,r>; beta and the flags from that exact norm */
 fame_status fame_ctx::cg_step_rc(int prec, void* p, void* r, void* x, int p0, int nprob, int npap) {
+    if (plane[pix(prec)]) {
+        KLine k = kline(prec, p0, active);
+        k.x = p; k.r = r; k.xs = x; k.cgsc = cgsc;
+        HIPCHK(launch_line(k, 1, LINE_EX_CG, prec, nprob));
+        KPlane kp = kplane(prec, p0, active);
+        kp.pap = pap_part;
+        HIPCHK(launch_plane(kp, prec, nprob));
+        HIPCHK(fame_cg_alpha(cgsc, pap_part, npap, nprob, active, stream));
+        k = kline(prec, p0, active, true);
+        k.r = r; k.cgsc = cgsc; k.rpart = partials2 + 3; k.rstep = 6;
+        HIPCHK(launch_line(k, 0, LINE_CO_CG, prec, nprob));
+        HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), nprob, active, stream));
+        return FAME_OK;
+    }
     KInner ki = kin(prec, p0, active, LIST_INV);
     ki.x = p; ki.pikind = 0;
     ki.cg_r = r; ki.cg_x = x; ki.cgsc = cgsc; ki.cg_ap = nullptr; ki.partials = partials2;
@@ -980,7 +1307,7 @@ fame_status fame_ctx::invar(int mode, const void* x, void* y, int p0, int nprob,
             for (int i = 0; i < nprob; ++i) if (msk[i]) it[i] += it32[i] - 1;
             /* the next sweep's start from r = b - QBQ64 xr, with its norm */
             CHK(qbq_residual32(xr, b, d32, p0, nprob, mask, (int)std::count(msk.begin(), msk.end(), 1)));
-            nbp = nblk_in[pix(8)];
+            nbp = inner_blocks(8);
         }
         for (int i = 0; i < nprob; ++i) it[i] += 1;
     }

@@ -211,7 +211,9 @@ fame_status fame_eig_grad(fame_ctx* ctx, int nwant, const double* freq, const vo
 /* Average durations in microseconds (hipEvent timing on the context stream) of
  * the five QBQ passes and of a whole QBQ over all wave vectors of the context,
  * us6 = {inner expand, middle inverse, outer eps, middle forward, inner contract,
- * whole QBQ}; prec = 8 (FP64) or 4 (FP32).  Measurement helper, no reference
+ * whole QBQ}; prec = 8 (FP64) or 4 (FP32).  With the plane kernel, which runs the
+ * middle and outer passes as one, the middle entries are 0 and its time is the
+ * outer one.  Measurement helper, no reference
  * counterpart.                                                                 */
 fame_status fame_time_qbq_passes(fame_ctx* ctx, int prec, int reps, double* us6);
 
@@ -219,7 +221,8 @@ fame_status fame_time_qbq_passes(fame_ctx* ctx, int prec, int reps, double* us6)
  * the kernels of one fused CG iteration with every wave vector active:
  * us8 = {inner expand with the x and p updates, middle inverse, outer eps with
  * the <p,Ap> sums, alpha, middle forward, inner contract with the r update and
- * <r,r> sums, beta, whole iteration}; prec = 8 or 4.  FAME_ERR_UNSUPPORTED when
+ * <r,r> sums, beta, whole iteration}; prec = 8 or 4 (the middle entries 0 with the
+ * plane kernel).  FAME_ERR_UNSUPPORTED when
  * an axis takes a Bluestein plan (that iteration form stores Ap).  Measurement
  * helper, no reference counterpart.                                          */
 fame_status fame_time_cg_passes(fame_ctx* ctx, int prec, int reps, double* us8);
@@ -229,7 +232,11 @@ fame_status fame_time_cg_passes(fame_ctx* ctx, int prec, int reps, double* us8);
  * current batch and keep the fastest.  fame_eigs runs it once per context and
  * precision unless FAME_AUTOTUNE=0.  choice (host, 6 ints, may be NULL)
  * receives {engine, lines} for the inner, middle and outer passes (engine 0
- * Stockham/Bluestein, 1 direct DFT on the matrix cores).  Replaces the fixed
+ * Stockham/Bluestein, 1 direct DFT on the matrix cores).  Where the two outer
+ * axes of a QBQ run as one pass over (b, c) planes in LDS, the middle and outer
+ * engines are 2, and the lines are those of the expanding kernel (inner), of
+ * the contracting kernel (middle) and the plane kernel's threads (outer).
+ * Replaces the fixed
  * cuFFT plans of FAME_Create_cublas (FAME_Main/FAME_Create_cublas.cu:16-25).  */
 fame_status fame_autotune(fame_ctx* ctx, int prec, int* choice);
 

@@ -1,0 +1,111 @@
+"""The plane path of the QBQ (the two outer axes in one pass over (b, c) planes in
+LDS) against the FP64 oracle, at the sizes where its kernels can go wrong: odd and
+even rows (linear or padded LDS rows), odd planes (padding of the plane pitch),
+one-, two- and three-pass axes, direct DFTs on the matrix cores along every axis,
+line counts that leave the last block of the inner kernels ragged, Gamma, and every
+lines-per-block and thread count its rule accepts.  Both precisions hold the bars of
+the axis passes: 1e-11 of the oracle in FP64, 2e-6 in FP32, 1e-8 in lambda for an
+FP32-refined solve, and the two paths agree within those bars."""
+import numpy as np
+import pytest
+
+import fame_amd as F
+import oracle as O
+from cases import SPHERE
+
+pytestmark = pytest.mark.gpu
+
+O.set_threads(8)
+
+# grid sides (a, b, c) reached: 9^3 (one radix per axis), 16^3 (one FP32 pass), 17^3 (direct DFT on
+# all axes), 18^3, 26^3 (13 x 2), 34^3 (2 x 17: direct), FCC 22x19x18, 41x36x33 (c = 41 direct),
+# BCC 17x16x13, hexagonal 31x26x22 and 16x13x11
+GRIDS = [("simple_cubic", 9), ("simple_cubic", 16), ("simple_cubic", 17), ("simple_cubic", 18), ("simple_cubic", 26),
+         ("simple_cubic", 34), ("face_centered_cubic", 22), ("face_centered_cubic", 41), ("body_centered_cubic", 17),
+         ("hexagonal", 31), ("hexagonal", 16)]
+
+
+def _rand(n, seed):
+    rng = np.random.default_rng(seed)
+    return rng.standard_normal(n) + 1j * rng.standard_normal(n)
+
+
+def _rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+def _setup(lt, nx):
+    lo = F.build_lattice(lt, nx, **({"c": 1.2} if lt == "hexagonal" else {}))
+    fl = F.to_fame_lattice(lo)
+    return fl, F.material_eps(lo, SPHERE, [13.0], 1.0)
+
+
+def _accepted(S, prec, tiles):
+    try:
+        S.set_tiles(prec, tiles)
+        return True
+    except F.FameError:
+        return False
+
+
+@pytest.mark.parametrize("lt,nx", GRIDS, ids=lambda v: str(v))
+@pytest.mark.parametrize("k", [(0.21, -0.13, 0.07), (0.0, 0.0, 0.0)], ids=["k", "gamma"])
+def test_plane_qbq_vs_oracle(gpu, lt, nx, k):
+    import torch
+    fl, eps = _setup(lt, nx)
+    T = O.Tables(O.lattice_from(fl), np.array(k))
+    S = F.Solver(fl, max_batch=1)
+    S.set_eps(eps)
+    S.set_wave_vectors(np.array(k))
+    x = _rand(2 * T.Nd, 3)
+    ref = T.qbq(1.0 / eps, x)
+    xd = torch.from_numpy(x).to("cuda")
+    seen = 0
+    for prec, op, bar in ((8, F.OP_QBQ, 1e-11), (4, F.OP_QBQ32, 2e-6)):
+        for eng in (0, 1):
+            for le, lc, nt in ((2, 4, 256), (4, 2, 512), (6, 8, 1024), (8, 12, 256), (16, 16, 512), (32, 24, 256)):
+                t = {"inner": (eng, le), "mid": (2, lc), "outer": (2, nt)}
+                if not _accepted(S, prec, t):
+                    continue
+                seen += 1
+                y = S.apply(op, 0, xd).cpu().numpy()
+                assert _rel(y, ref) < bar, (prec, t, _rel(y, ref))
+        # the axis passes on the same grid
+        if _accepted(S, prec, {"inner": (0, 4), "mid": (0, 8), "outer": (0, 8)}):
+            assert _rel(S.apply(op, 0, xd).cpu().numpy(), ref) < bar
+    assert seen >= 6
+    S.close()
+
+
+@pytest.mark.parametrize("lt,nx", [("simple_cubic", 17), ("face_centered_cubic", 22), ("body_centered_cubic", 16)])
+def test_plane_eigs_vs_axis_passes(gpu, lt, nx):
+    fl, eps = _setup(lt, nx)
+    ks = np.array([[0.21, -0.13, 0.07], [0.05, 0.31, -0.22], [0.4, 0.1, 0.2]])
+    S = F.Solver(fl, max_batch=3)
+    S.set_eps(eps)
+    S.set_wave_vectors(ks)
+    lam = {}
+    for plane in (False, True):
+        for prec in (8, 4):
+            t = {"inner": (1 if nx == 17 else 0, 4), "mid": (2, 8), "outer": (2, 256)} if plane else {"inner": (1, 4), "mid": (1, 16), "outer": (1, 16)}
+            S.set_tiles(prec, t)
+        for precision in (F.PREC_F64, F.PREC_F32_REFINE):
+            f, _, _, prof = S.eigs(5, 18, precision=precision)
+            assert all(p["converged"] for p in prof)
+            lam[plane, precision] = f ** 2
+    for key, v in lam.items():
+        assert np.max(np.abs(v - lam[False, F.PREC_F64]) / lam[False, F.PREC_F64]) < 1e-8, key
+    S.close()
+
+
+def test_plane_tiles_are_refused_where_unavailable(gpu):
+    fl, eps = _setup("simple_cubic", 18)
+    S = F.Solver(fl, max_batch=1)
+    S.set_eps(eps)
+    for prec, t in ((4, {"inner": (0, 3), "mid": (2, 8), "outer": (2, 256)}),      # FP32 moves pairs of lines
+                    (8, {"inner": (0, 64), "mid": (2, 8), "outer": (2, 256)}),
+                    (8, {"inner": (0, 4), "mid": (2, 8), "outer": (2, 300)}),
+                    (8, {"inner": (2, 4), "mid": (2, 8), "outer": (2, 256)})):
+        with pytest.raises(F.FameError):
+            S.set_tiles(prec, t)
+    S.close()
