@@ -213,11 +213,59 @@ static fame_status residuals_chunk(fame_ctx* c, int nwant, const double* freq, c
     return FAME_OK;
 }
 
+/* The same for all wave vectors on the plane layout, without a copy of the fields:
+ * the analysis reads them in the reference's layout and the synthesis compares its
+ * planes with them and stores nothing (General; Simple grids transpose the fields
+ * in and compare tile by tile).  One read-back at the end.                   */
+static bool residuals_by_planes(const fame_ctx* c, int nwant) {
+    /* two sums per plane in pap_part, 3 numbers per wave vector and band in partials2 */
+    return c->syn_ok && nwant <= 1024 && 2 * c->g.na <= xcd_round(c->g.na * c->g.nb);
+}
+static fame_status residuals_planes(fame_ctx* c, int nwant, const double* freq, const void* E_dev, double* res) {
+    const size_t N = c->N, N3 = 3 * N, pn = (size_t)c->g.nb * c->g.nc, es = (size_t)nwant * N3;
+    const int nk = c->nk, NB = 256;
+    const size_t nf = (size_t)nk * nwant;
+    std::vector<double> h(nf), out(2 * nf);
+    for (size_t i = 0; i < nf; ++i) h[i] = freq[i] * freq[i];
+    double* w2 = c->partials2;                 /* at least 6144 doubles per problem */
+    double* sums = c->partials2 + nf;
+    HIPCHK(hipMemcpyAsync(w2, h.data(), sizeof(double) * nf, hipMemcpyHostToDevice, c->stream));
+    for (int i = 0; i < nwant; ++i) {
+        const double2* E = (const double2*)E_dev + (size_t)i * N3;
+        KSyn s = c->ksyn(0);
+        s.ostride = es; s.E = E; s.eps = c->eps_ref; s.w2 = w2 + i; s.w2step = nwant; s.part = c->pap_part;
+        if (c->g.general) s.in = E;
+        else
+            HIPCHK(fame_launch_transpose(E, c->F64, (int)pn, c->g.na, c->g.na, c->PP, N, c->CS, 3, es, 3 * (size_t)c->CS, nullptr, nk,
+                                         c->stream));
+        HIPCHK(fame_launch_ana(s, nk, c->stream));
+        HIPCHK(fame_launch_curl(c->kline(8, 0, nullptr), 0, nk, c->stream));
+        if (c->g.general) {
+            HIPCHK(fame_launch_syn(s, SYN_RES, nk, c->stream));
+            HIPCHK(fame_reduce_partials(c->pap_part, 3 * c->g.na, 2, sums + 2 * (size_t)i * nk, nk, c->stream));
+        } else {
+            HIPCHK(fame_launch_syn(s, SYN_FIELD, nk, c->stream));
+            HIPCHK(fame_launch_resid_simple(c->F64, E, c->eps_ref, w2 + i, nwant, c->partials, NB, c->g.na, (int)pn, c->PP,
+                                            3 * (size_t)c->CS, es, nk, c->stream));
+            HIPCHK(fame_reduce_partials(c->partials, NB, 2, sums + 2 * (size_t)i * nk, nk, c->stream));
+        }
+    }
+    HIPCHK(hipMemcpyAsync(out.data(), sums, sizeof(double) * 2 * nf, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int i = 0; i < nwant; ++i)
+        for (int p = 0; p < nk; ++p) {
+            const double a = out[2 * ((size_t)i * nk + p)], b = out[2 * ((size_t)i * nk + p) + 1];
+            res[(size_t)p * nwant + i] = b > 0 ? std::sqrt(a / b) : 0.0;
+        }
+    return FAME_OK;
+}
+
 extern "C" fame_status fame_residuals(fame_ctx* c, int nwant, const double* freq, const void* E_dev, double* res) {
     if (!c || !freq || !E_dev || !res || nwant < 1) FAIL(FAME_ERR_ARG, "fame_residuals: bad arguments");
     if (!c->have_eps) FAIL(FAME_ERR_STATE, "fame_residuals: permittivity not set");
     HIPCHK(hipSetDevice(c->device));
     const int nk = c->nk;
+    if (residuals_by_planes(c, nwant)) return residuals_planes(c, nwant, freq, E_dev, res);
     const size_t N3 = 3 * (size_t)c->N;
     double2* Ecopy = nullptr;
     HIPCHK(hipMalloc(&Ecopy, 16 * N3 * nk));
@@ -260,6 +308,7 @@ extern "C" fame_status fame_residuals_noalloc(fame_ctx* c, int nwant, const doub
                                        std::to_string(FAME_NOALLOC_ELEMS) + " complex values (N <= " +
                                        std::to_string(FAME_NOALLOC_ELEMS / 3) + ")");
     HIPCHK(hipSetDevice(c->device));
+    if (residuals_by_planes(c, nwant)) return residuals_planes(c, nwant, freq, E_dev, res);   /* needs no scratch */
     double2* sc = nullptr;
     CHK(scratch_address(c->device, &sc));
     const int chunk = (int)std::min<size_t>((size_t)c->nk, FAME_NOALLOC_ELEMS / N3);

@@ -53,6 +53,7 @@ struct fame_ctx {
      * whether the solver takes it, the inner tiles (engine, lines per block) of
      * its expanding and contracting kernels, the launch templates, its tables */
     bool plane_ok[2] = {false, false}, plane[2] = {false, false};
+    bool syn_ok = false;          /* the FP64 one-way plane kernels (Qr, Qrs, restoration, residuals) */
     PassTile ltile[2], ctile[2];
     int PP = 0, CS = 0;           /* plane pitch and component stride (na PP)  */
     PlaneAxis laxis[2][2];        /* inner axis [precision][engine], n = 0 when not available */
@@ -130,6 +131,9 @@ struct fame_ctx {
     KPlane kplane(int prec, int p0, const int* act) const;
     hipError_t launch_line(const KLine& k, int expand, int mode, int prec, int nprob);
     hipError_t launch_plane(const KPlane& k, int prec, int nprob);
+    KSyn ksyn(int p0) const;
+    /* eps_ref (device) into the kernels' layouts */
+    fame_status spread_eps();
     int inner_blocks(int prec) const;   /* blocks per problem whose sums the contracting pass leaves */
     KInner kin(int prec, int p0, const int* act, int list) const;
     KAxis kmid(int prec, int p0, const int* act, int list) const;

@@ -89,7 +89,7 @@ struct PlaneStage {
 };
 struct PlaneAxis {
     int n, eng, nst;
-    unsigned mnl;                /* udiv magic for / lines                      */
+    unsigned mnl, mn;            /* udiv magics for / lines and / n             */
     int ntab;                    /* entries of W, kept in LDS                   */
     const void* W;               /* Stockham: exp(-2 pi i m / n), n entries; direct DFT: its
                                     (cos, -sin) fragments [tile][K step][64]    */
@@ -118,11 +118,8 @@ struct KLine {
     int PP, cs;                  /* plane pitch and component stride (na PP)    */
     int L, P;                    /* lines per block, LDS line pitch             */
     unsigned mLs;                /* udiv magic of the field accesses: / (L / 2) in FP32, / L in FP64 */
-    /* reduced vectors: mode f of the first half at [f - off], of the second at
-     * [half + f - off] (padded vectors: off 0, half N; the reference's layout at
-     * Gamma: off 1, half N - 1)                                              */
     const void* x;
-    int half, off;
+    int ref;                     /* reduced vectors in the reference's layout (2 Nd), not padded */
     const double* sig;           /* expand, plain: x scaled by sig[f] (optional) */
     void* r;                     /* CG residual; contract CO_RES: r32           */
     void* xs;                    /* CG solution; contract: y, or x32 of CO_RES  */
@@ -146,6 +143,21 @@ struct KPlane {
     PlaneAxis b, c;
     unsigned mnb;
     int nprob, nt;
+};
+
+/* what a one-way plane kernel (FP64) does after its inverse transforms (fame_plane64.hip) */
+enum { SYN_FIELD = 0, SYN_REF = 1, SYN_EPS = 2, SYN_RES = 3 };
+struct KSyn {
+    KPlane k;                    /* invB: 1 / (N eps) for SYN_EPS               */
+    const fame::ProbDev* prob;
+    const double2* in;           /* analysis: field in the reference's layout (General), or null: in place */
+    double2* out;                /* SYN_REF: field in the reference's layout    */
+    const double2* E;            /* SYN_RES: the fields, reference's layout (General) */
+    const double* eps;           /* SYN_RES: permittivity, reference's layout   */
+    const double* w2;            /* SYN_RES: omega^2 of problem p at w2[p w2step] */
+    size_t ostride;              /* problem stride of in / out / E              */
+    double* part;                /* SYN_EPS: |E|^2 per block; SYN_RES: |r|^2, |E|^2 per block */
+    int w2step;
 };
 
 struct KAxis {
@@ -202,6 +214,22 @@ hipError_t fame_launch_plane32(const KPlane& k, int nprob, hipStream_t s);
 hipError_t fame_launch_plane64(const KPlane& k, int nprob, hipStream_t s);
 hipError_t fame_prepare_plane32(int eb, int ec, size_t lds);
 hipError_t fame_prepare_plane64(int eb, int ec, size_t lds);
+hipError_t fame_prepare_syn(int eb, int ec);
+hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s);
+hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s);
+hipError_t fame_launch_curl(const KLine& k, int step, int nprob, hipStream_t s);
+/* out = s in^T for `batch` matrices (rows x cols, pitch ip) of each problem, s the
+ * square root of scale2[p] (null: 1) */
+hipError_t fame_launch_transpose(const double2* in, double2* out, int rows, int cols, int ip, int op, size_t ib, size_t ob,
+                                 int batch, size_t is, size_t os, const double* scale2, int nprob, hipStream_t s);
+/* partials of |F - w2 eps E|^2 and |E|^2, F in the plane layout [component][a][PP] of a
+ * Simple grid, E and eps in its reference layout [component][c b][a] */
+hipError_t fame_launch_resid_simple(const double2* F, const double2* E, const double* eps, const double* w2, int w2step,
+                                    double* part, int nblk, int na, int nl, int PP, size_t fs, size_t es, int nprob,
+                                    hipStream_t s);
+/* 1/eps, eps and 1 / (N eps) in the kernels' layouts from the reference's */
+hipError_t fame_launch_eps(const fame::GridDev& g, const double* eps, double* eps_int, double* ib64, float* ib32, double* p64,
+                           float* p32, int PP, hipStream_t s);
 hipError_t fame_launch_line_tab(const fame::GridDev& g, const fame::ProbDev* prob, LineTab* lt, void* tw64, void* tw32,
                                 void* mid64, void* mid32, int nprob, hipStream_t s);
 hipError_t fame_launch_xz_transpose(const void* in, void* out, int nx, int ny, int nz, int dir, size_t stride,

@@ -314,10 +314,15 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         c->kids_eps_ver = c->kids_k_ver = -1;
     }
     if (c->kids_eps_ver != c->eps_ver) {
-        std::vector<double> e(3 * (size_t)c->N);
-        HIPCHK(hipMemcpyAsync(e.data(), c->eps_ref, sizeof(double) * e.size(), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (fame_ctx* k : c->kids) CHK(fame_set_eps(k, e.data()));
+        /* device to device, on each child's stream (idle: its last solve ended
+         * with a synchronisation), the parent's own stream being drained        */
+        for (fame_ctx* k : c->kids) {
+            HIPCHK(hipMemcpyAsync(k->eps_ref, c->eps_ref, sizeof(double) * 3 * (size_t)c->N, hipMemcpyDeviceToDevice, k->stream));
+            CHK(k->spread_eps());
+            HIPCHK(hipStreamSynchronize(k->stream));
+            k->have_eps = true;
+            ++k->eps_ver;
+        }
         c->kids_eps_ver = c->eps_ver;
     }
     if (c->kids_k_ver != c->k_ver || c->kid_nk != c->nk) {
@@ -631,9 +636,32 @@ extern "C" fame_status fame_eigs_impl(fame_ctx* c, int precision, const fame_es*
 /* E_i = invB .* Qr(Sigma .* ev_i), times ||E_i|| (reference scaling), for band i
  * of every problem (FAME_Fast_Algorithms_Isotropic.cu:90-125).  ev: padded
  * reduced vectors of band i with per-problem stride ev_pstride.              */
-static fame_status restore_band(fame_ctx* c, int i, int nwant, const double2* ev, size_t ev_pstride, void* E_dev) {
+static fame_status restore_band(fame_ctx* c, int i, int nwant, const double2* ev, size_t ev_pstride, void* E_dev,
+                                bool ref = false) {
     const size_t N = c->N, n2 = 2 * N, N3 = 3 * N;
     const int nk = c->nk;
+    if (c->syn_ok) {
+        /* four kernels and no host round trip: the expansion scales by Sigma as it
+         * reads, the plane kernel applies 1/eps and sums |E|^2, the transpose to the
+         * reference's layout applies the norm.  Against the separate passes
+         * (conversion, scalings, norm, layout; 48 N s of traffic) 18.5 N s       */
+        KLine k = c->kline(8, 0, nullptr);
+        k.x = ev; k.xstride = ev_pstride; k.ref = ref ? 1 : 0; k.sig = c->sig;
+        HIPCHK(c->launch_line(k, 1, LINE_EX_PLAIN, 8, nk));
+        KSyn s = c->ksyn(0);
+        s.part = c->pap_part;
+        HIPCHK(fame_launch_syn(s, SYN_EPS, nk, c->stream));
+        HIPCHK(fame_reduce_partials(c->pap_part, 3 * c->g.na, 1, c->scal, nk, c->stream));
+        const size_t os = (size_t)c->out_pmul * nwant * N3, pn = (size_t)c->g.nb * c->g.nc;
+        double2* out = (double2*)E_dev + (size_t)i * N3;
+        if (c->g.general)
+            HIPCHK(fame_launch_transpose(c->F64, out, c->g.nc, c->g.nb, c->g.nb, c->g.nc, c->PP, pn, 3 * c->g.na, 3 * (size_t)c->CS,
+                                         os, c->scal, nk, c->stream));
+        else
+            HIPCHK(fame_launch_transpose(c->F64, out, c->g.na, (int)pn, c->PP, c->g.na, c->CS, N, 3, 3 * (size_t)c->CS, os, c->scal,
+                                         nk, c->stream));
+        return FAME_OK;
+    }
     double2* y = (double2*)c->ref64[0];
     std::vector<double> nr(nk);
     HIPCHK(fame_convert(y, 8, ev, 8, n2, n2, ev_pstride, nk, c->stream));
@@ -682,6 +710,10 @@ extern "C" fame_status fame_restore(fame_ctx* c, int nwant, const void* evr_dev,
     const size_t n2 = 2 * (size_t)c->N;
     double2* stage = (double2*)c->ref64[2];
     for (int i = 0; i < nwant; ++i) {
+        if (c->syn_ok) {
+            CHK(restore_band(c, i, nwant, (const double2*)evr_dev + (size_t)i * n2, (size_t)nwant * n2, E_dev, true));
+            continue;
+        }
         for (int p = 0; p < c->nk; ++p)
             HIPCHK(fame_launch_pack((const double2*)evr_dev + ((size_t)p * nwant + i) * n2, stage + (size_t)p * n2, c->N,
                                     c->nd[p], +1, 8, c->stream));

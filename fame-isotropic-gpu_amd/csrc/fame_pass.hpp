@@ -22,6 +22,11 @@ namespace fame {
  * private copy of a by-value argument that is indexed at run time           */
 typedef const __attribute__((address_space(4))) PlaneStage CStage;
 __device__ __forceinline__ CStage* cstage(const PlaneStage* p) { return (CStage*)(uintptr_t)p; }
+__device__ __forceinline__ PlaneStage load_stage(CStage* p) {
+    PlaneStage s;
+    s.R = p->R; s.Ns = p->Ns; s.nb = p->nb; s.tstep = p->tstep; s.mNs = p->mNs;
+    return s;
+}
 
 /* lines per round of a pass with nbf butterflies per line, NBT per thread, and
  * id / lpr as (id + 1/2) * (1 / lpr): exact, since the quotient is below 2^13 and
@@ -64,7 +69,7 @@ __device__ __forceinline__ V ld_uni(const V* base, unsigned o) {
  * hook values are under way, and each round fetches the next round's before its
  * own barrier. */
 template <typename T, typename T2, int R, int MAXE, bool INV, int HK>
-__device__ __forceinline__ void line_pass(T2* S, int nl, int LS, int ES, CStage& st, const T2* W,
+__device__ __forceinline__ void line_pass(T2* S, int nl, int LS, int ES, const PlaneStage& st, const T2* W,
                                           const Hook<T, T2>& hk, bool first, bool last) {
     constexpr int NBT = nbt_of(R, MAXE);
     const int nbf = st.nb, Ns = st.Ns, NT = (int)blockDim.x;
@@ -156,7 +161,7 @@ __device__ __forceinline__ void line_pass(T2* S, int nl, int LS, int ES, CStage&
  * are that forward pass's inputs, so the three run in registers on one LDS round
  * trip.  Returns this thread's share of <v, eps^-1 v> (hk.pap).              */
 template <typename T, typename T2, int R, int MAXE>
-__device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, CStage& st, const T2* W,
+__device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, const PlaneStage& st, const T2* W,
                                            const Hook<T, T2>& hk, bool only) {
     constexpr int NBT = nbt_of(R, MAXE);
     const int nbf = st.nb, NT = (int)blockDim.x;
@@ -267,8 +272,15 @@ __device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, CStage
 template <typename T, typename T2, bool INV, int HK>
 __device__ __forceinline__ void line_passes(T2* S, int nl, int LS, int ES, CStage* st, int s0, int s1, int nst,
                                             const T2* W, const Hook<T, T2>& hk) {
-#define LP(R) line_pass<T, T2, R, MaxE<T>::v, INV, HK>(S, nl, LS, ES, st[s], W, hk, s == 0, s + 1 == nst)
-    for (int s = s0; s < s1; ++s) { RADIX_SWITCH(st[s].R, LP) }
+    if (s0 >= s1) return;
+    PlaneStage cur = load_stage(st + s0);
+#define LP(R) line_pass<T, T2, R, MaxE<T>::v, INV, HK>(S, nl, LS, ES, cur, W, hk, s == 0, s + 1 == nst)
+    for (int s = s0; s < s1; ++s) {
+        /* the next pass's descriptor is on its way while this pass runs */
+        const PlaneStage next = load_stage(st + (s + 1 < s1 ? s + 1 : s));
+        RADIX_SWITCH(cur.R, LP)
+        cur = next;
+    }
 #undef LP
 }
 
@@ -413,9 +425,10 @@ __device__ __forceinline__ double column_round_trip(T2* S, int nl, int ES, const
     double acc = 0.0;
     if constexpr (ENG == ENG_STOCKHAM) {
         const int n = ax.nst;
+        const PlaneStage ms = load_stage(cstage(ax.st) + n - 1);
         line_passes<T, T2, true, HK_TIN>(S, nl, 1, ES, cstage(ax.st), 0, n - 1, n, W, hk);
-#define MP(R) acc = mid_pass<T, T2, R, MaxE<T>::v>(S, nl, 1, ES, cstage(ax.st)[n - 1], W, hk, n == 1)
-        RADIX_SWITCH(cstage(ax.st)[n - 1].R, MP)
+#define MP(R) acc = mid_pass<T, T2, R, MaxE<T>::v>(S, nl, 1, ES, ms, W, hk, n == 1)
+        RADIX_SWITCH(ms.R, MP)
 #undef MP
         line_passes<T, T2, false, HK_TOUT>(S, nl, 1, ES, cstage(ax.sf), 1, n, n, W, hk);
     } else {
@@ -439,6 +452,27 @@ __device__ __forceinline__ double column_round_trip(T2* S, int nl, int ES, const
         step([&](T2& e, unsigned o) { e = cmulc(e, hk.tw[o]); });
     }
     return acc;
+}
+
+/* one transform along c with the middle twiddle: inverse with it going in, or
+ * forward with its conjugate coming out.  Begins with a barrier, ends without. */
+template <typename T, typename T2, int ENG, bool INV>
+__device__ __forceinline__ void column_transform(T2* S, int nl, int ES, const PlaneAxis& ax, const T2* W,
+                                                 const Hook<T, T2>& hk) {
+    if constexpr (ENG == ENG_STOCKHAM) {
+        line_passes<T, T2, INV, INV ? HK_TIN : HK_TOUT>(S, nl, 1, ES, cstage(INV ? ax.st : ax.sf), 0, ax.nst, ax.nst, W, hk);
+    } else {
+        const int tot = nl * ax.n;
+        if (!INV) line_mfma<T, T2, INV>(S, nl, 1, ES, ax.n, W);
+        __syncthreads();
+        for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
+            const int m = udiv(idx, ax.mnl), l = idx - m * nl;
+            T2& e = S[l + m * ES];
+            const T2 w = hk.tw[(unsigned)(m * hk.ld + l)];
+            e = INV ? cmul(e, w) : cmulc(e, w);
+        }
+        if (INV) line_mfma<T, T2, INV>(S, nl, 1, ES, ax.n, W);
+    }
 }
 
 }  // namespace fame

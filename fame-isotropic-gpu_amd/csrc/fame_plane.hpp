@@ -162,7 +162,9 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
     const bool gam = k.prob[p].gamma != 0;
     const double iha2 = 2.0 * k.g.iha;
     T2* X = reinterpret_cast<T2*>(const_cast<void*>(k.x)) + (size_t)p * k.xstride;
-    const unsigned half = (unsigned)k.half, off = (unsigned)k.off;
+    /* reduced vectors: mode f of the first half at [f - off], of the second at
+     * [half + f - off]; the reference's layout leaves out mode 0 at Gamma     */
+    const unsigned off = k.ref && gam ? 1u : 0u, half = (unsigned)k.g.N - off;
     T beta = 0, al = 0;
     bool pend = false;
     if (MODE != EX_PLAIN) {
@@ -410,7 +412,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
     }
     line_transform<T, T2, ENG, false>(S, 3 * L, P, 1, k.a, m.W);
     __syncthreads();
-    const unsigned half = (unsigned)k.half, off = (unsigned)k.off;
+    const unsigned off = k.ref && gam ? 1u : 0u, half = (unsigned)k.g.N - off;
     const int tot = nl * na;
     double rn = 0.0;
     T al = 0;
@@ -682,7 +684,7 @@ static hipError_t launch_plane(const KPlane& k, int nprob, hipStream_t s) {
 template <typename T>
 static hipError_t prepare_plane(int eb, int ec, size_t lds) {
     for (int nt = 512; nt <= 1024; nt *= 2) {
-        const hipError_t e = hipFuncSetAttribute(plane_fn<T>(eb, ec, nt, lds), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute(plane_fn<T>(eb, ec, nt, lds), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

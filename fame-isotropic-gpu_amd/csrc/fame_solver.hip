@@ -356,6 +356,7 @@ static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q)
     q->W = eng == ENG_MFMA ? p.afrag[pi] : d.W;
     q->ntab = eng == ENG_MFMA ? nqt * ((m + 3) / 4) * 64 : p.n;
     q->mnl = fame_magic32(nl);
+    q->mn = fame_magic32(p.n);
     if (eng == ENG_STOCKHAM) { q->nst = d.nst; q->st = p.pst[pi]; q->sf = p.pst[pi] + d.nst; }
     q->n = p.n;
     return true;
@@ -395,6 +396,10 @@ fame_status fame_ctx::plane_setup() {
         if (!line_tile_ok(prec, eng, L)) { plane_ok[pi] = false; continue; }
         ltile[pi].eng = eng; ltile[pi].L = L; ltile[pi].P = g.na | 1;
         ctile[pi] = ltile[pi];
+        if (prec == 8) {
+            syn_ok = lds + 16 * (size_t)g.nc <= 160 * 1024 - 256;
+            if (syn_ok) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+        }
         HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng, lds) : fame_prepare_plane32(k.b.eng, k.c.eng, lds));
         /* before tuning: an FP64 plane that fills a CU alone pays where one
          * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
@@ -432,7 +437,6 @@ KLine fame_ctx::kline(int prec, int p0, const int* act, bool contract) const {
     k.f = prec == 8 ? (char*)F64 + 16 * k.fstride * p0 : (char*)F32 + 8 * k.fstride * p0;
     k.L = t.L; k.P = t.P;
     k.mLs = fame_magic32(prec == 8 ? t.L : t.L / 2);
-    k.half = N; k.off = 0;
     return k;
 }
 KPlane fame_ctx::kplane(int prec, int p0, const int* act) const {
@@ -445,6 +449,14 @@ KPlane fame_ctx::kplane(int prec, int p0, const int* act) const {
     k.invB = invBp[pi];
     k.tw = (char*)mtw[pi] + es * (size_t)g.nb * g.nc * p0;
     return k;
+}
+KSyn fame_ctx::ksyn(int p0) const {
+    KSyn a;
+    std::memset(&a, 0, sizeof(a));
+    a.k = kplane(8, p0, nullptr);
+    a.prob = prob_d + p0;
+    a.ostride = 3 * (size_t)N;
+    return a;
 }
 int fame_ctx::inner_blocks(int prec) const {
     const int pi = prec == 8 ? 0 : 1;
@@ -591,55 +603,23 @@ extern "C" fame_status fame_query(const fame_ctx* c, int* N, int* nk, int* len3)
     return FAME_OK;
 }
 
-/* reference layout (component-stacked, x fastest) -> kernel layout [c][b][a] */
-static size_t int_index(const GridDev& g, int x, int y, int z) {
-    if (g.general) return ((size_t)x * g.nb + y) * g.na + z;    /* [x][y][z] */
-    return x + (size_t)g.na * (y + (size_t)g.nb * z);            /* [z][y][x] */
+fame_status fame_ctx::spread_eps() {
+    HIPCHK(fame_launch_eps(g, eps_ref, eps_int, invB64, invB32, (double*)invBp[0], (float*)invBp[1], PP, stream));
+    return FAME_OK;
 }
 
 extern "C" fame_status fame_set_eps(fame_ctx* c, const double* eps) {
     if (!c || !eps) FAIL(FAME_ERR_ARG, "fame_set_eps: null argument");
-    const int Nx = c->lat.grid_nums[0], Ny = c->lat.grid_nums[1], Nz = c->lat.grid_nums[2];
-    const size_t N = c->N;
-    std::vector<double> e(3 * N), ib(3 * N);
-    std::vector<float> ib32(3 * N);
-    for (int comp = 0; comp < 3; ++comp)
-        for (int z = 0; z < Nz; ++z)
-            for (int y = 0; y < Ny; ++y)
-                for (int x = 0; x < Nx; ++x) {
-                    size_t r = x + (size_t)Nx * (y + (size_t)Ny * z);
-                    double v = eps[comp * N + r];
-                    if (!(v > 0)) FAIL(FAME_ERR_ARG, "fame_set_eps: permittivity must be positive");
-                    size_t q = comp * N + int_index(c->g, x, y, z);
-                    e[q] = v; ib[q] = 1.0 / v; ib32[q] = (float)(1.0 / v);
-                }
-    /* 1 / (N eps) in the plane layout [component][a][c][b] of pitch PP */
-    std::vector<double> pb;
-    std::vector<float> pb32;
-    if (c->plane_ok[0] || c->plane_ok[1]) {
-        pb.assign(3 * (size_t)c->CS, 0.0); pb32.assign(3 * (size_t)c->CS, 0.0f);
-        const size_t nl = (size_t)c->g.nb * c->g.nc;
-        const double sc = 1.0 / (double)N;
-        for (int comp = 0; comp < 3; ++comp)
-            for (size_t l = 0; l < nl; ++l)
-                for (int a = 0; a < c->g.na; ++a) {
-                    const size_t d = (size_t)comp * c->CS + (size_t)a * c->PP + l;
-                    pb[d] = ib[comp * N + l * c->g.na + a] * sc; pb32[d] = (float)pb[d];
-                }
-    }
-    /* the context's stream may still be running kernels that read the old values */
+    const size_t n = 3 * (size_t)c->N;
+    bool ok = true;
+    for (size_t i = 0; i < n; ++i) ok &= eps[i] > 0;
+    if (!ok) FAIL(FAME_ERR_ARG, "fame_set_eps: permittivity must be positive");
+    /* the context's stream may still be running kernels that read the old values;
+     * the copy is ordered on it (contexts of fame_eigs_many run on their own
+     * streams), and the caller's array is free once the stream is drained      */
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    /* ordered on the context's stream (contexts of fame_eigs_many run on their
-     * own streams); the host staging vectors live until the stream is drained */
-    HIPCHK(hipMemcpyAsync(c->eps_int, e.data(), sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->eps_ref, eps, sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->invB64, ib.data(), sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->invB32, ib32.data(), sizeof(float) * 3 * N, hipMemcpyHostToDevice, c->stream));
-    if (!pb.empty()) {
-        HIPCHK(hipMemcpyAsync(c->invBp[0], pb.data(), sizeof(double) * pb.size(), hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->invBp[1], pb32.data(), sizeof(float) * pb32.size(), hipMemcpyHostToDevice, c->stream));
-    }
+    HIPCHK(hipMemcpyAsync(c->eps_ref, eps, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    CHK(c->spread_eps());
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_eps = true;
     ++c->eps_ver;
@@ -852,14 +832,43 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
     const int N = c->N, Nd = c->nd[ik];
     double2* xin = (double2*)c->ref64[0];
     double2* yout = (double2*)c->ref64[1];
+    const size_t pn = (size_t)c->g.nb * c->g.nc;
     switch (op) {
         case FAME_OP_QR:
+            if (c->syn_ok) {
+                /* vector and field straight in the reference's layouts; a Simple
+                 * grid's field needs the transpose                           */
+                KLine k = c->kline(8, ik, nullptr);
+                k.x = x; k.ref = 1;
+                HIPCHK(c->launch_line(k, 1, LINE_EX_PLAIN, 8, 1));
+                KSyn s = c->ksyn(ik);
+                s.out = (double2*)y;
+                HIPCHK(fame_launch_syn(s, c->g.general ? SYN_REF : SYN_FIELD, 1, c->stream));
+                if (!c->g.general)
+                    HIPCHK(fame_launch_transpose((const double2*)k.f, (double2*)y, c->g.na, (int)pn, c->PP, c->g.na, c->CS, N, 3, 0, 0,
+                                                 nullptr, 1, c->stream));
+                break;
+            }
+            [[fallthrough]];
         case FAME_OP_PR:
             HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
             CHK(c->qr_field(xin, ik, 1, op == FAME_OP_PR ? 1 : 0, nullptr));
             CHK(c->field_to_ref(c->F64 + (size_t)ik * 3 * N, y, 1, 3 * (size_t)N));
             break;
         case FAME_OP_QRS:
+            if (c->syn_ok) {
+                KLine k = c->kline(8, ik, nullptr, true);
+                KSyn s = c->ksyn(ik);
+                if (c->g.general) s.in = (const double2*)x;
+                else
+                    HIPCHK(fame_launch_transpose((const double2*)x, (double2*)k.f, (int)pn, c->g.na, c->g.na, c->PP, N, c->CS, 3, 0, 0,
+                                                 nullptr, 1, c->stream));
+                HIPCHK(fame_launch_ana(s, 1, c->stream));
+                k.xs = y; k.ref = 1;
+                HIPCHK(c->launch_line(k, 0, LINE_CO_PLAIN, 8, 1));
+                break;
+            }
+            [[fallthrough]];
         case FAME_OP_PRS:
             CHK(c->field_from_ref(x, c->F64 + (size_t)ik * 3 * N, 1));
             CHK(c->qrs_field(yout, ik, 1, op == FAME_OP_PRS ? 1 : 0, nullptr));
@@ -868,13 +877,11 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
         case FAME_OP_QBQ:
             if (c->plane[0]) {
                 KLine k = c->kline(8, ik, nullptr);
-                k.off = N - Nd; k.half = Nd;
-                k.x = x;
+                k.x = x; k.ref = 1;
                 HIPCHK(c->launch_line(k, 1, LINE_EX_PLAIN, 8, 1));
                 HIPCHK(c->launch_plane(c->kplane(8, ik, nullptr), 8, 1));
                 k = c->kline(8, ik, nullptr, true);
-                k.off = N - Nd; k.half = Nd;
-                k.xs = y;
+                k.xs = y; k.ref = 1;
                 HIPCHK(c->launch_line(k, 0, LINE_CO_PLAIN, 8, 1));
                 ++c->cnt_qbq64;
                 break;

@@ -109,3 +109,55 @@ def test_plane_tiles_are_refused_where_unavailable(gpu):
         with pytest.raises(F.FameError):
             S.set_tiles(prec, t)
     S.close()
+
+
+@pytest.mark.parametrize("lt,nx", GRIDS + [("face_centered_cubic", 96)], ids=lambda v: str(v))
+def test_one_way_planes_vs_oracle(gpu, lt, nx):
+    """Qr, Qrs, restored fields, residuals and the gradient, a generic wave vector and
+    Gamma in one batch: per problem strides, the reference's layouts, and a
+    permittivity that differs from cell to cell and component to component (its three
+    layouts).  1e-11 of the oracle; residuals and gradients are sums of such terms."""
+    import torch
+    fl, _ = _setup(lt, nx)
+    ks = np.array([[0.21, -0.13, 0.07], [0.0, 0.0, 0.0]])
+    Ts = [O.Tables(O.lattice_from(fl), k) for k in ks]
+    S = F.Solver(fl, max_batch=2)
+    N, nw = S.N, 3
+    rng = np.random.default_rng(5)
+    eps = 1.0 + 12.0 * rng.random(3 * N)
+    S.set_eps(eps)
+    S.set_wave_vectors(ks)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda")
+    v = _rand(3 * N, 11)
+    evr = np.zeros((2, nw, 2 * N), complex)
+    freq = np.array([[0.3, 0.7, 1.1], [0.4, 0.5, 0.9]])
+    for i, T in enumerate(Ts):
+        x = _rand(2 * T.Nd, 7 + i)
+        assert _rel(S.apply(F.OP_QR, i, dev(x)).cpu().numpy(), T.qr(x)) < 1e-11
+        assert _rel(S.apply(F.OP_QRS, i, dev(v)).cpu().numpy(), T.qrs(v)) < 1e-11
+        if (lt, nx) in GRIDS:       # the largest element's error of any QBQ, axis passes too, is 1.7e-11 at FCC 96
+            ref = T.qbq(1.0 / eps, x)
+            for op, bar in ((F.OP_QBQ, 1e-11), (F.OP_QBQ32, 2e-6)):
+                assert _rel(S.apply(op, i, dev(x)).cpu().numpy(), ref) < bar
+        for j in range(nw):
+            evr[i, j, :2 * T.Nd] = _rand(2 * T.Nd, 20 + 3 * i + j)
+    E = S.restore(dev(evr))
+    res = S.residuals(freq, E)
+    Eh = E.cpu().numpy()
+    g, w = np.zeros(3 * N), np.array([[1.0, 0.0, -0.5], [0.25, 2.0, 0.75]])
+    for i, T in enumerate(Ts):
+        sig = np.tile(T.get(3), 2)
+        for j in range(nw):
+            if i == 1 and j < 2:        # Gamma: two constant fields, then the bands
+                e = np.full(3 * N, 1.0 / np.sqrt(3 * N))
+            else:
+                e = T.qr(sig * evr[i, j - 2 * i, :2 * T.Nd]) / eps
+                e = e * np.linalg.norm(e)
+            assert _rel(Eh[i, j], e) < 1e-11
+            r = T.curlh(T.curl(Eh[i, j])) - freq[i, j] ** 2 * eps * Eh[i, j]
+            r = np.linalg.norm(r) / np.linalg.norm(Eh[i, j])
+            assert abs(res[i, j] - r) <= 1e-11 * r
+            a = np.abs(Eh[i, j]) ** 2
+            g -= w[i, j] * freq[i, j] ** 2 / (eps @ a) * a
+    assert _rel(S.eig_vjp(freq, E, w).cpu().numpy(), g) < 1e-11
+    S.close()
