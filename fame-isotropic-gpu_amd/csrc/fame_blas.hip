@@ -97,7 +97,7 @@ __global__ void k_cg_init_scal(CgScal* sc, const double* partials, int nblk, dou
     c.rr = s; c.rr0 = s; c.pap_re = c.pap_im = 0; c.alpha_re = c.alpha_im = 0; c.beta = 0;
     c.tol2 = tol * tol; c.iters = 1; c.maxit = maxit;
     c.active = (!mask || mask[p]) && (s > c.tol2) && (1 <= maxit);
-    c.pend = 0;
+    c.pend = 0; c.upd = 0;
     sc[p] = c;
     active[p] = c.active;
 }
@@ -155,21 +155,18 @@ __global__ void k_cg_alpha(CgScal* sc, const double* pap, int npap, const int* a
     c.pend = 1;
 }
 
-/* <r,r> of the residual the contracting pass updated (slot 3 of its 6-double
- * block partials): b = r1 / r0 and the stopping rule (CG.cu:66-78) */
-__global__ void k_cg_beta(CgScal* sc, const double* partials, int nblk, int* active) {
+/* <r,r> of the residual the contracting pass updated (its block sums, every step
+ * doubles): b = r1 / r0 and the stopping rule (CG.cu:66-78) */
+__global__ void k_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int* active) {
     const int p = blockIdx.x;
     if (!active[p]) return;
     double v[1] = {0.0};
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) v[0] += partials[((size_t)p * nblk + b) * 6 + 3];
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) v[0] += partials[((size_t)p * nblk + b) * step];
     block_sum_all<1>(v);
     if (threadIdx.x != 0) return;
     CgScal& c = sc[p];
-    const double s = v[0];
-    c.beta = s / c.rr;
-    c.rr = s;
-    c.iters += 1;
-    c.active = (s > c.tol2) && (c.iters <= c.maxit);
+    cg_rule(v[0], c.tol2, c.maxit, c.rr, c.beta, c.iters, c.active);
+    c.upd = 0;
     active[p] = c.active;
 }
 
@@ -475,8 +472,8 @@ hipError_t fame_cg_alpha(CgScal* sc, const double* pap, int npap, int nprob, con
     hipLaunchKernelGGL(k_cg_alpha, dim3(nprob), dim3(RB), 0, s, sc, pap, npap, active);
     return hipGetLastError();
 }
-hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_beta, dim3(nprob), dim3(RB), 0, s, sc, partials, nblk, active);
+hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s) {
+    hipLaunchKernelGGL(k_cg_beta, dim3(nprob), dim3(RB), 0, s, sc, partials, nblk, step, active);
     return hipGetLastError();
 }
 hipError_t fame_cg_alpha_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s) {
@@ -624,7 +621,7 @@ __global__ void k_cg_init_scal2(CgScal* sc, const double* partials, int nblk, do
     c.rr = s; c.rr0 = s; c.pap_re = c.pap_im = 0; c.alpha_re = c.alpha_im = 0; c.beta = 0;
     c.tol2 = fmax(tol * tol, reltol * reltol * s); c.iters = 1; c.maxit = maxit;
     c.active = (!mask || mask[p]) && (s > c.tol2) && (1 <= maxit);
-    c.pend = 0;
+    c.pend = 0; c.upd = 0;
     sc[p] = c;
     active[p] = c.active;
 }

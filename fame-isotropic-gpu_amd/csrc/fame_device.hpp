@@ -96,6 +96,37 @@ __device__ __forceinline__ void batched_loop(int total, Ld ld, Use use) {
     }
 }
 
+/* the same in two parts: the first group's loads, and the loop that begins with
+ * using them; what stands between runs under the loads */
+template <int U, typename Ld, typename R>
+__device__ __forceinline__ void batch_load(int i0, int total, Ld ld, R (&r)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int idx = i0 + u * (int)blockDim.x;
+        if (idx < total) r[u] = ld(idx);
+    }
+}
+template <int U, typename Ld, typename Use, typename R>
+__device__ __forceinline__ void batched_loop_from(int total, R (&r)[U], Ld ld, Use use) {
+    for (int i0 = (int)threadIdx.x; i0 < total;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int idx = i0 + u * (int)blockDim.x;
+            if (idx < total) use(idx, r[u]);
+        }
+        i0 += U * (int)blockDim.x;
+        batch_load<U>(i0, total, ld, r);
+    }
+}
+/* ... with mid() (every thread, barriers included) there; false ends the loop */
+template <int U, typename Ld, typename Mid, typename Use>
+__device__ __forceinline__ bool batched_loop_over(int total, Ld ld, Mid mid, Use use) {
+    decltype(ld(0)) r[U];
+    batch_load<U>((int)threadIdx.x, total, ld, r);
+    if (!mid()) return false;
+    batched_loop_from<U>(total, r, ld, use);
+    return true;
+}
 
 enum { PRE_NONE = 0, PRE_CHIRP = 1, PRE_CHIRP_CONJ = 2, PRE_BM = 3, PRE_BP = 4 };
 enum { POST_NONE = 0, POST_CHIRP = 1, POST_CHIRP_CONJ = 2 };

@@ -77,6 +77,7 @@ struct fame_ctx {
     double* partials2 = nullptr;  /* [problem][inner blocks][2, or 6 inside CG] */
     double* pap_part = nullptr;   /* [problem][3][outer blocks]: <p,QBQ p> block sums of the outer pass */
     CgScal* cgsc = nullptr;
+    CgScal* cgsc2 = nullptr;      /* the plane path's second copy (expansion -> contraction) */
     int* active = nullptr;
     int* mask = nullptr;
     double* scal = nullptr;       /* 64 doubles per problem of small device scalars */
@@ -134,7 +135,10 @@ struct fame_ctx {
     KSyn ksyn(int p0) const;
     /* eps_ref (device) into the kernels' layouts */
     fame_status spread_eps();
-    int inner_blocks(int prec) const;   /* blocks per problem whose sums the contracting pass leaves */
+    int inner_blocks(int prec) const;
+    /* the plane path's inner kernels form alpha and beta themselves */
+    bool folds(int prec) const;
+    KLine cg_line(int prec, int p0, bool contract, void* p, void* r, void* x) const;   /* blocks per problem whose sums the contracting pass leaves */
     KInner kin(int prec, int p0, const int* act, int list) const;
     KAxis kmid(int prec, int p0, const int* act, int list) const;
     KAxis kout(int prec, int p0, const int* act, int list) const;

@@ -29,7 +29,18 @@ struct CgScal {
     int maxit;
     int active;       /* 1 while iterating                                      */
     int pend;         /* 1 when x still lacks alpha p of the last iteration    */
+    int upd;          /* 1 when rr, beta, iters and active still lack the last iteration's <r,r> */
 };
+
+#ifdef __HIPCC__
+/* b = r1 / r0 and the stopping rule (CG.cu:66-78) from the new <r, r> */
+__device__ __forceinline__ void cg_rule(double s, double tol2, int maxit, double& rr, double& beta, int& iters, int& active) {
+    beta = s / rr;
+    rr = s;
+    iters += 1;
+    active = (s > tol2) && (iters <= maxit);
+}
+#endif
 
 struct KInner {
     fame::GridDev g;
@@ -130,6 +141,15 @@ struct KLine {
     void* p32;
     double* rpart;               /* contract: block sums of <r, r>, every rstep doubles */
     int rstep;
+    /* scalars of the iteration formed by the inner kernels themselves (null: cgsc
+     * holds them): the expansion reads cgsc and the nrp sums of <r, r> per problem at
+     * rpart and writes sc2 and act_out, the contraction reads sc2 and the npap sums
+     * of <p, QBQ p> per problem at pap and writes cgsc                          */
+    CgScal* sc2;
+    CgScal* sc1;                 /* cgsc, for the contraction's write           */
+    int* act_out;
+    const double* pap;
+    int nrp, npap;
 };
 struct KPlane {
     fame::GridDev g;
@@ -253,7 +273,7 @@ hipError_t fame_cg_init_scal(CgScal* sc, const double* partials, int nblk, doubl
  * the active flags from the exact <r,r> of the updated residual (slot 3 of the
  * inner partials) */
 hipError_t fame_cg_alpha(CgScal* sc, const double* pap, int npap, int nprob, const int* active, hipStream_t s);
-hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s);
+hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s);
 hipError_t fame_cg_alpha_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s);
 hipError_t fame_cg_finish_x(void* x, const void* p, const CgScal* sc, size_t n, size_t stride, int nprob, int prec,
                             hipStream_t s);

@@ -28,6 +28,20 @@ __device__ __forceinline__ PlaneStage load_stage(CStage* p) {
     return s;
 }
 
+/* One scalar load from each 64-byte line of a kernel's arguments (BYTES of them),
+ * all under way together, at its start: the pass descriptors that a small grid's
+ * block reads one after another between its barriers then come from the scalar
+ * cache instead of one memory round trip each                                 */
+template <int BYTES>
+__device__ __forceinline__ void touch_args() {
+    typedef const __attribute__((address_space(4))) unsigned CUint;
+    CUint* a = (CUint*)__builtin_amdgcn_kernarg_segment_ptr();
+    unsigned v = 0;
+#pragma unroll
+    for (int i = 0; i < BYTES / 4; i += 16) v ^= a[i];
+    asm volatile("" :: "s"(v));
+}
+
 /* lines per round of a pass with nbf butterflies per line, NBT per thread, and
  * id / lpr as (id + 1/2) * (1 / lpr): exact, since the quotient is below 2^13 and
  * its distance from an integer at least 1 / (2 lpr)                          */

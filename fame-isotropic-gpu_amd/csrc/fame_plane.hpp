@@ -128,6 +128,28 @@ struct InnerLds {
 };
 __device__ __forceinline__ int inner_tile() { return xcd_tile(); }
 
+/* CG scalars inside the inner kernels.  A reduction kernel of one block per problem
+ * took 4.4 us, twice per iteration (of 33 us on a 32^3 grid, of 110 at FCC 96);
+ * here every block sums the up to 2048 block sums of the kernel before (from L2,
+ * behind the loads of its tables), all in the same order, so that all hold the
+ * same alpha and beta.  State goes back and forth between two copies, each kernel
+ * reading one and its first block writing the other.
+ * wave_part: this thread's share, reduced over its wave into red; the block's
+ * next barrier makes it visible to wave_total                                */
+__device__ __forceinline__ void wave_part(const double* v, int n, double* red) {
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n; i += FFT_THREADS) s += v[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+}
+__device__ __forceinline__ double wave_total(const double* red) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < FFT_THREADS / 64; ++w) s += red[w];
+    return s;
+}
+
 /* copy the tables of a block's lines l0.. (at most L) into LDS */
 template <typename T2>
 __device__ __forceinline__ void inner_tables(const KLine& k, const InnerLds<T2>& m, int p, int l0, int nl) {
@@ -143,22 +165,30 @@ __device__ __forceinline__ void inner_tables(const KLine& k, const InnerLds<T2>&
     for (int i = threadIdx.x; i < nl * tpl; i += blockDim.x) m.tw[i] = ts[i];
 }
 
+/* field by field: a struct assignment goes through scratch */
+__device__ __forceinline__ void cg_copy(CgScal& o, const CgScal& c) {
+    o.rr = c.rr; o.rr0 = c.rr0; o.pap_re = c.pap_re; o.pap_im = c.pap_im;
+    o.alpha_re = c.alpha_re; o.alpha_im = c.alpha_im; o.beta = c.beta; o.tol2 = c.tol2;
+    o.iters = c.iters; o.maxit = c.maxit; o.active = c.active; o.pend = c.pend; o.upd = c.upd;
+}
+
 /* F = twid . IFFT_a(Pi x), field in the plane layout.  EX_CG: x is the search
  * direction p, and x_sol += alpha p (pending), p = r + beta p ride on the read;
  * EX_FX: x += fx32 + alpha fp32 of the FP32 solve that just ended.          */
 template <typename T, int ENG, int PIK, int MODE>
 __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
     typedef typename C2<T>::T2 T2;
+    touch_args<sizeof(KLine)>();
     const int p = blockIdx.y;
-    if (k.active && !k.active[p]) return;
     const int nlines = k.g.nb * k.g.nc, na = k.g.na, L = k.L, P = k.P;
     const int tile = inner_tile(), l0 = tile * L;
     if (l0 >= nlines) return;
+    const bool fold = MODE == EX_CG && k.sc2;
+    if (!fold && k.active && !k.active[p]) return;
+    __shared__ double red[FFT_THREADS / 64];
     const int nl = min(L, nlines - l0);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const InnerLds<T2> m(smem_raw, na, k.a.ntab, L, P);
-    inner_tables<T2>(k, m, p, l0, nl);
-    __syncthreads();
     const bool gam = k.prob[p].gamma != 0;
     const double iha2 = 2.0 * k.g.iha;
     T2* X = reinterpret_cast<T2*>(const_cast<void*>(k.x)) + (size_t)p * k.xstride;
@@ -166,11 +196,32 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
      * [half + f - off]; the reference's layout leaves out mode 0 at Gamma     */
     const unsigned off = k.ref && gam ? 1u : 0u, half = (unsigned)k.g.N - off;
     T beta = 0, al = 0;
-    bool pend = false;
-    if (MODE != EX_PLAIN) {
-        const CgScal& cs = k.cgsc[p];
-        beta = (T)cs.beta; al = (T)cs.alpha_re; pend = cs.pend != 0;
-    }
+    bool pend = true;
+    /* under the first loads of the vectors: the tables and the scalars */
+    auto start = [&]() -> bool {
+        if (fold) wave_part(k.rpart + (size_t)p * k.nrp, k.nrp, red);
+        inner_tables<T2>(k, m, p, l0, nl);
+        __syncthreads();
+        if (MODE == EX_PLAIN) return true;
+        const CgScal& c = k.cgsc[p];
+        double bd = c.beta;
+        pend = c.pend != 0;
+        al = (T)c.alpha_re;
+        if (fold) {
+            double rr = c.rr;
+            int it = c.iters, act = c.active;
+            if (act && c.upd) cg_rule(wave_total(red), c.tol2, c.maxit, rr, bd, it, act);
+            if (tile == 0 && threadIdx.x == 0) {
+                CgScal& o = k.sc2[p];
+                cg_copy(o, c);
+                o.rr = rr; o.beta = bd; o.iters = it; o.active = act; o.upd = 0;
+                k.act_out[p] = act;
+            }
+            if (!act) return false;
+        }
+        beta = (T)bd;
+        return true;
+    };
     T2* S = m.S;
     const int tot = nl * na;
     auto put = [&](int line, int a, unsigned f, T2 x1, T2 x2) {
@@ -182,6 +233,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) S[(c * L + line) * P + a] = rnd<T2>(u[c]);
     };
+    bool on = true;
     if constexpr (MODE == EX_CG) {
         const T2* R = reinterpret_cast<const T2*>(k.r) + (size_t)p * k.xstride;
         T2* Y = reinterpret_cast<T2*>(k.xs) + (size_t)p * k.xstride;
@@ -191,7 +243,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
                 done = true;
                 /* two consecutive modes of a line per thread, 16-byte accesses */
                 struct In { float4 x1, x2, r1, r2, s1, s2; };
-                batched_loop<1>(tot >> 1,
+                on = batched_loop_over<1>(tot >> 1,
                     [&](int i) -> In {
                         const unsigned f = (unsigned)(l0 * na + 2 * i);
                         In d;
@@ -205,6 +257,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
                         }
                         return d;
                     },
+                    start,
                     [&](int i, const In& d) {
                         const int line = udiv(2 * i, k.g.m_na), a = 2 * i - line * na;
                         const unsigned f = (unsigned)(l0 * na + 2 * i);
@@ -227,7 +280,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
         }
         if (!done) {
             struct In { T2 x1, x2, r1, r2, s1, s2; };
-            batched_loop<2>(tot,
+            on = batched_loop_over<2>(tot,
                 [&](int i) -> In {
                     const unsigned f = (unsigned)(l0 * na + i);
                     In d;
@@ -236,6 +289,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
                     if (pend) { d.s1 = Y[f]; d.s2 = Y[half + f]; }
                     return d;
                 },
+                start,
                 [&](int i, const In& d) {
                     const int line = udiv(i, k.g.m_na), a = i - line * na;
                     const unsigned f = (unsigned)(l0 * na + i);
@@ -257,7 +311,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
         const float2* FP = MODE == EX_FX ? reinterpret_cast<const float2*>(k.fp32) + (size_t)p * k.xstride : nullptr;
         const double* sg = k.sig ? k.sig + (size_t)p * k.g.N : nullptr;
         struct In { T2 x1, x2; float2 s1, s2, v1, v2; };
-        batched_loop<2>(tot,
+        on = batched_loop_over<2>(tot,
             [&](int i) -> In {
                 const unsigned f = (unsigned)(l0 * na + i);
                 In d;
@@ -272,6 +326,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
                 }
                 return d;
             },
+            start,
             [&](int i, const In& d) {
                 const int line = udiv(i, k.g.m_na), a = i - line * na;
                 const unsigned f = (unsigned)(l0 * na + i);
@@ -289,6 +344,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
                 put(line, a, f, x1, x2);
             });
     }
+    if (!on) return;
     if (nl < L) {   /* lines past the last one transform as zeros */
         T2 z; z.x = 0; z.y = 0;
         for (int i = threadIdx.x; i < 3 * (L - nl) * na; i += blockDim.x) {
@@ -341,26 +397,54 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
 template <typename T, int ENG, int PIK, int MODE>
 __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
     typedef typename C2<T>::T2 T2;
+    touch_args<sizeof(KLine)>();
     const int p = blockIdx.y;
-    if (k.active && !k.active[p]) return;
     const int nlines = k.g.nb * k.g.nc, na = k.g.na, L = k.L, P = k.P;
     const int tile = inner_tile(), l0 = tile * L;
     if (l0 >= nlines) return;
+    const bool fold = MODE == CO_CG && k.sc2;
+    if (!fold && k.active && !k.active[p]) return;
+    __shared__ double red[FFT_THREADS / 64];
     const int nl = min(L, nlines - l0);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const InnerLds<T2> m(smem_raw, na, k.a.ntab, L, P);
-    inner_tables<T2>(k, m, p, l0, nl);
-    __syncthreads();
+    T al = 0;
+    auto start = [&]() -> bool {
+        if (fold) wave_part(k.pap + (size_t)p * k.npap, k.npap, red);
+        inner_tables<T2>(k, m, p, l0, nl);
+        __syncthreads();
+        if (fold) {
+            const CgScal& c = k.sc2[p];
+            const int act = c.active;
+            /* a = r1 / dot  (CG.cu:60-63); the quadratic form is real */
+            const double pq = wave_total(red), a = c.rr / pq;
+            if (tile == 0 && threadIdx.x == 0) {
+                CgScal& o = k.sc1[p];
+                cg_copy(o, c);
+                if (act) {
+                    o.pap_re = pq; o.pap_im = 0.0;
+                    o.alpha_re = a; o.alpha_im = 0.0;
+                    o.pend = 1; o.upd = 1;
+                }
+            }
+            if (!act) return false;
+            al = (T)a;
+        } else if (MODE == CO_CG) {
+            al = (T)k.cgsc[p].alpha_re;
+        }
+        return true;
+    };
     const bool gam = k.prob[p].gamma != 0;
     const double iha2 = 2.0 * k.g.iha;
     const int tpl = inner_tw_per_line(na);
     T2* S = m.S;
     const T2* F = reinterpret_cast<const T2*>(k.f) + (size_t)p * k.fstride + l0;
     const unsigned PP = (unsigned)k.PP, cs = (unsigned)k.cs;
+    bool on;
     if constexpr (sizeof(T) == 4) {
         struct In { float4 v[3]; };
         const int Lh = L >> 1;
-        batched_loop<1>(Lh * na,
+        on = batched_loop_over<1>(Lh * na,
             [&](int i) -> In {
                 const int a = udiv(i, k.mLs), line = 2 * (i - a * Lh);
                 const unsigned f = (unsigned)a * PP + line;
@@ -373,6 +457,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
                 }
                 return d;
             },
+            start,
             [&](int i, const In& d) {
                 const int a = udiv(i, k.mLs), line = 2 * (i - a * Lh);
                 const T2* t0 = m.tw + line * tpl;
@@ -389,7 +474,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
             });
     } else {
         struct In { T2 v[3]; };
-        batched_loop<2>(L * na,
+        on = batched_loop_over<2>(L * na,
             [&](int i) -> In {
                 const int a = udiv(i, k.mLs), line = i - a * L;
                 const unsigned f = (unsigned)a * PP + line;
@@ -401,6 +486,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
                 }
                 return d;
             },
+            start,
             [&](int i, const In& d) {
                 const int a = udiv(i, k.mLs), line = i - a * L;
                 const T2* t0 = m.tw + line * tpl;
@@ -410,13 +496,15 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
                 for (int c = 0; c < 3; ++c) S[(c * L + line) * P + a] = cmulc(d.v[c], w);
             });
     }
-    line_transform<T, T2, ENG, false>(S, 3 * L, P, 1, k.a, m.W);
-    __syncthreads();
+    if (!on) return;
+    auto transform = [&]() -> bool {
+        line_transform<T, T2, ENG, false>(S, 3 * L, P, 1, k.a, m.W);
+        __syncthreads();
+        return true;
+    };
     const unsigned off = k.ref && gam ? 1u : 0u, half = (unsigned)k.g.N - off;
     const int tot = nl * na;
     double rn = 0.0;
-    T al = 0;
-    if (MODE == CO_CG) al = (T)k.cgsc[p].alpha_re;
     auto take = [&](int line, int a, unsigned f, T2& o1, T2& o2) {
         double2 y1 = make_double2(0, 0), y2 = make_double2(0, 0);
         if (!(gam && f == 0)) {
@@ -426,54 +514,56 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
         o1 = rnd<T2>(y1); o2 = rnd<T2>(y2);
     };
     if constexpr (MODE == CO_CG) {
+        /* the residual's first group is loaded before the transform */
         T2* R = reinterpret_cast<T2*>(k.r) + (size_t)p * k.xstride;
-        bool done = false;
+        struct In1 { T2 r1, r2; };
+        struct In2 { float4 r1, r2; };
+        auto ld1 = [&](int i) -> In1 {
+            const unsigned f = (unsigned)(l0 * na + i);
+            In1 d;
+            d.r1 = R[f]; d.r2 = R[half + f];
+            return d;
+        };
+        auto use1 = [&](int i, const In1& d) {
+            const int line = udiv(i, k.g.m_na), a = i - line * na;
+            const unsigned f = (unsigned)(l0 * na + i);
+            T2 o1, o2, r1 = d.r1, r2 = d.r2;
+            take(line, a, f, o1, o2);
+            r1.x -= al * o1.x; r1.y -= al * o1.y;
+            r2.x -= al * o2.x; r2.y -= al * o2.y;
+            rn += (double)r1.x * r1.x + (double)r1.y * r1.y + (double)r2.x * r2.x + (double)r2.y * r2.y;
+            R[f] = r1; R[half + f] = r2;
+        };
         if constexpr (sizeof(T) == 4) {
-            if (!(na & 1) && al16(R) && !(half & 1)) {
-                done = true;
-                struct In { float4 r1, r2; };
-                batched_loop<1>(tot >> 1,
-                    [&](int i) -> In {
-                        const unsigned f = (unsigned)(l0 * na + 2 * i);
-                        In d;
-                        d.r1 = *reinterpret_cast<const float4*>(R + f);
-                        d.r2 = *reinterpret_cast<const float4*>(R + half + f);
-                        return d;
-                    },
-                    [&](int i, const In& d) {
-                        const int line = udiv(2 * i, k.g.m_na), a = 2 * i - line * na;
-                        const unsigned f = (unsigned)(l0 * na + 2 * i);
-                        float2 a1, a2, b1, b2;
-                        take(line, a, f, a1, a2);
-                        take(line, a + 1, f + 1, b1, b2);
-                        const float4 r1 = make_float4(d.r1.x - al * a1.x, d.r1.y - al * a1.y, d.r1.z - al * b1.x, d.r1.w - al * b1.y);
-                        const float4 r2 = make_float4(d.r2.x - al * a2.x, d.r2.y - al * a2.y, d.r2.z - al * b2.x, d.r2.w - al * b2.y);
-                        rn += (double)r1.x * r1.x + (double)r1.y * r1.y + (double)r1.z * r1.z + (double)r1.w * r1.w +
-                              (double)r2.x * r2.x + (double)r2.y * r2.y + (double)r2.z * r2.z + (double)r2.w * r2.w;
-                        *reinterpret_cast<float4*>(R + f) = r1;
-                        *reinterpret_cast<float4*>(R + half + f) = r2;
-                    });
-            }
-        }
-        if (!done) {
-            struct In { T2 r1, r2; };
-            batched_loop<2>(tot,
-                [&](int i) -> In {
-                    const unsigned f = (unsigned)(l0 * na + i);
-                    In d;
-                    d.r1 = R[f]; d.r2 = R[half + f];
-                    return d;
-                },
-                [&](int i, const In& d) {
-                    const int line = udiv(i, k.g.m_na), a = i - line * na;
-                    const unsigned f = (unsigned)(l0 * na + i);
-                    T2 o1, o2, r1 = d.r1, r2 = d.r2;
-                    take(line, a, f, o1, o2);
-                    r1.x -= al * o1.x; r1.y -= al * o1.y;
-                    r2.x -= al * o2.x; r2.y -= al * o2.y;
-                    rn += (double)r1.x * r1.x + (double)r1.y * r1.y + (double)r2.x * r2.x + (double)r2.y * r2.y;
-                    R[f] = r1; R[half + f] = r2;
+            auto ld2 = [&](int i) -> In2 {
+                const unsigned f = (unsigned)(l0 * na + 2 * i);
+                In2 d;
+                d.r1 = *reinterpret_cast<const float4*>(R + f);
+                d.r2 = *reinterpret_cast<const float4*>(R + half + f);
+                return d;
+            };
+            const bool pairs = !(na & 1) && al16(R) && !(half & 1);
+            In2 d[1];
+            if (pairs) batch_load<1>((int)threadIdx.x, tot >> 1, ld2, d);
+            transform();
+            if (pairs)
+                batched_loop_from<1>(tot >> 1, d, ld2, [&](int i, const In2& d) {
+                    const int line = udiv(2 * i, k.g.m_na), a = 2 * i - line * na;
+                    const unsigned f = (unsigned)(l0 * na + 2 * i);
+                    float2 a1, a2, b1, b2;
+                    take(line, a, f, a1, a2);
+                    take(line, a + 1, f + 1, b1, b2);
+                    const float4 r1 = make_float4(d.r1.x - al * a1.x, d.r1.y - al * a1.y, d.r1.z - al * b1.x, d.r1.w - al * b1.y);
+                    const float4 r2 = make_float4(d.r2.x - al * a2.x, d.r2.y - al * a2.y, d.r2.z - al * b2.x, d.r2.w - al * b2.y);
+                    rn += (double)r1.x * r1.x + (double)r1.y * r1.y + (double)r1.z * r1.z + (double)r1.w * r1.w +
+                          (double)r2.x * r2.x + (double)r2.y * r2.y + (double)r2.z * r2.z + (double)r2.w * r2.w;
+                    *reinterpret_cast<float4*>(R + f) = r1;
+                    *reinterpret_cast<float4*>(R + half + f) = r2;
                 });
+            else
+                batched_loop<2>(tot, ld1, use1);
+        } else {
+            batched_loop_over<2>(tot, ld1, transform, use1);
         }
     } else if constexpr (MODE == CO_RES) {
         const T2* B = reinterpret_cast<const T2*>(k.rb) + (size_t)p * k.xstride;
@@ -481,13 +571,14 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
         float2* P32 = reinterpret_cast<float2*>(k.p32) + (size_t)p * k.xstride;
         float2* X32 = reinterpret_cast<float2*>(k.xs) + (size_t)p * k.xstride;
         struct In { T2 b1, b2; };
-        batched_loop<2>(tot,
+        batched_loop_over<2>(tot,
             [&](int i) -> In {
                 const unsigned f = (unsigned)(l0 * na + i);
                 In d;
                 d.b1 = B[f]; d.b2 = B[half + f];
                 return d;
             },
+            transform,
             [&](int i, const In& d) {
                 const int line = udiv(i, k.g.m_na), a = i - line * na;
                 const unsigned f = (unsigned)(l0 * na + i);
@@ -504,6 +595,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
             });
     } else {
         T2* Y = reinterpret_cast<T2*>(k.xs) + (size_t)p * k.xstride;
+        transform();
         for (int i = threadIdx.x; i < tot; i += blockDim.x) {
             const int line = udiv(i, k.g.m_na), a = i - line * na;
             const unsigned f = (unsigned)(l0 * na + i);
@@ -513,7 +605,6 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
         }
     }
     if (MODE != CO_PLAIN) {
-        __shared__ double red[FFT_THREADS / 64];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) rn += __shfl_xor(rn, o);
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rn;
@@ -591,6 +682,7 @@ __global__ void __launch_bounds__(TB) k_plane(KPlane k) {
     typedef typename C2<T>::T2 T2;
     /* blocks of one XCD (x mod 8) take a run of consecutive planes, problem by
      * problem: the problem's middle twiddles stay in that XCD's L2            */
+    touch_args<sizeof(KPlane)>();
     const int npl = 3 * k.g.na;
     const int id = xcd_tile();
     if (id >= npl * k.nprob) return;

@@ -373,7 +373,14 @@ fame_status fame_ctx::plane_setup() {
         const int prec = pi == 0 ? 8 : 4;
         KPlane& k = kpl[pi];
         std::memset(&k, 0, sizeof(k));
-        auto engine = [&](int axis) { return (ax[axis][0].blue || eng_forced == 1) ? ENG_MFMA : ENG_STOCKHAM; };
+        /* up to 24 points the direct DFT on the matrix cores: one step between
+         * barriers instead of two or three passes.  The plane kernel of a 16^3 grid,
+         * one wave vector, 11.3 -> 8.7 us in FP64 (10.7 -> 8.1 in FP32), 24^3 12.2
+         * -> 10.6 (12.5 -> 9.4), eight 24^3 16.9 -> 15.4; from 32^3 on the passes
+         * win (eight in FP64 20.8 against 29.1)                               */
+        auto engine = [&](int axis) {
+            return (ax[axis][0].blue || eng_forced == 1 || (eng_forced < 0 && ax[axis][1].n > 0 && ax[axis][1].n <= 24)) ? ENG_MFMA : ENG_STOCKHAM;
+        };
         if (!plane_axis(ax[AX_MID][engine(AX_MID)], engine(AX_MID), pi, g.nc, &k.b)) continue;
         if (!plane_axis(ax[AX_OUTER][engine(AX_OUTER)], engine(AX_OUTER), pi, g.nb, &k.c)) continue;
         const size_t lds = fame_plane_lds(g.nb, g.nc, k.b.ntab + k.c.ntab, prec);
@@ -463,6 +470,24 @@ int fame_ctx::inner_blocks(int prec) const {
     return plane[pi] ? (g.nb * g.nc + ctile[pi].L - 1) / ctile[pi].L : nblk_in[pi];
 }
 
+/* every block of the expansion reads all block sums of <r, r>: 2048 of them are
+ * 16 KB beside the 100 KB of vector and field that such a grid's block moves     */
+bool fame_ctx::folds(int prec) const { return plane[prec == 8 ? 0 : 1] && inner_blocks(prec) <= 2048; }
+
+/* inner kernels of a CG iteration on the plane path */
+KLine fame_ctx::cg_line(int prec, int p0, bool contract, void* p, void* r, void* x) const {
+    KLine k = kline(prec, p0, active, contract);
+    k.x = p; k.r = r; k.xs = x;
+    k.cgsc = cgsc;
+    k.rpart = partials2; k.rstep = 1;
+    if (folds(prec)) {
+        k.sc2 = cgsc2; k.sc1 = cgsc; k.act_out = active;
+        k.nrp = inner_blocks(prec);
+        k.pap = pap_part; k.npap = 3 * g.na;
+    }
+    return k;
+}
+
 extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int device, fame_ctx** out) {
     if (!lat || !out || max_batch < 1) FAIL(FAME_ERR_ARG, "fame_create: null argument or max_batch < 1");
     for (int i = 0; i < 3; ++i) if (lat->grid_nums[i] < 1 || lat->grid_nums[i] > 1024) FAIL(FAME_ERR_ARG, "grid_nums out of range");
@@ -537,14 +562,17 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
     A(c->F32, 8 * 3 * NF * B);
     if (c->plane_ok[0] || c->plane_ok[1]) {
         const size_t nl = (size_t)g.nb * g.nc, tpl = inner_tw_per_line(g.na);
-        A(c->ltab, sizeof(LineTab) * nl * B);
-        for (int pi = 0; pi < 2; ++pi) {
-            const size_t es = pi ? 8 : 16;
-            A(c->invBp[pi], es / 2 * 3 * (size_t)c->CS);
-            A(c->ltw[pi], es * nl * tpl * B);
-            A(c->mtw[pi], es * nl * B);
-        }
-        A(c->eatab, 16 * (size_t)g.na);
+        /* the plane path's tables in one allocation (each costs the host 10 us) */
+        struct { void** p; size_t n; } part[] = {
+            {(void**)&c->ltab, sizeof(LineTab) * nl * B}, {(void**)&c->eatab, 16 * (size_t)g.na}, {(void**)&c->cgsc2, sizeof(CgScal) * B},
+            {(void**)&c->invBp[0], 8 * 3 * (size_t)c->CS}, {(void**)&c->invBp[1], 4 * 3 * (size_t)c->CS},
+            {(void**)&c->ltw[0], 16 * nl * tpl * B}, {(void**)&c->ltw[1], 8 * nl * tpl * B},
+            {(void**)&c->mtw[0], 16 * nl * B}, {(void**)&c->mtw[1], 8 * nl * B}};
+        size_t total = 0;
+        for (const auto& q : part) total += (q.n + 255) & ~(size_t)255;
+        char* base = nullptr;
+        A(base, total);
+        for (const auto& q : part) { *q.p = base; base += (q.n + 255) & ~(size_t)255; }
         std::vector<double> ea(2 * (size_t)g.na);
         for (int a = 0; a < g.na; ++a) {
             const long double x = 3.14159265358979323846264338327950288L * a / g.na;
@@ -973,7 +1001,7 @@ fame_status fame_ctx::tune(int prec) {
                     t.eng = eng; t.L = L;
                     KLine k = kline(prec, 0, nullptr, contract);
                     k.x = x; k.r = r; k.xs = y; k.cgsc = cgsc;
-                    k.rpart = partials2 + 3; k.rstep = 6;
+                    k.rpart = partials2; k.rstep = 1;
                     float ms = 0;
                     if (!timed([&] { return launch_line(k, !contract, contract ? (int)LINE_CO_CG : (int)LINE_EX_CG, prec, nk); }, &ms)) {
                         st = FAME_ERR_HIP;
@@ -1135,6 +1163,8 @@ fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, do
             it += k;
         }
         done_it += chunk;
+        /* the last iteration's beta, count and flags, which the next expansion would form */
+        if (folds(prec)) HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), 1, nprob, active, stream));
         /* the whole scalar state comes back, so that the last check also
          * holds the final iteration counts (no read-back after the loop) */
         HIPCHK(hipMemcpyAsync(sc_h, cgsc, sizeof(CgScal) * nprob, hipMemcpyDeviceToHost, stream));
@@ -1175,17 +1205,14 @@ fame_status fame_ctx::cg_step_ap(int prec, void* p, void* r, void* x, void* Ap, 
  * <r,r>; beta and the flags from that exact norm */
 fame_status fame_ctx::cg_step_rc(int prec, void* p, void* r, void* x, int p0, int nprob, int npap) {
     if (plane[pix(prec)]) {
-        KLine k = kline(prec, p0, active);
-        k.x = p; k.r = r; k.xs = x; k.cgsc = cgsc;
-        HIPCHK(launch_line(k, 1, LINE_EX_CG, prec, nprob));
+        const bool fold = folds(prec);
+        HIPCHK(launch_line(cg_line(prec, p0, false, p, r, x), 1, LINE_EX_CG, prec, nprob));
         KPlane kp = kplane(prec, p0, active);
         kp.pap = pap_part;
         HIPCHK(launch_plane(kp, prec, nprob));
-        HIPCHK(fame_cg_alpha(cgsc, pap_part, npap, nprob, active, stream));
-        k = kline(prec, p0, active, true);
-        k.r = r; k.cgsc = cgsc; k.rpart = partials2 + 3; k.rstep = 6;
-        HIPCHK(launch_line(k, 0, LINE_CO_CG, prec, nprob));
-        HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), nprob, active, stream));
+        if (!fold) HIPCHK(fame_cg_alpha(cgsc, pap_part, npap, nprob, active, stream));
+        HIPCHK(launch_line(cg_line(prec, p0, true, p, r, x), 0, LINE_CO_CG, prec, nprob));
+        if (!fold) HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), 1, nprob, active, stream));
         return FAME_OK;
     }
     KInner ki = kin(prec, p0, active, LIST_INV);
@@ -1202,12 +1229,14 @@ fame_status fame_ctx::cg_step_rc(int prec, void* p, void* r, void* x, int p0, in
     kc.x = p; kc.y = r; kc.pikind = 0;
     kc.cg_r = r; kc.cgsc = cgsc; kc.partials = partials2;
     HIPCHK(fame_launch_inner(kc, 0, prec, nprob, stream));
-    HIPCHK(fame_cg_beta(cgsc, partials2, nblk_in[pix(prec)], nprob, active, stream));
+    HIPCHK(fame_cg_beta(cgsc, partials2 + 3, nblk_in[pix(prec)], 6, nprob, active, stream));
     return FAME_OK;
 }
 
 /* `count` CG iterations (CG.cu:53-78) on the masked batch, as cg_step_rc
- * when the outer pass can sum <p,Ap> (no Bluestein plan), else cg_step_ap.
+ * when the outer pass can sum <p,Ap> (no Bluestein plan), else cg_step_ap.  On the
+ * plane path an iteration is three kernels: the expansion and the contraction form
+ * beta and alpha themselves (folds).
  * The reference's alpha, beta and stopping rule are kept; the x and p updates
  * of iteration k are applied while iteration k+1 reads p anyway (k_cg_begin sets
  * p = r and beta = 0, so the first pass leaves p = r).  The last x update is

@@ -161,3 +161,22 @@ def test_one_way_planes_vs_oracle(gpu, lt, nx):
             g -= w[i, j] * freq[i, j] ** 2 / (eps @ a) * a
     assert _rel(S.eig_vjp(freq, E, w).cpu().numpy(), g) < 1e-11
     S.close()
+
+
+@pytest.mark.parametrize("prec", [8, 4])
+def test_cg_scalars_in_the_inner_kernels(gpu, prec):
+    """alpha and beta formed inside the inner kernels (up to 2048 blocks: 8 lines each
+    here) against the separate reduction kernels (2304 blocks of 4 lines): the sums
+    differ in order only, so the solutions of the 1e-12 solve agree to its accuracy."""
+    import torch
+    fl, eps = _setup("simple_cubic", 96)
+    S = F.Solver(fl, max_batch=1)
+    S.set_eps(eps)
+    S.set_wave_vectors(np.array([[0.21, -0.13, 0.07]]))
+    x = torch.from_numpy(_rand(2 * S.nd[0], 5)).to("cuda")
+    y = []
+    for lines in (4, 8):
+        S.set_tiles(prec, {"inner": (0, lines), "mid": (2, lines), "outer": (2, 512)})
+        y.append(S.apply(F.OP_INVAR if prec == 8 else F.OP_INVAR_MIXED, 0, x).cpu().numpy())
+    assert np.linalg.norm(y[0] - y[1]) < 1e-10 * np.linalg.norm(y[1])
+    S.close()
