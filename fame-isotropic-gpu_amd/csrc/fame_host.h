@@ -53,12 +53,13 @@ struct fame_ctx {
      * whether the solver takes it, the inner tiles (engine, lines per block) of
      * its expanding and contracting kernels, the launch templates, its tables */
     bool plane_ok[2] = {false, false}, plane[2] = {false, false};
-    bool syn_ok = false;          /* the FP64 one-way plane kernels (Qr, Qrs, restoration, residuals) */
     PassTile ltile[2], ctile[2];
     int PP = 0, CS = 0;           /* plane pitch and component stride (na PP)  */
     PlaneAxis laxis[2][2];        /* inner axis [precision][engine], n = 0 when not available */
     KPlane kpl[2];
+    PlaneAxis wide_ax[2];         /* b and c of the FP64 plane kernel's wide variant */
     void *invBp[2] = {nullptr, nullptr}, *ltw[2] = {nullptr, nullptr}, *mtw[2] = {nullptr, nullptr}, *eatab = nullptr;
+    double2* otw = nullptr;
     LineTab* ltab = nullptr;
     /* wave vectors */
     int nk = 0;

@@ -163,13 +163,14 @@ struct KPlane {
     PlaneAxis b, c;
     unsigned mnb;
     int nprob, nt;
+    int wide;                    /* FP64: the variant of at most 512 threads with 16 elements each */
 };
 
 /* what a one-way plane kernel (FP64) does after its inverse transforms (fame_plane64.hip) */
 enum { SYN_FIELD = 0, SYN_REF = 1, SYN_EPS = 2, SYN_RES = 3 };
 struct KSyn {
     KPlane k;                    /* invB: 1 / (N eps) for SYN_EPS               */
-    const fame::ProbDev* prob;
+    const double2* outer;        /* exp(2 i pi r0 c / nc), nc per problem       */
     const double2* in;           /* analysis: field in the reference's layout (General), or null: in place */
     double2* out;                /* SYN_REF: field in the reference's layout    */
     const double2* E;            /* SYN_RES: the fields, reference's layout (General) */
@@ -232,8 +233,8 @@ hipError_t fame_launch_line32(const KLine& k, int expand, int mode, int nprob, h
 hipError_t fame_launch_line64(const KLine& k, int expand, int mode, int nprob, hipStream_t s);
 hipError_t fame_launch_plane32(const KPlane& k, int nprob, hipStream_t s);
 hipError_t fame_launch_plane64(const KPlane& k, int nprob, hipStream_t s);
-hipError_t fame_prepare_plane32(int eb, int ec, size_t lds);
-hipError_t fame_prepare_plane64(int eb, int ec, size_t lds);
+hipError_t fame_prepare_plane32(int eb, int ec);
+hipError_t fame_prepare_plane64(int eb, int ec);
 hipError_t fame_prepare_syn(int eb, int ec);
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s);
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s);
@@ -251,7 +252,7 @@ hipError_t fame_launch_resid_simple(const double2* F, const double2* E, const do
 hipError_t fame_launch_eps(const fame::GridDev& g, const double* eps, double* eps_int, double* ib64, float* ib32, double* p64,
                            float* p32, int PP, hipStream_t s);
 hipError_t fame_launch_line_tab(const fame::GridDev& g, const fame::ProbDev* prob, LineTab* lt, void* tw64, void* tw32,
-                                void* mid64, void* mid32, int nprob, hipStream_t s);
+                                void* mid64, void* mid32, double2* outer, int nprob, hipStream_t s);
 hipError_t fame_launch_xz_transpose(const void* in, void* out, int nx, int ny, int nz, int dir, size_t stride,
                                     int ncomp, int nprob, int prec, hipStream_t s);
 hipError_t fame_launch_pack(const void* in, void* out, int N, int Nd, int dir, int prec, hipStream_t s);

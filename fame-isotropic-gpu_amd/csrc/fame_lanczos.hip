@@ -346,7 +346,7 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
                 same = same && k->tile[a][pi].eng == c->tile[a][pi].eng && k->tile[a][pi].L == c->tile[a][pi].L;
         for (int pi = 0; pi < 2; ++pi)
             same = same && k->plane[pi] == c->plane[pi] && k->ltile[pi].eng == c->ltile[pi].eng && k->ltile[pi].L == c->ltile[pi].L &&
-                   k->ctile[pi].L == c->ctile[pi].L && k->kpl[pi].nt == c->kpl[pi].nt;
+                   k->ctile[pi].L == c->ctile[pi].L && k->kpl[pi].nt == c->kpl[pi].nt && k->kpl[pi].wide == c->kpl[pi].wide;
         if (!same) {
             for (int pi = 0; pi < 2; ++pi) {
                 for (int a = 0; a < 3; ++a) k->tile[a][pi] = c->tile[a][pi];
@@ -355,6 +355,7 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
                 k->ltile[pi] = c->ltile[pi];
                 k->ctile[pi] = c->ctile[pi];
                 k->kpl[pi].nt = c->kpl[pi].nt;
+                k->kpl[pi].wide = c->kpl[pi].wide;
             }
             k->drop_graphs();
         }
@@ -640,7 +641,7 @@ static fame_status restore_band(fame_ctx* c, int i, int nwant, const double2* ev
                                 bool ref = false) {
     const size_t N = c->N, n2 = 2 * N, N3 = 3 * N;
     const int nk = c->nk;
-    if (c->syn_ok) {
+    if (c->plane_ok[0]) {
         /* four kernels and no host round trip: the expansion scales by Sigma as it
          * reads, the plane kernel applies 1/eps and sums |E|^2, the transpose to the
          * reference's layout applies the norm.  Against the separate passes
@@ -710,7 +711,7 @@ extern "C" fame_status fame_restore(fame_ctx* c, int nwant, const void* evr_dev,
     const size_t n2 = 2 * (size_t)c->N;
     double2* stage = (double2*)c->ref64[2];
     for (int i = 0; i < nwant; ++i) {
-        if (c->syn_ok) {
+        if (c->plane_ok[0]) {
             CHK(restore_band(c, i, nwant, (const double2*)evr_dev + (size_t)i * n2, (size_t)nwant * n2, E_dev, true));
             continue;
         }

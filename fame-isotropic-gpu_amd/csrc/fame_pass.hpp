@@ -256,8 +256,8 @@ __device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, const 
     return acc;
 }
 
-/* run CASE(R) for radix r: the compound radices exist in FP32 only */
-#define RADIX_SWITCH(r, CASE)                                                                                        \
+/* run CASE(R) for radix r: the compound radices where a thread holds 16 elements */
+#define RADIX_SWITCH(r, MAXE, CASE)                                                                                  \
     switch (r) {                                                                                                     \
         case 2: CASE(2); break;                                                                                      \
         case 3: CASE(3); break;                                                                                      \
@@ -268,7 +268,7 @@ __device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, const 
         case 11: CASE(11); break;                                                                                    \
         case 13: CASE(13); break;                                                                                    \
         default:                                                                                                     \
-            if constexpr (MaxE<T>::v >= 16) {                                                                        \
+            if constexpr (MAXE >= 16) {                                                                              \
                 switch (r) {                                                                                         \
                     case 6: CASE(6); break;                                                                          \
                     case 9: CASE(9); break;                                                                          \
@@ -283,16 +283,16 @@ __device__ __forceinline__ double mid_pass(T2* S, int nl, int LS, int ES, const 
     }
 
 /* passes s0 .. s1 - 1 of one transform (no barrier after the last one) */
-template <typename T, typename T2, bool INV, int HK>
+template <typename T, typename T2, bool INV, int HK, int MAXE>
 __device__ __forceinline__ void line_passes(T2* S, int nl, int LS, int ES, CStage* st, int s0, int s1, int nst,
                                             const T2* W, const Hook<T, T2>& hk) {
     if (s0 >= s1) return;
     PlaneStage cur = load_stage(st + s0);
-#define LP(R) line_pass<T, T2, R, MaxE<T>::v, INV, HK>(S, nl, LS, ES, cur, W, hk, s == 0, s + 1 == nst)
+#define LP(R) line_pass<T, T2, R, MAXE, INV, HK>(S, nl, LS, ES, cur, W, hk, s == 0, s + 1 == nst)
     for (int s = s0; s < s1; ++s) {
         /* the next pass's descriptor is on its way while this pass runs */
         const PlaneStage next = load_stage(st + (s + 1 < s1 ? s + 1 : s));
-        RADIX_SWITCH(cur.R, LP)
+        RADIX_SWITCH(cur.R, MAXE, LP)
         cur = next;
     }
 #undef LP
@@ -419,12 +419,12 @@ __device__ __forceinline__ void line_mfma(T2* S, int nl, int LS, int ES, int n, 
 }
 
 /* one transform without hooks; begins with a barrier, ends without one */
-template <typename T, typename T2, int ENG, bool INV>
+template <typename T, typename T2, int ENG, bool INV, int MAXE = MaxE<T>::v>
 __device__ __forceinline__ void line_transform(T2* S, int nl, int LS, int ES, const PlaneAxis& ax, const T2* W) {
     if constexpr (ENG == ENG_STOCKHAM) {
         Hook<T, T2> hk;
         hk.tw = nullptr; hk.eps = nullptr; hk.ld = 0; hk.pap = false;
-        line_passes<T, T2, INV, 0>(S, nl, LS, ES, cstage(INV ? ax.st : ax.sf), 0, ax.nst, ax.nst, W, hk);
+        line_passes<T, T2, INV, 0, MAXE>(S, nl, LS, ES, cstage(INV ? ax.st : ax.sf), 0, ax.nst, ax.nst, W, hk);
     } else {
         line_mfma<T, T2, INV>(S, nl, LS, ES, ax.n, W);
     }
@@ -433,18 +433,18 @@ __device__ __forceinline__ void line_transform(T2* S, int nl, int LS, int ES, co
 /* the c axis of a plane (nl columns, element stride ES): middle twiddle, inverse
  * transform, 1/eps, forward transform, conjugate twiddle; returns the <v, eps^-1 v>
  * share.  Begins with a barrier, ends without one.                           */
-template <typename T, typename T2, int ENG>
+template <typename T, typename T2, int ENG, int MAXE = MaxE<T>::v>
 __device__ __forceinline__ double column_round_trip(T2* S, int nl, int ES, const PlaneAxis& ax, const T2* W,
                                                     const Hook<T, T2>& hk) {
     double acc = 0.0;
     if constexpr (ENG == ENG_STOCKHAM) {
         const int n = ax.nst;
         const PlaneStage ms = load_stage(cstage(ax.st) + n - 1);
-        line_passes<T, T2, true, HK_TIN>(S, nl, 1, ES, cstage(ax.st), 0, n - 1, n, W, hk);
-#define MP(R) acc = mid_pass<T, T2, R, MaxE<T>::v>(S, nl, 1, ES, ms, W, hk, n == 1)
-        RADIX_SWITCH(ms.R, MP)
+        line_passes<T, T2, true, HK_TIN, MAXE>(S, nl, 1, ES, cstage(ax.st), 0, n - 1, n, W, hk);
+#define MP(R) acc = mid_pass<T, T2, R, MAXE>(S, nl, 1, ES, ms, W, hk, n == 1)
+        RADIX_SWITCH(ms.R, MAXE, MP)
 #undef MP
-        line_passes<T, T2, false, HK_TOUT>(S, nl, 1, ES, cstage(ax.sf), 1, n, n, W, hk);
+        line_passes<T, T2, false, HK_TOUT, MAXE>(S, nl, 1, ES, cstage(ax.sf), 1, n, n, W, hk);
     } else {
         /* the elementwise steps as passes of their own, columns fastest */
         const int tot = nl * ax.n;
@@ -470,11 +470,11 @@ __device__ __forceinline__ double column_round_trip(T2* S, int nl, int ES, const
 
 /* one transform along c with the middle twiddle: inverse with it going in, or
  * forward with its conjugate coming out.  Begins with a barrier, ends without. */
-template <typename T, typename T2, int ENG, bool INV>
+template <typename T, typename T2, int ENG, bool INV, int MAXE = MaxE<T>::v>
 __device__ __forceinline__ void column_transform(T2* S, int nl, int ES, const PlaneAxis& ax, const T2* W,
                                                  const Hook<T, T2>& hk) {
     if constexpr (ENG == ENG_STOCKHAM) {
-        line_passes<T, T2, INV, INV ? HK_TIN : HK_TOUT>(S, nl, 1, ES, cstage(INV ? ax.st : ax.sf), 0, ax.nst, ax.nst, W, hk);
+        line_passes<T, T2, INV, INV ? HK_TIN : HK_TOUT, MAXE>(S, nl, 1, ES, cstage(INV ? ax.st : ax.sf), 0, ax.nst, ax.nst, W, hk);
     } else {
         const int tot = nl * ax.n;
         if (!INV) line_mfma<T, T2, INV>(S, nl, 1, ES, ax.n, W);

@@ -680,6 +680,9 @@ __device__ __forceinline__ void rows_out(const T2* S, T2* G, int nb, int Pb, uns
 template <typename T, int ENGB, int ENGC, int TB>
 __global__ void __launch_bounds__(TB) k_plane(KPlane k) {
     typedef typename C2<T>::T2 T2;
+    /* FP64: 16 elements per thread, and with them the compound radices, where a
+     * block of 512 threads leaves 256 registers                              */
+    constexpr int MAXE = sizeof(T) == 8 && TB == 512 ? 16 : MaxE<T>::v;
     /* blocks of one XCD (x mod 8) take a run of consecutive planes, problem by
      * problem: the problem's middle twiddles stay in that XCD's L2            */
     touch_args<sizeof(KPlane)>();
@@ -704,9 +707,9 @@ __global__ void __launch_bounds__(TB) k_plane(KPlane k) {
     hk.ld = nb;
     hk.pap = k.pap != nullptr;
     rows_in<T, T2, 4>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
-    line_transform<T, T2, ENGB, true>(S, nc, Pb, 1, k.b, Wb);
-    double vw = column_round_trip<T, T2, ENGC>(S, nb, Pb, k.c, Wc, hk);
-    line_transform<T, T2, ENGB, false>(S, nc, Pb, 1, k.b, Wb);
+    line_transform<T, T2, ENGB, true, MAXE>(S, nc, Pb, 1, k.b, Wb);
+    double vw = column_round_trip<T, T2, ENGC, MAXE>(S, nb, Pb, k.c, Wc, hk);
+    line_transform<T, T2, ENGB, false, MAXE>(S, nc, Pb, 1, k.b, Wb);
     __syncthreads();
     rows_out<T, T2>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
     if (hk.pap) {
@@ -761,8 +764,8 @@ static const void* plane_fn(int eb, int ec) {
     return ec == ENG_MFMA ? (const void*)k_plane<T, ENG_STOCKHAM, ENG_MFMA, TB> : (const void*)k_plane<T, ENG_STOCKHAM, ENG_STOCKHAM, TB>;
 }
 template <typename T>
-static const void* plane_fn(int eb, int ec, int nt, size_t lds) {
-    if constexpr (sizeof(T) == 8) if (nt <= 512 && lds > FAME_LDS_HALF) return plane_fn<T, 512>(eb, ec);
+static const void* plane_fn(int eb, int ec, int wide) {
+    if constexpr (sizeof(T) == 8) if (wide) return plane_fn<T, 512>(eb, ec);
     return plane_fn<T, 1024>(eb, ec);
 }
 template <typename T>
@@ -771,12 +774,12 @@ static hipError_t launch_plane(const KPlane& k, int nprob, hipStream_t s) {
     q.nprob = nprob;
     void* arg[] = {&q};
     const size_t lds = fame_plane_lds(k.b.n, k.c.n, k.b.ntab + k.c.ntab, (int)sizeof(T));
-    return hipLaunchKernel(plane_fn<T>(k.b.eng, k.c.eng, k.nt, lds), dim3(xcd_round(3 * k.g.na * nprob)), dim3(k.nt), arg, lds, s);
+    return hipLaunchKernel(plane_fn<T>(k.b.eng, k.c.eng, k.wide), dim3(xcd_round(3 * k.g.na * nprob)), dim3(k.nt), arg, lds, s);
 }
 template <typename T>
-static hipError_t prepare_plane(int eb, int ec, size_t lds) {
-    for (int nt = 512; nt <= 1024; nt *= 2) {
-        const hipError_t e = hipFuncSetAttribute(plane_fn<T>(eb, ec, nt, lds), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
+static hipError_t prepare_plane(int eb, int ec) {
+    for (int wide = 0; wide < 2; ++wide) {
+        const hipError_t e = hipFuncSetAttribute(plane_fn<T>(eb, ec, wide), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

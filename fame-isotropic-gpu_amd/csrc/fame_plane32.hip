@@ -5,4 +5,4 @@ using namespace fame;
 
 hipError_t fame_launch_line32(const KLine& k, int expand, int mode, int nprob, hipStream_t s) { return launch_line<float>(k, expand, mode, nprob, s); }
 hipError_t fame_launch_plane32(const KPlane& k, int nprob, hipStream_t s) { return launch_plane<float>(k, nprob, s); }
-hipError_t fame_prepare_plane32(int eb, int ec, size_t lds) { return prepare_plane<float>(eb, ec, lds); }
+hipError_t fame_prepare_plane32(int eb, int ec) { return prepare_plane<float>(eb, ec); }

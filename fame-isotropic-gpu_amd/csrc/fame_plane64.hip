@@ -6,13 +6,13 @@ using namespace fame;
 
 hipError_t fame_launch_line64(const KLine& k, int expand, int mode, int nprob, hipStream_t s) { return launch_line<double>(k, expand, mode, nprob, s); }
 hipError_t fame_launch_plane64(const KPlane& k, int nprob, hipStream_t s) { return launch_plane<double>(k, nprob, s); }
-hipError_t fame_prepare_plane64(int eb, int ec, size_t lds) { return prepare_plane<double>(eb, ec, lds); }
+hipError_t fame_prepare_plane64(int eb, int ec) { return prepare_plane<double>(eb, ec); }
 
 /* per line (b, c) of every problem: its symbols and inner-axis phase, the inner
  * twiddle factors in both precisions, and the middle twiddles of its nb entries'
  * plane (entry gl itself: exp(2 pi i (s0 + s1 c) b / nb))                    */
 __global__ void k_line_tab(GridDev g, const ProbDev* prob, LineTab* lt, double2* tw64, float2* tw32, double2* mid64,
-                           float2* mid32) {
+                           float2* mid32, double2* outer) {
     const int p = blockIdx.y, nlines = g.nb * g.nc, tpl = inner_tw_per_line(g.na);
     const ProbDev pr = prob[p];
     for (int gl = blockIdx.x * blockDim.x + threadIdx.x; gl < nlines; gl += gridDim.x * blockDim.x) {
@@ -35,12 +35,13 @@ __global__ void k_line_tab(GridDev g, const ProbDev* prob, LineTab* lt, double2*
         const double2 w = expipi(2.0 * (pr.s0 + pr.s1 * (double)c) / (double)g.nb * (double)b);
         mid64[o] = w;
         mid32[o] = make_float2((float)w.x, (float)w.y);
+        if (b == 0) outer[(size_t)p * g.nc + c] = expipi(2.0 * pr.r0 * (double)c / (double)g.nc);
     }
 }
 hipError_t fame_launch_line_tab(const GridDev& g, const ProbDev* prob, LineTab* lt, void* tw64, void* tw32, void* mid64,
-                                void* mid32, int nprob, hipStream_t s) {
+                                void* mid32, double2* outer, int nprob, hipStream_t s) {
     hipLaunchKernelGGL(k_line_tab, dim3((g.nb * g.nc + 63) / 64, nprob), dim3(64), 0, s, g, prob, lt, (double2*)tw64, (float2*)tw32,
-                       (double2*)mid64, (float2*)mid32);
+                       (double2*)mid64, (float2*)mid32, outer);
     return hipGetLastError();
 }
 
@@ -50,19 +51,15 @@ hipError_t fame_launch_line_tab(const GridDev& g, const ProbDev* prob, LineTab* 
  * of fixed a) straight in the reference's layout, transposed on the way through
  * LDS.  They replace k_mid + k_outer + k_xz_transpose (18 N s of field traffic) and
  * the conversions of the reduced vector (8 N s) by one pass (6 N s): Qrs of
- * a 50 x 43 x 35 grid 59 -> 34 us, residuals of 4 wave vectors x 12 bands on the
+ * a 50 x 42 x 36 grid 59 -> 34 us, residuals of 4 wave vectors x 12 bands on the
  * FCC 64 grid 3.27 -> 1.56 ms.  Bound by the LDS passes and, where a plane is over
- * half a CU's LDS, by one block per CU: Qr at FCC 96 stays at 97 us.          */
+ * half a CU's LDS, by one block per CU.  The outer phases come from a table in
+ * global memory, so that every grid whose k_plane fits the LDS fits here too  */
 namespace fame {
 
 __device__ __forceinline__ void plane_tables(const KPlane& k, double2* Wb, double2* Wc) {
     for (int i = threadIdx.x; i < k.b.ntab; i += blockDim.x) Wb[i] = reinterpret_cast<const double2*>(k.b.W)[i];
     for (int i = threadIdx.x; i < k.c.ntab; i += blockDim.x) Wc[i] = reinterpret_cast<const double2*>(k.c.W)[i];
-}
-
-/* D_c = exp(2 i pi r0 c / nc), nc entries */
-__device__ __forceinline__ void outer_phases(double2* D, const ProbDev& pr, int nc) {
-    for (int c = threadIdx.x; c < nc; c += blockDim.x) D[c] = expipi(2.0 * pr.r0 * (double)c / (double)nc);
 }
 
 __device__ __forceinline__ double block_sum(double v, double* red) {
@@ -94,17 +91,16 @@ __global__ void __launch_bounds__(512) k_syn(KSyn a) {
     T2* S = reinterpret_cast<T2*>(smem_raw);
     T2* Wb = S + ((nc * Pb + 1) & ~1);
     T2* Wc = Wb + k.b.ntab;
-    T2* D = Wc + k.c.ntab;
+    const T2* D = a.outer + (size_t)p * nc;      /* exp(2 i pi r0 c / nc) */
     plane_tables(k, Wb, Wc);
-    outer_phases(D, a.prob[p], nc);
     const size_t po = (size_t)pl * k.PP;
     T2* F = reinterpret_cast<T2*>(k.f) + (size_t)p * k.fstride + po;
     Hook<double, T2> hk;
     hk.tw = reinterpret_cast<const T2*>(k.tw) + (size_t)p * plane;
     hk.eps = nullptr; hk.ld = nb; hk.pap = false;
     rows_in<double, T2, 4>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
-    line_transform<double, T2, ENGB, true>(S, nc, Pb, 1, k.b, Wb);
-    column_transform<double, T2, ENGC, true>(S, nb, Pb, k.c, Wc, hk);
+    line_transform<double, T2, ENGB, true, 16>(S, nc, Pb, 1, k.b, Wb);
+    column_transform<double, T2, ENGC, true, 16>(S, nb, Pb, k.c, Wc, hk);
     __syncthreads();
     const double invN = 1.0 / (double)k.g.N;
     if constexpr (MODE == SYN_FIELD || MODE == SYN_EPS) {
@@ -172,10 +168,8 @@ __global__ void __launch_bounds__(512) k_ana(KSyn a) {
     T2* S = reinterpret_cast<T2*>(smem_raw);
     T2* Wb = S + ((nc * Pb + 1) & ~1);
     T2* Wc = Wb + k.b.ntab;
-    T2* D = Wc + k.c.ntab;
+    const T2* D = a.outer + (size_t)p * nc;
     plane_tables(k, Wb, Wc);
-    outer_phases(D, a.prob[p], nc);
-    __syncthreads();
     T2* F = reinterpret_cast<T2*>(k.f) + (size_t)p * k.fstride + (size_t)pl * k.PP;
     if (a.in) {
         const int comp = pl / k.g.na, ai = pl - comp * k.g.na;
@@ -195,8 +189,8 @@ __global__ void __launch_bounds__(512) k_ana(KSyn a) {
     Hook<double, T2> hk;
     hk.tw = reinterpret_cast<const T2*>(k.tw) + (size_t)p * plane;
     hk.eps = nullptr; hk.ld = nb; hk.pap = false;
-    column_transform<double, T2, ENGC, false>(S, nb, Pb, k.c, Wc, hk);
-    line_transform<double, T2, ENGB, false>(S, nc, Pb, 1, k.b, Wb);
+    column_transform<double, T2, ENGC, false, 16>(S, nb, Pb, k.c, Wc, hk);
+    line_transform<double, T2, ENGB, false, 16>(S, nc, Pb, 1, k.b, Wb);
     __syncthreads();
     rows_out<double, T2>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
 }
@@ -412,7 +406,7 @@ static hipError_t launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) 
     void* arg[] = {&q};
     const int nt = k.k.nt > 512 ? 512 : k.k.nt;
     return hipLaunchKernel(syn_fn(k.k.b.eng, k.k.c.eng, mode), dim3(xcd_round(3 * k.k.g.na * nprob)), dim3(nt), arg,
-                           fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab + k.k.c.n, 8), s);
+                           fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab, 8), s);
 }
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) { return launch_syn(k, mode, nprob, s); }
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s) { return launch_syn(k, 4, nprob, s); }

@@ -347,7 +347,7 @@ bool fame_ctx::line_tile_ok(int prec, int eng, int L) const {
 }
 
 /* an axis of the plane path: its Stockham passes, or the direct DFT */
-static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q) {
+static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q, bool wide = false) {
     std::memset(q, 0, sizeof(*q));
     if (p.n < 2 || (eng == ENG_STOCKHAM ? p.blue != 0 : p.n < 8)) return false;
     const LinePlanDev& d = p.lists[pi][LIST_FWD];
@@ -357,7 +357,9 @@ static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q)
     q->ntab = eng == ENG_MFMA ? nqt * ((m + 3) / 4) * 64 : p.n;
     q->mnl = fame_magic32(nl);
     q->mn = fame_magic32(p.n);
-    if (eng == ENG_STOCKHAM) { q->nst = d.nst; q->st = p.pst[pi]; q->sf = p.pst[pi] + d.nst; }
+    /* the wide variant's passes: FP32's radices, the same table of roots */
+    const int pl = wide ? 1 : pi;
+    if (eng == ENG_STOCKHAM) { q->nst = p.lists[pl][LIST_FWD].nst; q->st = p.pst[pl]; q->sf = p.pst[pl] + q->nst; }
     q->n = p.n;
     return true;
 }
@@ -373,22 +375,34 @@ fame_status fame_ctx::plane_setup() {
         const int prec = pi == 0 ? 8 : 4;
         KPlane& k = kpl[pi];
         std::memset(&k, 0, sizeof(k));
-        /* up to 24 points the direct DFT on the matrix cores: one step between
+        /* 8 to 24 points: the direct DFT on the matrix cores: one step between
          * barriers instead of two or three passes.  The plane kernel of a 16^3 grid,
          * one wave vector, 11.3 -> 8.7 us in FP64 (10.7 -> 8.1 in FP32), 24^3 12.2
          * -> 10.6 (12.5 -> 9.4), eight 24^3 16.9 -> 15.4; from 32^3 on the passes
          * win (eight in FP64 20.8 against 29.1)                               */
         auto engine = [&](int axis) {
-            return (ax[axis][0].blue || eng_forced == 1 || (eng_forced < 0 && ax[axis][1].n > 0 && ax[axis][1].n <= 24)) ? ENG_MFMA : ENG_STOCKHAM;
+            return (ax[axis][0].blue || eng_forced == 1 || (eng_forced < 0 && ax[axis][1].n >= 8 && ax[axis][1].n <= 24)) ? ENG_MFMA : ENG_STOCKHAM;
         };
         if (!plane_axis(ax[AX_MID][engine(AX_MID)], engine(AX_MID), pi, g.nc, &k.b)) continue;
         if (!plane_axis(ax[AX_OUTER][engine(AX_OUTER)], engine(AX_OUTER), pi, g.nb, &k.c)) continue;
+        if (prec == 8) {
+            plane_axis(ax[AX_MID][k.b.eng], k.b.eng, pi, g.nc, &wide_ax[0], true);
+            plane_axis(ax[AX_OUTER][k.c.eng], k.c.eng, pi, g.nb, &wide_ax[1], true);
+        }
         const size_t lds = fame_plane_lds(g.nb, g.nc, k.b.ntab + k.c.ntab, prec);
         if (lds > 160 * 1024 - 256) continue;
         k.g = g;
         k.PP = PP;
         k.mnb = fame_magic32(g.nb);
+        /* FP64, wide variant (2 waves per SIMD, 16 elements per thread): where a
+         * plane fills the CU alone anyway, or the compound radices save a pass
+         * (48^3: 21.6 -> 18.5 us, eight 72.2 -> 63.9; FCC 96: 54 -> 50, four 227
+         * -> 188).  At equal passes the narrow one's 4 waves per SIMD are better
+         * (16 x 64^3: 170 against 193).  Many blocks: two of 256 threads per CU
+         * instead of one of 512                                               */
+        k.wide = prec == 8 && (lds > FAME_LDS_HALF || wide_ax[0].nst + wide_ax[1].nst < k.b.nst + k.c.nst);
         k.nt = lds > FAME_LDS_HALF ? (prec == 8 ? 512 : 1024) : lds > 24 * 1024 ? 512 : 256;
+        if (k.wide && lds <= FAME_LDS_HALF) k.nt = 3 * g.na * maxb > 512 ? 256 : 512;
         bool any = false;
         for (int e = 0; e < 2; ++e) {
             if (eng_forced >= 0 && e != eng_forced && !(eng_forced == 0 && ax[AX_INNER][0].blue)) { laxis[pi][e].n = 0; continue; }
@@ -403,11 +417,8 @@ fame_status fame_ctx::plane_setup() {
         if (!line_tile_ok(prec, eng, L)) { plane_ok[pi] = false; continue; }
         ltile[pi].eng = eng; ltile[pi].L = L; ltile[pi].P = g.na | 1;
         ctile[pi] = ltile[pi];
-        if (prec == 8) {
-            syn_ok = lds + 16 * (size_t)g.nc <= 160 * 1024 - 256;
-            if (syn_ok) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
-        }
-        HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng, lds) : fame_prepare_plane32(k.b.eng, k.c.eng, lds));
+        if (prec == 8) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+        HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng) : fame_prepare_plane32(k.b.eng, k.c.eng));
         /* before tuning: an FP64 plane that fills a CU alone pays where one
          * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
          * iteration in 112 us against 134 by axis passes; SC 96, 288 blocks: 193
@@ -425,7 +436,9 @@ hipError_t fame_ctx::launch_plane(const KPlane& k, int prec, int nprob) {
 }
 
 /* threads per block of the plane kernel (within its launch bounds) */
-static bool plane_threads_ok(int prec, int nt) { return nt == 256 || nt == 512 || nt == 1024; }
+static bool plane_threads_ok(int prec, int nt, int wide) {
+    return (nt == 256 || nt == 512 || (nt == 1024 && !wide)) && (prec == 8 || !wide);
+}
 
 KLine fame_ctx::kline(int prec, int p0, const int* act, bool contract) const {
     const int pi = prec == 8 ? 0 : 1;
@@ -450,6 +463,7 @@ KPlane fame_ctx::kplane(int prec, int p0, const int* act) const {
     const int pi = prec == 8 ? 0 : 1;
     const size_t es = prec == 8 ? 16 : 8;
     KPlane k = kpl[pi];
+    if (k.wide) { k.b = wide_ax[0]; k.c = wide_ax[1]; }
     k.active = act;
     k.fstride = 3 * (size_t)CS;
     k.f = prec == 8 ? (char*)F64 + 16 * k.fstride * p0 : (char*)F32 + 8 * k.fstride * p0;
@@ -461,7 +475,8 @@ KSyn fame_ctx::ksyn(int p0) const {
     KSyn a;
     std::memset(&a, 0, sizeof(a));
     a.k = kplane(8, p0, nullptr);
-    a.prob = prob_d + p0;
+    a.k.b = wide_ax[0]; a.k.c = wide_ax[1];
+    a.outer = otw + (size_t)g.nc * p0;
     a.ostride = 3 * (size_t)N;
     return a;
 }
@@ -567,7 +582,8 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
             {(void**)&c->ltab, sizeof(LineTab) * nl * B}, {(void**)&c->eatab, 16 * (size_t)g.na}, {(void**)&c->cgsc2, sizeof(CgScal) * B},
             {(void**)&c->invBp[0], 8 * 3 * (size_t)c->CS}, {(void**)&c->invBp[1], 4 * 3 * (size_t)c->CS},
             {(void**)&c->ltw[0], 16 * nl * tpl * B}, {(void**)&c->ltw[1], 8 * nl * tpl * B},
-            {(void**)&c->mtw[0], 16 * nl * B}, {(void**)&c->mtw[1], 8 * nl * B}};
+            {(void**)&c->mtw[0], 16 * nl * B}, {(void**)&c->mtw[1], 8 * nl * B},
+            {(void**)&c->otw, 16 * (size_t)g.nc * B}};
         size_t total = 0;
         for (const auto& q : part) total += (q.n + 255) & ~(size_t)255;
         char* base = nullptr;
@@ -700,7 +716,7 @@ extern "C" fame_status fame_set_wave_vectors(fame_ctx* c, int nk, const double* 
     HIPCHK(hipMemcpyAsync(c->prob_d, c->prob_h.data(), sizeof(ProbDev) * nk, hipMemcpyHostToDevice, c->stream));
     HIPCHK(fame_launch_sigma(c->g, c->prob_d, c->sig, c->sig_inv, nk, c->stream));
     if (c->ltab)
-        HIPCHK(fame_launch_line_tab(c->g, c->prob_d, c->ltab, c->ltw[0], c->ltw[1], c->mtw[0], c->mtw[1], nk, c->stream));
+        HIPCHK(fame_launch_line_tab(c->g, c->prob_d, c->ltab, c->ltw[0], c->ltw[1], c->mtw[0], c->mtw[1], c->otw, nk, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     ++c->k_ver;
     return FAME_OK;
@@ -863,7 +879,7 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
     const size_t pn = (size_t)c->g.nb * c->g.nc;
     switch (op) {
         case FAME_OP_QR:
-            if (c->syn_ok) {
+            if (c->plane_ok[0]) {
                 /* vector and field straight in the reference's layouts; a Simple
                  * grid's field needs the transpose                           */
                 KLine k = c->kline(8, ik, nullptr);
@@ -884,7 +900,7 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             CHK(c->field_to_ref(c->F64 + (size_t)ik * 3 * N, y, 1, 3 * (size_t)N));
             break;
         case FAME_OP_QRS:
-            if (c->syn_ok) {
+            if (c->plane_ok[0]) {
                 KLine k = c->kline(8, ik, nullptr, true);
                 KSyn s = c->ksyn(ik);
                 if (c->g.general) s.in = (const double2*)x;
@@ -1013,23 +1029,26 @@ fame_status fame_ctx::tune(int prec) {
             t = best;
             plane_ms += best_ms;
         }
-        int best_nt = kpl[pi].nt;
+        int best_nt = kpl[pi].nt, best_wide = kpl[pi].wide;
         float best_ms = 1e30f;
-        for (int nt = 256; nt <= 1024 && st == FAME_OK; nt *= 2) {
-            if (!plane_threads_ok(prec, nt)) continue;
-            KPlane k = kplane(prec, 0, nullptr);
-            k.nt = nt;
-            k.pap = pap_part;
-            float ms = 0;
-            if (!timed([&] { return launch_plane(k, prec, nk); }, &ms)) { st = FAME_ERR_HIP; break; }
-            if (ms < best_ms) { best_ms = ms; best_nt = nt; }
-        }
+        for (int wide = 0; wide < (prec == 8 ? 2 : 1) && st == FAME_OK; ++wide)
+            for (int nt = 256; nt <= 1024 && st == FAME_OK; nt *= 2) {
+                if (!plane_threads_ok(prec, nt, wide)) continue;
+                kpl[pi].wide = wide;
+                KPlane k = kplane(prec, 0, nullptr);
+                k.nt = nt;
+                k.pap = pap_part;
+                float ms = 0;
+                if (!timed([&] { return launch_plane(k, prec, nk); }, &ms)) { st = FAME_ERR_HIP; break; }
+                if (ms < best_ms) { best_ms = ms; best_nt = nt; best_wide = wide; }
+            }
         kpl[pi].nt = best_nt;
+        kpl[pi].wide = best_wide;
         plane_ms += best_ms;
     }
     /* a plane that leaves room for two blocks per CU beats the axis passes by 8% to
      * 30% at every batch measured; one that fills the CU alone may not, so both
-     * are timed                                                               */
+     * are tuned and compared                                                  */
     const size_t plds = plane_ok[pi] ? fame_plane_lds(g.nb, g.nc, kpl[pi].b.ntab + kpl[pi].c.ntab, prec) : 0;
     const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF;
     plane[pi] = plane_ok[pi];
@@ -1075,6 +1094,31 @@ fame_status fame_ctx::tune(int prec) {
         tile[a][pi] = best;
         axis_ms += best_ms;
     }
+    if (axis_too && plane_ok[pi] && st == FAME_OK) {
+        /* whole iterations against each other: the axis passes' inner kernels in
+         * their CG forms too (tuned alone they look cheaper than they are: four
+         * BCC 128 problems ran 532 us of axis passes for 455 of planes)        */
+        void** V = prec == 8 ? cg64 : cg32;
+        void* xs = prec == 8 ? ref64[1] : cg32[4];
+        const size_t n2 = 2 * (size_t)N;
+        for (int w = 0; w < 2 && st == FAME_OK; ++w) {
+            plane[pi] = w == 1;
+            nblk_in[pi] = (g.nb * g.nc + tile[AX_INNER][pi].L - 1) / tile[AX_INNER][pi].L;
+            const int npap = pap_blocks(prec);
+            float ms = 0;
+            /* every byte of b 0x3c: nonzero and finite */
+            if (hipMemsetAsync(V[3], 0x3c, es * n2 * nk, stream) != hipSuccess ||
+                fame_cg_begin(xs, V[0], V[1], V[3], partials, NBLK_VEC, n2, n2, nk, prec, nullptr, stream) != hipSuccess ||
+                fame_cg_init_scal2(cgsc, partials, NBLK_VEC, 0.0, 0.0, 1 << 30, nk, active, nullptr, stream) != hipSuccess ||
+                !timed([&] {
+                    return (npap ? cg_step_rc(prec, V[1], V[0], xs, 0, nk, npap) : cg_step_ap(prec, V[1], V[0], xs, V[2], 0, nk)) == FAME_OK
+                               ? hipSuccess : hipErrorUnknown;
+                }, &ms))
+                st = FAME_ERR_HIP;
+            (w ? plane_ms : axis_ms) = ms;
+        }
+        plane[pi] = true;
+    }
     if (axis_too && axis_ms < plane_ms) plane[pi] = false;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -1090,15 +1134,17 @@ extern "C" fame_status fame_set_tiles(fame_ctx* c, int prec, const int* choice) 
     const int pi = prec == 8 ? 0 : 1;
     /* engine 2 for the middle and outer passes: the plane path, whose middle
      * entry holds the contracting kernel's lines and outer entry the plane
-     * kernel's threads                                                        */
-    if (choice[2] == 2 && choice[4] == 2) {
+     * kernel's threads (outer engine 3: its wide variant)                     */
+    if (choice[2] == 2 && (choice[4] == 2 || choice[4] == 3)) {
+        const int wide = choice[4] == 3;
         if (!c->line_tile_ok(prec, choice[0], choice[1]) || !c->line_tile_ok(prec, choice[0], choice[3]) ||
-            !plane_threads_ok(prec, choice[5]))
+            !plane_threads_ok(prec, choice[5], wide))
             FAIL(FAME_ERR_ARG, "fame_set_tiles: engine, lines per block or threads not available for the plane path");
         c->plane[pi] = true;
         c->ltile[pi].eng = c->ctile[pi].eng = choice[0];
         c->ltile[pi].L = choice[1]; c->ctile[pi].L = choice[3];
         c->kpl[pi].nt = choice[5];
+        c->kpl[pi].wide = wide;
         c->tuned[pi] = true;
         c->drop_graphs();
         return FAME_OK;
@@ -1129,7 +1175,7 @@ extern "C" fame_status fame_autotune(fame_ctx* c, int prec, int* choice) {
         if (c->plane[pi]) {
             choice[0] = c->ltile[pi].eng; choice[1] = c->ltile[pi].L;
             choice[2] = 2; choice[3] = c->ctile[pi].L;
-            choice[4] = 2; choice[5] = c->kpl[pi].nt;
+            choice[4] = c->kpl[pi].wide ? 3 : 2; choice[5] = c->kpl[pi].nt;
         }
     }
     return FAME_OK;

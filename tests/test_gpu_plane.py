@@ -70,6 +70,11 @@ def test_plane_qbq_vs_oracle(gpu, lt, nx, k):
                 seen += 1
                 y = S.apply(op, 0, xd).cpu().numpy()
                 assert _rel(y, ref) < bar, (prec, t, _rel(y, ref))
+                t["outer"] = (3, nt)        # FP64: 16 elements per thread, compound radices
+                assert _accepted(S, prec, t) == (prec == 8 and nt <= 512)
+                if prec == 8 and nt <= 512:
+                    y = S.apply(op, 0, xd).cpu().numpy()
+                    assert _rel(y, ref) < bar, (prec, t, _rel(y, ref))
         # the axis passes on the same grid
         if _accepted(S, prec, {"inner": (0, 4), "mid": (0, 8), "outer": (0, 8)}):
             assert _rel(S.apply(op, 0, xd).cpu().numpy(), ref) < bar
@@ -105,6 +110,8 @@ def test_plane_tiles_are_refused_where_unavailable(gpu):
     for prec, t in ((4, {"inner": (0, 3), "mid": (2, 8), "outer": (2, 256)}),      # FP32 moves pairs of lines
                     (8, {"inner": (0, 64), "mid": (2, 8), "outer": (2, 256)}),
                     (8, {"inner": (0, 4), "mid": (2, 8), "outer": (2, 300)}),
+                    (8, {"inner": (0, 4), "mid": (2, 8), "outer": (3, 1024)}),
+                    (4, {"inner": (0, 4), "mid": (2, 8), "outer": (3, 256)}),
                     (8, {"inner": (2, 4), "mid": (2, 8), "outer": (2, 256)})):
         with pytest.raises(F.FameError):
             S.set_tiles(prec, t)
