@@ -157,17 +157,38 @@ __global__ void k_cg_alpha(CgScal* sc, const double* pap, int npap, const int* a
 
 /* <r,r> of the residual the contracting pass updated (its block sums, every step
  * doubles): b = r1 / r0 and the stopping rule (CG.cu:66-78) */
-__global__ void k_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int* active) {
+__device__ __forceinline__ void note_done(CgNote* n, unsigned seq) {
+    __threadfence_system();
+    __hip_atomic_store(&n->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void k_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int* active, CgNote* note, unsigned seq) {
     const int p = blockIdx.x;
-    if (!active[p]) return;
-    double v[1] = {0.0};
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) v[0] += partials[((size_t)p * nblk + b) * step];
-    block_sum_all<1>(v);
-    if (threadIdx.x != 0) return;
     CgScal& c = sc[p];
-    cg_rule(v[0], c.tol2, c.maxit, c.rr, c.beta, c.iters, c.active);
-    c.upd = 0;
-    active[p] = c.active;
+    if (active[p]) {
+        double v[1] = {0.0};
+        for (int b = threadIdx.x; b < nblk; b += blockDim.x) v[0] += partials[((size_t)p * nblk + b) * step];
+        block_sum_all<1>(v);
+        if (threadIdx.x == 0) {
+            cg_rule(v[0], c.tol2, c.maxit, c.rr, c.beta, c.iters, c.active);
+            c.upd = 0;
+            active[p] = c.active;
+        }
+    }
+    if (note && threadIdx.x == 0) {
+        note[p].sc = c;
+        note_done(note + p, seq);
+    }
+}
+__global__ void k_cg_note(const CgScal* sc, CgNote* note, unsigned seq) {
+    note[blockIdx.x].sc = sc[blockIdx.x];
+    note_done(note + blockIdx.x, seq);
+}
+__global__ void k_sum_note(const double* partials, int nblk, CgNote* note, unsigned seq) {
+    const int p = blockIdx.x;
+    const double s = sum_partials(partials, p, nblk, 1, 0);
+    if (threadIdx.x != 0) return;
+    note[p].sum = s;
+    note_done(note + p, seq);
 }
 
 /* the solution update x += alpha p still pending at the end of a solve */
@@ -189,13 +210,15 @@ __global__ void __launch_bounds__(RB) k_cg_finish_x(typename V2<T>::t* x, const 
 /* start of an FP32 solve from an FP64 right-hand side (the refinement's
  * residual): x = 0, r = p = b rounded to FP32, and the partials of <r,r> */
 __global__ void __launch_bounds__(RB) k_cg_begin_from64(float2* x, float2* r, float2* pv, const double2* b,
-                                                        double* partials, size_t n, size_t stride, const int* mask) {
+                                                        double* partials, size_t n, size_t stride, const int* mask,
+                                                        double2* x64) {
     const int p = blockIdx.y;
     double acc[1] = {0.0};
     if (!mask || mask[p]) {
         const size_t o = (size_t)p * stride;
         for (size_t i = (size_t)blockIdx.x * RB + threadIdx.x; i < n; i += (size_t)gridDim.x * RB) {
             const double2 w = b[o + i];
+            if (x64) x64[o + i] = make_double2(0.0, 0.0);
             const float2 v = make_float2((float)w.x, (float)w.y);
             x[o + i] = make_float2(0.0f, 0.0f); r[o + i] = v; pv[o + i] = v;
             const float s = v.x * v.x + v.y * v.y;
@@ -472,8 +495,17 @@ hipError_t fame_cg_alpha(CgScal* sc, const double* pap, int npap, int nprob, con
     hipLaunchKernelGGL(k_cg_alpha, dim3(nprob), dim3(RB), 0, s, sc, pap, npap, active);
     return hipGetLastError();
 }
-hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_beta, dim3(nprob), dim3(RB), 0, s, sc, partials, nblk, step, active);
+hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s,
+                        CgNote* note, unsigned seq) {
+    hipLaunchKernelGGL(k_cg_beta, dim3(nprob), dim3(RB), 0, s, sc, partials, nblk, step, active, note, seq);
+    return hipGetLastError();
+}
+hipError_t fame_cg_note(const CgScal* sc, int nprob, CgNote* note, unsigned seq, hipStream_t s) {
+    hipLaunchKernelGGL(k_cg_note, dim3(nprob), dim3(1), 0, s, sc, note, seq);
+    return hipGetLastError();
+}
+hipError_t fame_sum_note(const double* partials, int nblk, int nprob, CgNote* note, unsigned seq, hipStream_t s) {
+    hipLaunchKernelGGL(k_sum_note, dim3(nprob), dim3(RB), 0, s, partials, nblk, note, seq);
     return hipGetLastError();
 }
 hipError_t fame_cg_alpha_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s) {
@@ -493,9 +525,9 @@ hipError_t fame_cg_finish_x(void* x, const void* p, const CgScal* sc, size_t n, 
 }
 
 hipError_t fame_cg_begin_mixed(void* x32, void* r32, void* p32, const void* b64, double* partials, int nblk, size_t n,
-                               size_t stride, int nprob, const int* mask, hipStream_t s) {
+                               size_t stride, int nprob, const int* mask, hipStream_t s, void* x64) {
     hipLaunchKernelGGL(k_cg_begin_from64, vgrid(n, nprob, nblk), dim3(RB), 0, s, (float2*)x32, (float2*)r32, (float2*)p32,
-                       (const double2*)b64, partials, n, stride, mask);
+                       (const double2*)b64, partials, n, stride, mask, (double2*)x64);
     return hipGetLastError();
 }
 

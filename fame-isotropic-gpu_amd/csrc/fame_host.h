@@ -14,6 +14,10 @@ enum { LINE_EX_PLAIN = 0, LINE_EX_CG = 1, LINE_EX_FX = 2, LINE_CO_PLAIN = 0, LIN
 
 #define NBLK_VEC 1024   /* blocks per problem of the vector/reduction kernels */
 #define CG_GRAPH_ITERS 4   /* CG iterations per captured graph (fewer launch gaps between them) */
+/* and per graph of a solve that has come back often enough to pay for its capture:
+ * the gap between two graph launches is 8.4 us, 7% of four 32^3 iterations       */
+#define CG_GRAPH_LONG 16
+#define CG_GRAPH_USES 32   /* short graphs launched before the long one is captured */
 
 enum { FFT_ENGINE_AUTO = 0, FFT_ENGINE_STOCKHAM = 1, FFT_ENGINE_MFMA = 2 };
 enum { AX_INNER = 0, AX_MID = 1, AX_OUTER = 2 };
@@ -82,12 +86,17 @@ struct fame_ctx {
     int* active = nullptr;
     int* mask = nullptr;
     double* scal = nullptr;       /* 64 doubles per problem of small device scalars */
-    CgScal* sc_h = nullptr;       /* pinned host copy of cgsc */
+    std::vector<CgScal> sc_h;     /* host copy of cgsc */
+    CgNote* note = nullptr;       /* pinned, polled by the host */
+    unsigned note_seq = 0;
+    fame_status wait_notes(int nprob);
     std::vector<void*> allocs;
     std::vector<void*> big;       /* Lanczos basis etc., reallocated per solve shape */
     std::vector<size_t> big_bytes;  /* their sizes (the shape they were allocated for) */
     /* tuning / state */
-    int cg_predict[2] = {40, 40};
+    /* iterations the next solve is expected to take, per precision and refinement sweep */
+    int cg_predict[2][4] = {{24}, {24}};   /* 0: not known, the sweep before's count */
+    int cg_last[2][4] = {};
     /* inverse-iteration sweeps applied by fame_eigs to the converged Ritz pairs
      * (fame_set_refinement; 0 = the reference's algorithm), their absolute CG
      * tolerance and iteration limit */
@@ -121,7 +130,8 @@ struct fame_ctx {
      * checks of the active flags.  FAME_GRAPH=0 launches eagerly instead.   */
     bool use_graphs = true;
     hipStream_t cap_stream = nullptr;
-    std::map<std::tuple<int, int, int, const void*, int>, hipGraphExec_t> cg_graphs;
+    struct CgGraph { hipGraphExec_t exec = nullptr; int uses = 0; };
+    std::map<std::tuple<int, int, int, const void*, int>, CgGraph> cg_graphs;
     void drop_graphs();
     fame_status cg_iteration(int prec, void* x, int p0, int nprob, int count = 1);
     fame_status cg_step_ap(int prec, void* p, void* r, void* x, void* Ap, int p0, int nprob);
@@ -156,7 +166,8 @@ struct fame_ctx {
      * begun_nblk > 0: x, r, p were set up by qbq_residual32 (or the caller),
      * with the <r,r> partials in partials, begun_nblk per problem */
     fame_status cg(int prec, const void* b, void* x, int p0, int nprob, double tol, double reltol, int maxit,
-                   const int* mask_dev, int* iters, bool b64 = false, bool defer_finish = false, int begun_nblk = 0);
+                   const int* mask_dev, int* iters, bool b64 = false, bool defer_finish = false, int begun_nblk = 0,
+                   int slot = 0);
     /* refinement residual: xr += x32 + alpha p32 (the FP32 solve's result and
      * its pending update) on the first pass, then QBQ64 xr, whose last pass
      * stores the next FP32 solve's start r = p = FP32(b - QBQ64 xr), x = 0, and

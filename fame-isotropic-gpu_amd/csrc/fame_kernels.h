@@ -32,6 +32,14 @@ struct CgScal {
     int upd;          /* 1 when rr, beta, iters and active still lack the last iteration's <r,r> */
 };
 
+/* what a solve tells the host, in pinned memory that the host polls: the scalar
+ * state or a sum, then the sequence number that the host waits for            */
+struct CgNote {
+    CgScal sc;
+    double sum;
+    unsigned seq;
+};
+
 #ifdef __HIPCC__
 /* b = r1 / r0 and the stopping rule (CG.cu:66-78) from the new <r, r> */
 __device__ __forceinline__ void cg_rule(double s, double tol2, int maxit, double& rr, double& beta, int& iters, int& active) {
@@ -274,14 +282,18 @@ hipError_t fame_cg_init_scal(CgScal* sc, const double* partials, int nblk, doubl
  * the active flags from the exact <r,r> of the updated residual (slot 3 of the
  * inner partials) */
 hipError_t fame_cg_alpha(CgScal* sc, const double* pap, int npap, int nprob, const int* active, hipStream_t s);
-hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s);
+hipError_t fame_cg_beta(CgScal* sc, const double* partials, int nblk, int step, int nprob, int* active, hipStream_t s,
+                        CgNote* note = nullptr, unsigned seq = 0);
+/* the scalar state, or the sum of nblk partials per problem, into the notes */
+hipError_t fame_cg_note(const CgScal* sc, int nprob, CgNote* note, unsigned seq, hipStream_t s);
+hipError_t fame_sum_note(const double* partials, int nblk, int nprob, CgNote* note, unsigned seq, hipStream_t s);
 hipError_t fame_cg_alpha_beta(CgScal* sc, const double* partials, int nblk, int nprob, int* active, hipStream_t s);
 hipError_t fame_cg_finish_x(void* x, const void* p, const CgScal* sc, size_t n, size_t stride, int nprob, int prec,
                             hipStream_t s);
 /* an FP32 solve inside FP64 refinement starting from the FP64 right-hand
  * side: x32 = 0, r32 = p32 = b64 rounded, with the <r,r> partials */
 hipError_t fame_cg_begin_mixed(void* x32, void* r32, void* p32, const void* b64, double* partials, int nblk, size_t n,
-                               size_t stride, int nprob, const int* mask, hipStream_t s);
+                               size_t stride, int nprob, const int* mask, hipStream_t s, void* x64 = nullptr);
 
 /* generic helpers (complex double unless prec says float) */
 hipError_t fame_scale_real(void* y, const void* x, const double* sreal, size_t n, size_t xstride, size_t sstride,

@@ -326,7 +326,7 @@ static fame_status dalloc(fame_ctx* c, void** p, size_t bytes) {
 }
 
 void fame_ctx::drop_graphs() {
-    for (auto& kv : cg_graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto& kv : cg_graphs) (void)hipGraphExecDestroy(kv.second.exec);
     cg_graphs.clear();
 }
 
@@ -612,7 +612,9 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
     A(c->mask, sizeof(int) * B);
     A(c->scal, sizeof(double) * 64 * B);
 #undef A
-    HIPCHK(hipHostMalloc((void**)&c->sc_h, sizeof(CgScal) * B, 0));
+    c->sc_h.resize(B);
+    HIPCHK(hipHostMalloc((void**)&c->note, sizeof(CgNote) * B, hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset((void*)c->note, 0, sizeof(CgNote) * B);
     c->big.clear();
     *out = c;
     return FAME_OK;
@@ -627,7 +629,10 @@ extern "C" fame_status fame_destroy(fame_ctx* c) {
         (void)hipStreamDestroy(c->stream);
         c->stream = nullptr;
     }
-    if (c->sc_h) (void)hipHostFree(c->sc_h);
+    if (c->note) {
+        (void)hipSetDevice(c->device);
+        (void)hipHostFree(c->note);
+    }
     delete c;
     return FAME_OK;
 }
@@ -948,11 +953,16 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
         }
         case FAME_OP_INVAR:
         case FAME_OP_INVAR_MIXED: {
-            HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
             int it = 0;
             fame_ls ls = c->ls_last.maxit > 0 ? c->ls_last : fame_ls{1000, 1e-12};
-            CHK(c->invar(op == FAME_OP_INVAR ? FAME_PREC_F64 : FAME_PREC_F32_REFINE, xin, yout, ik, 1, nullptr, ls, &it));
-            HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
+            const int mode = op == FAME_OP_INVAR ? FAME_PREC_F64 : FAME_PREC_F32_REFINE;
+            if (Nd == N) {      /* no mode left out: the padded layout is the reference's */
+                CHK(c->invar(mode, x, yout, ik, 1, nullptr, ls, &it, 0, y, 2 * (size_t)N));
+            } else {
+                HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
+                CHK(c->invar(mode, xin, yout, ik, 1, nullptr, ls, &it));
+                HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
+            }
             c->last_iters = it;
             break;
         }
@@ -1001,9 +1011,9 @@ fame_status fame_ctx::tune(int prec) {
         void* r = prec == 8 ? cg64[0] : cg32[0];
         HIPCHK(hipMemsetAsync(r, 0, es * 2 * (size_t)N * nk, stream));
         HIPCHK(hipMemsetAsync(y, 0, es * 2 * (size_t)N * nk, stream));
-        std::memset(sc_h, 0, sizeof(CgScal) * nk);
+        std::fill(sc_h.begin(), sc_h.end(), CgScal{});
         for (int i = 0; i < nk; ++i) sc_h[i].pend = 1;    /* x read and written, as inside a solve */
-        HIPCHK(hipMemcpyAsync(cgsc, sc_h, sizeof(CgScal) * nk, hipMemcpyHostToDevice, stream));
+        HIPCHK(hipMemcpyAsync(cgsc, sc_h.data(), sizeof(CgScal) * nk, hipMemcpyHostToDevice, stream));
         plane_ms = 0;
         for (int contract = 0; contract < 2 && st == FAME_OK; ++contract) {
             PassTile& t = contract ? ctile[pi] : ltile[pi];
@@ -1184,11 +1194,30 @@ extern "C" fame_status fame_autotune(fame_ctx* c, int prec, int* choice) {
 /* ======================================================================== */
 /*  CG (batched)                                                             */
 /* ======================================================================== */
+/* wait until the notes of nprob problems carry note_seq.  The host polls: a copy
+ * kernel and hipStreamSynchronize took 35 us from the last kernel's end to the
+ * next one's start, this 10; a failed stream is noticed by its query           */
+fame_status fame_ctx::wait_notes(int nprob) {
+    for (int i = 0; i < nprob; ++i) {
+        const unsigned* q = &note[i].seq;
+        unsigned spins = 0;
+        while (__atomic_load_n(q, __ATOMIC_ACQUIRE) != note_seq) {
+            __builtin_ia32_pause();
+            if ((++spins & 0x3fff) != 0) continue;
+            const hipError_t e = hipStreamQuery(stream);
+            if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+            HIPCHK(e);
+            if (__atomic_load_n(q, __ATOMIC_ACQUIRE) != note_seq) FAIL(FAME_ERR_HIP, "solve: the device's note did not arrive");
+        }
+    }
+    return FAME_OK;
+}
+
 /* Solve QBQ x = b for problems p0..p0+nprob-1 (padded layout, precision prec).
  * Stops per problem when <r,r> <= max(tol^2, reltol^2 <b,b>) or after maxit
  * (reference counter semantics, CG.cu:36-78).  iters[] (host) receives k.    */
 fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, double tol, double reltol, int maxit,
-                         const int* mask_dev, int* iters, bool b64, bool defer_finish, int begun_nblk) {
+                         const int* mask_dev, int* iters, bool b64, bool defer_finish, int begun_nblk, int slot) {
     if (b64 && prec != 4) FAIL(FAME_ERR_ARG, "cg: an FP64 right-hand side needs prec 4");
     void** V = prec == 8 ? cg64 : cg32;
     const size_t n = 2 * (size_t)N, st = 2 * (size_t)N;
@@ -1201,24 +1230,34 @@ fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, do
     else HIPCHK(fame_cg_begin(x, r, p, b, partials, NBLK_VEC, n, st, nprob, prec, mask_dev, stream));
     HIPCHK(fame_cg_init_scal2(cgsc, partials, nbp, tol, reltol, maxit, nprob, active, mask_dev, stream));
     int done_it = 0;
-    int chunk = std::max(1, std::min(maxit, cg_predict[pix(prec)] - 1));
+    /* the iterations expected: an iteration too many costs three launches that
+     * return at once (10 us), one too few a round trip to the host (40 us)     */
+    int& predict = cg_predict[pix(prec)][slot];
+    if (predict == 0) predict = cg_last[pix(prec)][slot - 1];
+    int chunk = std::max(1, std::min(maxit, predict));
     while (true) {
         for (int it = 0; it < chunk;) {
-            const int k = std::min(chunk - it, CG_GRAPH_ITERS);
+            const int left = chunk - it;
+            int k = std::min(left, CG_GRAPH_ITERS);
+            if (left >= CG_GRAPH_LONG && use_graphs) {
+                const auto q = cg_graphs.find(std::make_tuple(prec, p0, nprob, (const void*)x, CG_GRAPH_ITERS));
+                if (q != cg_graphs.end() && q->second.uses >= CG_GRAPH_USES) k = CG_GRAPH_LONG;
+            }
             CHK(cg_iteration(prec, x, p0, nprob, k));
             it += k;
         }
         done_it += chunk;
-        /* the last iteration's beta, count and flags, which the next expansion would form */
-        if (folds(prec)) HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), 1, nprob, active, stream));
-        /* the whole scalar state comes back, so that the last check also
-         * holds the final iteration counts (no read-back after the loop) */
-        HIPCHK(hipMemcpyAsync(sc_h, cgsc, sizeof(CgScal) * nprob, hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
+        /* the last iteration's beta, count and flags, which the next expansion would
+         * form; the whole scalar state comes back, so that the last check also holds
+         * the final iteration counts                                           */
+        ++note_seq;
+        if (folds(prec)) HIPCHK(fame_cg_beta(cgsc, partials2, inner_blocks(prec), 1, nprob, active, stream, note, note_seq));
+        else HIPCHK(fame_cg_note(cgsc, nprob, note, note_seq, stream));
+        CHK(wait_notes(nprob));
         int any = 0;
-        for (int i = 0; i < nprob; ++i) any |= sc_h[i].active;
+        for (int i = 0; i < nprob; ++i) { sc_h[i] = note[i].sc; any |= sc_h[i].active; }
         if (!any || done_it >= maxit) break;
-        chunk = 2;
+        chunk = CG_GRAPH_ITERS;
     }
     if (!defer_finish) HIPCHK(fame_cg_finish_x(x, p, cgsc, n, st, nprob, prec, stream));
     int mx = 0;
@@ -1229,7 +1268,10 @@ fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, do
         applied += sc_h[i].iters - 1;
     }
     if (prec == 8) cnt_qbq64 += applied; else cnt_qbq32 += applied;
-    cg_predict[pix(prec)] = std::max(2, mx - 1);
+    int& last = cg_last[pix(prec)][slot];
+    const int its = std::max(1, mx - 1);
+    predict = std::max(its, std::min(last, its + 1));      /* counts that go up and down by one: the larger */
+    last = its;
     return FAME_OK;
 }
 
@@ -1321,9 +1363,10 @@ fame_status fame_ctx::cg_iteration(int prec, void* x, int p0, int nprob, int cou
         e = hipGraphInstantiate(&ex, gr, nullptr, nullptr, 0);
         (void)hipGraphDestroy(gr);
         HIPCHK(e);
-        itg = cg_graphs.emplace(key, ex).first;
+        itg = cg_graphs.emplace(key, CgGraph{ex, 0}).first;
     }
-    HIPCHK(hipGraphLaunch(itg->second, stream));
+    ++itg->second.uses;
+    HIPCHK(hipGraphLaunch(itg->second.exec, stream));
     return FAME_OK;
 }
 
@@ -1362,10 +1405,9 @@ fame_status fame_ctx::invar(int mode, const void* x, void* y, int p0, int nprob,
          * x = 0) with its norm on its last, so no FP64 residual vector is kept */
         double2* xr = (double2*)y;
         float2* d32 = (float2*)cg32[4] + st * p0;
-        HIPCHK(hipMemsetAsync(xr, 0, 16 * st * nprob, stream));
         /* the first FP32 solve starts from b (x = 0, r = p = FP32(b)) */
         HIPCHK(fame_cg_begin_mixed(d32, (char*)cg32[0] + 8 * st * p0, (char*)cg32[1] + 8 * st * p0, b, partials,
-                                   NBLK_VEC, n, st, nprob, nullptr, stream));
+                                   NBLK_VEC, n, st, nprob, nullptr, stream, xr));
         int nbp = NBLK_VEC;
         std::vector<int> msk(nprob, 1);
         if (mask_host) {
@@ -1376,19 +1418,26 @@ fame_status fame_ctx::invar(int mode, const void* x, void* y, int p0, int nprob,
         }
         double tol2 = ls.tol * ls.tol;
         for (int sweep = 0; sweep < refine_max_sweeps; ++sweep) {
-            HIPCHK(fame_reduce_partials(partials, nbp, 1, scal, nprob, stream));
-            std::vector<double> rn(nprob);
-            HIPCHK(hipMemcpyAsync(rn.data(), scal, sizeof(double) * nprob, hipMemcpyDeviceToHost, stream));
-            HIPCHK(hipStreamSynchronize(stream));
-            int any = 0;
-            for (int i = 0; i < nprob; ++i) { msk[i] = msk[i] && (rn[i] > tol2); any |= msk[i]; }
-            if (!any) break;
-            HIPCHK(hipMemcpyAsync(mask, msk.data(), sizeof(int) * nprob, hipMemcpyHostToDevice, stream));
+            /* the residual's norm decides on the host from the second sweep on; a
+             * right-hand side below the tolerance ends the first solve at once   */
+            if (sweep > 0) {
+                ++note_seq;
+                HIPCHK(fame_sum_note(partials, nbp, nprob, note, note_seq, stream));
+                CHK(wait_notes(nprob));
+                for (int i = 0; i < nprob; ++i) msk[i] = msk[i] && (note[i].sum > tol2);
+            }
+            const int on = (int)std::count(msk.begin(), msk.end(), 1);
+            if (!on) break;
+            const int* md = nullptr;
+            if (on < nprob) {
+                HIPCHK(hipMemcpyAsync(mask, msk.data(), sizeof(int) * nprob, hipMemcpyHostToDevice, stream));
+                md = mask;
+            }
             std::vector<int> it32(nprob, 0);
-            CHK(cg(4, b, d32, p0, nprob, ls.tol, refine_reltol, ls.maxit, mask, it32.data(), true, true, nbp));
+            CHK(cg(4, b, d32, p0, nprob, ls.tol, refine_reltol, ls.maxit, md, it32.data(), true, true, nbp, std::min(sweep, 3)));
             for (int i = 0; i < nprob; ++i) if (msk[i]) it[i] += it32[i] - 1;
             /* the next sweep's start from r = b - QBQ64 xr, with its norm */
-            CHK(qbq_residual32(xr, b, d32, p0, nprob, mask, (int)std::count(msk.begin(), msk.end(), 1)));
+            CHK(qbq_residual32(xr, b, d32, p0, nprob, md, on));
             nbp = inner_blocks(8);
         }
         for (int i = 0; i < nprob; ++i) it[i] += 1;
