@@ -472,7 +472,7 @@ extern "C" fame_status fame_eig_grad(fame_ctx* c, int nwant, const double* freq,
     /* as many bands at a time as stay in the 256 MB of Infinity Cache between the
      * norm's pass and the sum's.  One host round trip per call instead of one per
      * band: with the restoration before it, SC 64, 4 wave vectors x 6 bands,
-     * 2.49 -> 0.80 ms                                                          */
+     * 2.49 -> 0.75 ms                                                          */
     const int chunk = (int)std::min<size_t>(GRAD_CHUNK, std::max<size_t>(1, ((size_t)192 << 20) / (16 * N3)));
     if (nk < 1) HIPCHK(hipMemsetAsync(grad_dev, 0, sizeof(double) * N3, c->stream));
     for (int p = 0; p < nk; ++p) {

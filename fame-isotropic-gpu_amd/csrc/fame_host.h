@@ -61,6 +61,7 @@ struct fame_ctx {
     int PP = 0, CS = 0;           /* plane pitch and component stride (na PP)  */
     PlaneAxis laxis[2][2];        /* inner axis [precision][engine], n = 0 when not available */
     KPlane kpl[2];
+    int syn_wide = 0;             /* the one-way kernels' variant */
     PlaneAxis wide_ax[2];         /* b and c of the FP64 plane kernel's wide variant */
     void *invBp[2] = {nullptr, nullptr}, *ltw[2] = {nullptr, nullptr}, *mtw[2] = {nullptr, nullptr}, *eatab = nullptr;
     double2* otw = nullptr;

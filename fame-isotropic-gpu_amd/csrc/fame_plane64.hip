@@ -52,7 +52,7 @@ hipError_t fame_launch_line_tab(const GridDev& g, const ProbDev* prob, LineTab* 
  * LDS.  They replace k_mid + k_outer + k_xz_transpose (18 N s of field traffic) and
  * the conversions of the reduced vector (8 N s) by one pass (6 N s): Qrs of
  * a 50 x 42 x 36 grid 59 -> 34 us, residuals of 4 wave vectors x 12 bands on the
- * FCC 64 grid 3.27 -> 1.56 ms.  Bound by the LDS passes and, where a plane is over
+ * FCC 64 grid 3.27 -> 1.32 ms.  Bound by the LDS passes and, where a plane is over
  * half a CU's LDS, by one block per CU.  The outer phases come from a table in
  * global memory, so that every grid whose k_plane fits the LDS fits here too  */
 namespace fame {
@@ -77,8 +77,9 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
  *   SYN_REF    D/N v into out, reference's layout;
  *   SYN_EPS    D v / (N eps) back in place, with its |.|^2 per block;
  *   SYN_RES    |D/N v - w2 eps E|^2 and |E|^2 per block, nothing stored          */
-template <int ENGB, int ENGC, int MODE>
-__global__ void __launch_bounds__(512) k_syn(KSyn a) {
+template <int ENGB, int ENGC, int MODE, int TB>
+__global__ void __launch_bounds__(TB) k_syn(KSyn a) {
+    constexpr int MAXE = TB == 512 ? 16 : 8;     /* as k_plane */
     typedef double2 T2;
     const KPlane& k = a.k;
     const int npl = 3 * k.g.na;
@@ -99,24 +100,20 @@ __global__ void __launch_bounds__(512) k_syn(KSyn a) {
     hk.tw = reinterpret_cast<const T2*>(k.tw) + (size_t)p * plane;
     hk.eps = nullptr; hk.ld = nb; hk.pap = false;
     rows_in<double, T2, 4>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
-    line_transform<double, T2, ENGB, true, 16>(S, nc, Pb, 1, k.b, Wb);
-    column_transform<double, T2, ENGC, true, 16>(S, nb, Pb, k.c, Wc, hk);
+    line_transform<double, T2, ENGB, true, MAXE>(S, nc, Pb, 1, k.b, Wb);
+    column_transform<double, T2, ENGC, true, MAXE>(S, nb, Pb, k.c, Wc, hk);
     __syncthreads();
     const double invN = 1.0 / (double)k.g.N;
     if constexpr (MODE == SYN_FIELD || MODE == SYN_EPS) {
         const double* ie = reinterpret_cast<const double*>(k.invB) + po;
         double acc = 0.0;
-        for (int i = threadIdx.x; i < plane; i += blockDim.x) {
-            const int c = udiv(i, k.mnb), b = i - c * nb;
-            T2 v = cmul(S[c * Pb + b], D[c]);
-            if (MODE == SYN_EPS) {
-                v = cscale(v, ie[i]);
-                acc += v.x * v.x + v.y * v.y;
-            } else {
-                v = cscale(v, invN);
-            }
-            F[i] = v;
-        }
+        batched_loop<8>(plane, [&](int i) -> double { return MODE == SYN_EPS ? ie[i] : invN; },
+            [&](int i, double e) {
+                const int c = udiv(i, k.mnb), b = i - c * nb;
+                const T2 v = cscale(cmul(S[c * Pb + b], D[c]), e);
+                if (MODE == SYN_EPS) acc += v.x * v.x + v.y * v.y;
+                F[i] = v;
+            });
         if constexpr (MODE == SYN_EPS) {
             const double s = block_sum(acc, red);
             if (threadIdx.x == 0) a.part[(size_t)p * npl + pl] = s;
@@ -136,13 +133,15 @@ __global__ void __launch_bounds__(512) k_syn(KSyn a) {
             const double* ep = a.eps + ro;
             const double w2 = a.w2[(size_t)p * a.w2step];
             double r2 = 0.0, e2 = 0.0;
-            for (int i = threadIdx.x; i < plane; i += blockDim.x) {
-                const int b = udiv(i, k.c.mn), c = i - b * nc;
-                const T2 v = cscale(cmul(S[c * Pb + b], D[c]), invN), e = E[i];
-                const double s = w2 * ep[i], rx = v.x - s * e.x, ry = v.y - s * e.y;
-                r2 += rx * rx + ry * ry;
-                e2 += e.x * e.x + e.y * e.y;
-            }
+            struct In { T2 e; double ep; };
+            batched_loop<4>(plane, [&](int i) -> In { return In{E[i], ep[i]}; },
+                [&](int i, const In& d) {
+                    const int b = udiv(i, k.c.mn), c = i - b * nc;
+                    const T2 v = cscale(cmul(S[c * Pb + b], D[c]), invN), e = d.e;
+                    const double s = w2 * d.ep, rx = v.x - s * e.x, ry = v.y - s * e.y;
+                    r2 += rx * rx + ry * ry;
+                    e2 += e.x * e.x + e.y * e.y;
+                });
             r2 = block_sum(r2, red);
             e2 = block_sum(e2, red);
             if (threadIdx.x == 0) {
@@ -155,8 +154,9 @@ __global__ void __launch_bounds__(512) k_syn(KSyn a) {
 
 /* conj outer twiddle and forward transforms along c and b of one plane, read from
  * `in` (reference's layout, General) or in place, stored in the plane layout  */
-template <int ENGB, int ENGC>
-__global__ void __launch_bounds__(512) k_ana(KSyn a) {
+template <int ENGB, int ENGC, int TB>
+__global__ void __launch_bounds__(TB) k_ana(KSyn a) {
+    constexpr int MAXE = TB == 512 ? 16 : 8;
     typedef double2 T2;
     const KPlane& k = a.k;
     const int npl = 3 * k.g.na;
@@ -189,8 +189,8 @@ __global__ void __launch_bounds__(512) k_ana(KSyn a) {
     Hook<double, T2> hk;
     hk.tw = reinterpret_cast<const T2*>(k.tw) + (size_t)p * plane;
     hk.eps = nullptr; hk.ld = nb; hk.pap = false;
-    column_transform<double, T2, ENGC, false, 16>(S, nb, Pb, k.c, Wc, hk);
-    line_transform<double, T2, ENGB, false, 16>(S, nc, Pb, 1, k.b, Wb);
+    column_transform<double, T2, ENGC, false, MAXE>(S, nb, Pb, k.c, Wc, hk);
+    line_transform<double, T2, ENGB, false, MAXE>(S, nc, Pb, 1, k.b, Wb);
     __syncthreads();
     rows_out<double, T2>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
 }
@@ -379,34 +379,41 @@ __global__ void __launch_bounds__(256) k_eps(GridDev g, const double* __restrict
 
 }  // namespace fame
 
-template <int EB, int EC>
+template <int EB, int EC, int TB>
 static const void* syn_fn(int mode) {
     switch (mode) {
-        case SYN_FIELD: return (const void*)k_syn<EB, EC, SYN_FIELD>;
-        case SYN_REF: return (const void*)k_syn<EB, EC, SYN_REF>;
-        case SYN_EPS: return (const void*)k_syn<EB, EC, SYN_EPS>;
-        case SYN_RES: return (const void*)k_syn<EB, EC, SYN_RES>;
-        default: return (const void*)k_ana<EB, EC>;
+        case SYN_FIELD: return (const void*)k_syn<EB, EC, SYN_FIELD, TB>;
+        case SYN_REF: return (const void*)k_syn<EB, EC, SYN_REF, TB>;
+        case SYN_EPS: return (const void*)k_syn<EB, EC, SYN_EPS, TB>;
+        case SYN_RES: return (const void*)k_syn<EB, EC, SYN_RES, TB>;
+        default: return (const void*)k_ana<EB, EC, TB>;
     }
 }
+template <int TB>
 static const void* syn_fn(int eb, int ec, int mode) {
-    if (eb == ENG_MFMA) return ec == ENG_MFMA ? syn_fn<ENG_MFMA, ENG_MFMA>(mode) : syn_fn<ENG_MFMA, ENG_STOCKHAM>(mode);
-    return ec == ENG_MFMA ? syn_fn<ENG_STOCKHAM, ENG_MFMA>(mode) : syn_fn<ENG_STOCKHAM, ENG_STOCKHAM>(mode);
+    if (eb == ENG_MFMA) return ec == ENG_MFMA ? syn_fn<ENG_MFMA, ENG_MFMA, TB>(mode) : syn_fn<ENG_MFMA, ENG_STOCKHAM, TB>(mode);
+    return ec == ENG_MFMA ? syn_fn<ENG_STOCKHAM, ENG_MFMA, TB>(mode) : syn_fn<ENG_STOCKHAM, ENG_STOCKHAM, TB>(mode);
 }
 hipError_t fame_prepare_syn(int eb, int ec) {
-    for (int m = 0; m < 5; ++m) {
-        const hipError_t e = hipFuncSetAttribute(syn_fn(eb, ec, m), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
+    for (int m = 0; m < 10; ++m) {
+        const hipError_t e = hipFuncSetAttribute(m < 5 ? syn_fn<512>(eb, ec, m) : syn_fn<1024>(eb, ec, m - 5),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
+/* the wide variant (k.wide) where k_plane starts with it; its 256 registers leave a
+ * CU 512 threads, in two blocks where two planes fit and there are that many.
+ * The narrow one's two blocks of 512 threads: residuals of 4 wave vectors x 12
+ * bands, FCC 64, 1.32 ms against 1.54 with the wide one                       */
 static hipError_t launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) {
     KSyn q = k;
     q.k.nprob = nprob;
     void* arg[] = {&q};
-    const int nt = k.k.nt > 512 ? 512 : k.k.nt;
-    return hipLaunchKernel(syn_fn(k.k.b.eng, k.k.c.eng, mode), dim3(xcd_round(3 * k.k.g.na * nprob)), dim3(nt), arg,
-                           fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab, 8), s);
+    const size_t lds = fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab, 8);
+    const int nt = lds <= FAME_LDS_HALF && k.k.wide && 3 * k.k.g.na * nprob > 512 ? 256 : 512;
+    return hipLaunchKernel(k.k.wide ? syn_fn<512>(k.k.b.eng, k.k.c.eng, mode) : syn_fn<1024>(k.k.b.eng, k.k.c.eng, mode),
+                           dim3(xcd_round(3 * k.k.g.na * nprob)), dim3(nt), arg, lds, s);
 }
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) { return launch_syn(k, mode, nprob, s); }
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s) { return launch_syn(k, 4, nprob, s); }

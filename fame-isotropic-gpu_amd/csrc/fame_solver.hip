@@ -417,7 +417,10 @@ fame_status fame_ctx::plane_setup() {
         if (!line_tile_ok(prec, eng, L)) { plane_ok[pi] = false; continue; }
         ltile[pi].eng = eng; ltile[pi].L = L; ltile[pi].P = g.na | 1;
         ctile[pi] = ltile[pi];
-        if (prec == 8) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+        if (prec == 8) {
+            syn_wide = k.wide;
+            HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+        }
         HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng) : fame_prepare_plane32(k.b.eng, k.c.eng));
         /* before tuning: an FP64 plane that fills a CU alone pays where one
          * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
@@ -475,7 +478,9 @@ KSyn fame_ctx::ksyn(int p0) const {
     KSyn a;
     std::memset(&a, 0, sizeof(a));
     a.k = kplane(8, p0, nullptr);
-    a.k.b = wide_ax[0]; a.k.c = wide_ax[1];
+    a.k.wide = syn_wide;
+    a.k.b = syn_wide ? wide_ax[0] : kpl[0].b;
+    a.k.c = syn_wide ? wide_ax[1] : kpl[0].c;
     a.outer = otw + (size_t)g.nc * p0;
     a.ostride = 3 * (size_t)N;
     return a;
@@ -882,6 +887,12 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
     double2* xin = (double2*)c->ref64[0];
     double2* yout = (double2*)c->ref64[1];
     const size_t pn = (size_t)c->g.nb * c->g.nc;
+    /* with no mode left out the padded layout is the reference's: no copies */
+    const bool same = Nd == N;
+    const void* xi = same ? x : xin;
+    void* yo = same ? y : (void*)yout;
+    auto pack = [&]() { return same ? hipSuccess : fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream); };
+    auto unpack = [&]() { return same ? hipSuccess : fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream); };
     switch (op) {
         case FAME_OP_QR:
             if (c->plane_ok[0]) {
@@ -900,8 +911,8 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             }
             [[fallthrough]];
         case FAME_OP_PR:
-            HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
-            CHK(c->qr_field(xin, ik, 1, op == FAME_OP_PR ? 1 : 0, nullptr));
+            HIPCHK(pack());
+            CHK(c->qr_field(xi, ik, 1, op == FAME_OP_PR ? 1 : 0, nullptr));
             CHK(c->field_to_ref(c->F64 + (size_t)ik * 3 * N, y, 1, 3 * (size_t)N));
             break;
         case FAME_OP_QRS:
@@ -920,8 +931,8 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             [[fallthrough]];
         case FAME_OP_PRS:
             CHK(c->field_from_ref(x, c->F64 + (size_t)ik * 3 * N, 1));
-            CHK(c->qrs_field(yout, ik, 1, op == FAME_OP_PRS ? 1 : 0, nullptr));
-            HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
+            CHK(c->qrs_field(yo, ik, 1, op == FAME_OP_PRS ? 1 : 0, nullptr));
+            HIPCHK(unpack());
             break;
         case FAME_OP_QBQ:
             if (c->plane[0]) {
@@ -935,20 +946,20 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
                 ++c->cnt_qbq64;
                 break;
             }
-            HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
+            HIPCHK(pack());
             /* the field slot used by qbq is that of problem ik */
-            CHK(c->qbq(8, xin, yout, ik, 1, nullptr, nullptr));
-            HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
+            CHK(c->qbq(8, xi, yo, ik, 1, nullptr, nullptr));
+            HIPCHK(unpack());
             break;
         case FAME_OP_QBQ32: {
             /* FP32 QBQ (the inner operator of the mixed-precision solver), FP64 in/out */
             float2* x32 = (float2*)c->cg32[3] + (size_t)ik * 2 * N;
             float2* y32 = (float2*)c->cg32[4] + (size_t)ik * 2 * N;
-            HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
-            HIPCHK(fame_convert(x32, 4, xin, 8, 2 * (size_t)N, 0, 0, 1, c->stream));
+            HIPCHK(pack());
+            HIPCHK(fame_convert(x32, 4, xi, 8, 2 * (size_t)N, 0, 0, 1, c->stream));
             CHK(c->qbq(4, x32, y32, ik, 1, nullptr, nullptr));
-            HIPCHK(fame_convert(yout, 8, y32, 4, 2 * (size_t)N, 0, 0, 1, c->stream));
-            HIPCHK(fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream));
+            HIPCHK(fame_convert(yo, 8, y32, 4, 2 * (size_t)N, 0, 0, 1, c->stream));
+            HIPCHK(unpack());
             break;
         }
         case FAME_OP_INVAR:
@@ -956,7 +967,7 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             int it = 0;
             fame_ls ls = c->ls_last.maxit > 0 ? c->ls_last : fame_ls{1000, 1e-12};
             const int mode = op == FAME_OP_INVAR ? FAME_PREC_F64 : FAME_PREC_F32_REFINE;
-            if (Nd == N) {      /* no mode left out: the padded layout is the reference's */
+            if (same) {
                 CHK(c->invar(mode, x, yout, ik, 1, nullptr, ls, &it, 0, y, 2 * (size_t)N));
             } else {
                 HIPCHK(fame_launch_pack(x, xin, N, Nd, +1, 8, c->stream));
