@@ -328,7 +328,9 @@ def main():
     traffic, traffic_note = measured_traffic(f"k_{cg_names[dom]}_fp32", tiles, list(fl.grid_nums), args.nk)
     qbq_alg = (10 * N * s32 + 3 * N * r32) * args.nk
     qbq_gbs = qbq_alg / (us32[5] * 1e-6) / 1e9
-    cg_iter_gbs = sum(cg_bytes) * args.nk / (cg32[7] * 1e-6) / 1e9
+    # the kernels that ran: with the outer axes in one plane pass (reported as
+    # cg_outer_eps) there are no middle passes
+    cg_iter_gbs = sum(b for b, t in zip(cg_bytes, cg32) if t > 0) * args.nk / (cg32[7] * 1e-6) / 1e9
     S.close()
 
     # ---- plain FP64, one wave vector at a time ----
@@ -418,7 +420,8 @@ def main():
         "cg_iteration_us": float(cg32[7]), "cg_iteration_gbs": cg_iter_gbs,
         "cg_kernels_us": dict(zip(cg_names, map(float, cg32[:7]))),
         "tuned_tiles": tiles,
-        "roofline": {"bound": "hbm", "kernel": f"{cg_names[dom]} (FP32 k_inner/k_mid/k_outer with the fused CG "
+        "roofline": {"bound": "hbm", "kernel": f"{cg_names[dom]} (FP32 "
+                                               f"{'k_inner/k_mid/k_outer' if cg32[1] > 0 else 'k_expand/k_plane/k_contract'} with the fused CG "
                                                f"updates, {args.nk} wave vectors active per launch)",
                      "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_note,

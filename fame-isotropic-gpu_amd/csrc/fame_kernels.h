@@ -170,7 +170,7 @@ struct KPlane {
     double* pap;                 /* optional <v, eps^-1 v / N> per block, [problem][component][a] */
     PlaneAxis b, c;
     unsigned mnb;
-    int nprob, nt;
+    int nt;
     int wide;                    /* FP64: the variant of at most 512 threads with 16 elements each */
 };
 

@@ -284,13 +284,15 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         c->kids.clear();
         c->kid_nk = 0;
         /* a child holds the per-problem work vectors of its wave vectors
-         * (about 400 N bytes each) and its own permittivity; the Lanczos
+         * (about 400 N bytes each, and the plane path's tables) and its own
+         * permittivity; the Lanczos
          * buffers (U, W) move from the parent to the children */
         size_t freeb = 0, totalb = 0;
         HIPCHK(hipMemGetInfo(&freeb, &totalb));
         const size_t N = c->N, n2 = 2 * N;
         const size_t lz = 16 * n2 * ((size_t)nstep + 1 + (size_t)nwant + 1) * (size_t)c->nk;
-        const size_t need = 400 * N * (size_t)c->nk + 100 * N * (size_t)G + lz + ((size_t)1 << 30);
+        const size_t tab = (size_t)c->g.nb * c->g.nc * (sizeof(LineTab) + 24 * ((size_t)inner_tw_per_line(c->g.na) + 1));
+        const size_t need = (400 * N + tab) * (size_t)c->nk + 136 * N * (size_t)G + lz + ((size_t)1 << 30);
         if (freeb < need) return FAME_OK;
         for (int i = 0; i < G; ++i) {
             fame_ctx* k = nullptr;

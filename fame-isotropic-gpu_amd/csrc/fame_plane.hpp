@@ -185,6 +185,12 @@ __global__ void __launch_bounds__(FFT_THREADS) k_expand(KLine k) {
     if (l0 >= nlines) return;
     const bool fold = MODE == EX_CG && k.sc2;
     if (!fold && k.active && !k.active[p]) return;
+    /* in a batch the blocks of problems that are done must not load anything; a
+     * single problem is rarely done, and its loads need not wait for the flag   */
+    if (fold && gridDim.y > 1 && !k.cgsc[p].active) {
+        if (tile == 0 && threadIdx.x == 0) { cg_copy(k.sc2[p], k.cgsc[p]); k.act_out[p] = 0; }
+        return;
+    }
     __shared__ double red[FFT_THREADS / 64];
     const int nl = min(L, nlines - l0);
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -404,6 +410,10 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
     if (l0 >= nlines) return;
     const bool fold = MODE == CO_CG && k.sc2;
     if (!fold && k.active && !k.active[p]) return;
+    if (fold && gridDim.y > 1 && !k.sc2[p].active) {
+        if (tile == 0 && threadIdx.x == 0) cg_copy(k.sc1[p], k.sc2[p]);
+        return;
+    }
     __shared__ double red[FFT_THREADS / 64];
     const int nl = min(L, nlines - l0);
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -683,13 +693,13 @@ __global__ void __launch_bounds__(TB) k_plane(KPlane k) {
     /* FP64: 16 elements per thread, and with them the compound radices, where a
      * block of 512 threads leaves 256 registers                              */
     constexpr int MAXE = sizeof(T) == 8 && TB == 512 ? 16 : MaxE<T>::v;
-    /* blocks of one XCD (x mod 8) take a run of consecutive planes, problem by
-     * problem: the problem's middle twiddles stay in that XCD's L2            */
+    /* every problem's planes go to all XCDs, a run of consecutive ones each: late in
+     * a batch's solve only a few problems iterate (a run over all problems' planes
+     * kept those on one or two XCDs: 4.62 k-pts/s on the FCC 96 batch of 30)   */
     touch_args<sizeof(KPlane)>();
     const int npl = 3 * k.g.na;
-    const int id = xcd_tile();
-    if (id >= npl * k.nprob) return;
-    const int p = id / npl, pl = id - p * npl;
+    const int p = blockIdx.y, pl = xcd_tile();
+    if (pl >= npl) return;
     if (k.active && !k.active[p]) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int nb = k.b.n, nc = k.c.n, plane = nb * nc, Pb = nb | 1;
@@ -771,10 +781,9 @@ static const void* plane_fn(int eb, int ec, int wide) {
 template <typename T>
 static hipError_t launch_plane(const KPlane& k, int nprob, hipStream_t s) {
     KPlane q = k;
-    q.nprob = nprob;
     void* arg[] = {&q};
     const size_t lds = fame_plane_lds(k.b.n, k.c.n, k.b.ntab + k.c.ntab, (int)sizeof(T));
-    return hipLaunchKernel(plane_fn<T>(k.b.eng, k.c.eng, k.wide), dim3(xcd_round(3 * k.g.na * nprob)), dim3(k.nt), arg, lds, s);
+    return hipLaunchKernel(plane_fn<T>(k.b.eng, k.c.eng, k.wide), dim3(xcd_round(3 * k.g.na), nprob), dim3(k.nt), arg, lds, s);
 }
 template <typename T>
 static hipError_t prepare_plane(int eb, int ec) {

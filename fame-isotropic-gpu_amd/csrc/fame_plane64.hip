@@ -83,9 +83,8 @@ __global__ void __launch_bounds__(TB) k_syn(KSyn a) {
     typedef double2 T2;
     const KPlane& k = a.k;
     const int npl = 3 * k.g.na;
-    const int id = xcd_tile();
-    if (id >= npl * k.nprob) return;
-    const int p = id / npl, pl = id - p * npl;
+    const int p = blockIdx.y, pl = xcd_tile();
+    if (pl >= npl) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ double red[8];
     const int nb = k.b.n, nc = k.c.n, plane = nb * nc, Pb = nb | 1;
@@ -160,9 +159,8 @@ __global__ void __launch_bounds__(TB) k_ana(KSyn a) {
     typedef double2 T2;
     const KPlane& k = a.k;
     const int npl = 3 * k.g.na;
-    const int id = xcd_tile();
-    if (id >= npl * k.nprob) return;
-    const int p = id / npl, pl = id - p * npl;
+    const int p = blockIdx.y, pl = xcd_tile();
+    if (pl >= npl) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int nb = k.b.n, nc = k.c.n, plane = nb * nc, Pb = nb | 1;
     T2* S = reinterpret_cast<T2*>(smem_raw);
@@ -408,12 +406,11 @@ hipError_t fame_prepare_syn(int eb, int ec) {
  * bands, FCC 64, 1.32 ms against 1.54 with the wide one                       */
 static hipError_t launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) {
     KSyn q = k;
-    q.k.nprob = nprob;
     void* arg[] = {&q};
     const size_t lds = fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab, 8);
     const int nt = lds <= FAME_LDS_HALF && k.k.wide && 3 * k.k.g.na * nprob > 512 ? 256 : 512;
     return hipLaunchKernel(k.k.wide ? syn_fn<512>(k.k.b.eng, k.k.c.eng, mode) : syn_fn<1024>(k.k.b.eng, k.k.c.eng, mode),
-                           dim3(xcd_round(3 * k.k.g.na * nprob)), dim3(nt), arg, lds, s);
+                           dim3(xcd_round(3 * k.k.g.na), nprob), dim3(nt), arg, lds, s);
 }
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) { return launch_syn(k, mode, nprob, s); }
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s) { return launch_syn(k, 4, nprob, s); }

@@ -221,8 +221,9 @@ fame_status fame_time_qbq_passes(fame_ctx* ctx, int prec, int reps, double* us6)
  * the kernels of one fused CG iteration with every wave vector active:
  * us8 = {inner expand with the x and p updates, middle inverse, outer eps with
  * the <p,Ap> sums, alpha, middle forward, inner contract with the r update and
- * <r,r> sums, beta, whole iteration}; prec = 8 or 4 (the middle entries 0 with the
- * plane kernel).  FAME_ERR_UNSUPPORTED when
+ * <r,r> sums, beta, whole iteration}; prec = 8 or 4.  With the plane kernel the
+ * middle entries are 0, and so are alpha and beta where the inner kernels form
+ * them.  FAME_ERR_UNSUPPORTED when
  * an axis takes a Bluestein plan (that iteration form stores Ap).  Measurement
  * helper, no reference counterpart.                                          */
 fame_status fame_time_cg_passes(fame_ctx* ctx, int prec, int reps, double* us8);
@@ -235,7 +236,8 @@ fame_status fame_time_cg_passes(fame_ctx* ctx, int prec, int reps, double* us8);
  * Stockham/Bluestein, 1 direct DFT on the matrix cores).  Where the two outer
  * axes of a QBQ run as one pass over (b, c) planes in LDS, the middle and outer
  * engines are 2, and the lines are those of the expanding kernel (inner), of
- * the contracting kernel (middle) and the plane kernel's threads (outer).
+ * the contracting kernel (middle) and the plane kernel's threads (outer); outer
+ * engine 3 is the FP64 plane kernel's variant of at most 512 threads.
  * Replaces the fixed
  * cuFFT plans of FAME_Create_cublas (FAME_Main/FAME_Create_cublas.cu:16-25).  */
 fame_status fame_autotune(fame_ctx* ctx, int prec, int* choice);
