@@ -61,7 +61,9 @@ static bool is_prime_radix(int r) { return r == 2 || r == 3 || r == 4 || r == 5 
  * (the twiddle-free first pass gets the largest butterfly).  compound = false
  * leaves out 6, 9, 10, 12, 15 and 16: the FP64 kernels hold 8 complex elements
  * per thread, and the extra registers of the two-level butterflies cost them
- * more waves than the saved pass gives back (measured on gfx950).           */
+ * more waves than the saved pass gives back (measured on gfx950).  Where a plane
+ * of the plane kernel fills a CU there are registers to spare: its wide variant
+ * takes FP32's radices.                                                      */
 static bool factor_gpu(int n, std::vector<int>* rad, bool compound = true) {
     static const int RADS[] = {16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
     std::vector<double> cost(n + 1, 1e30);
