@@ -191,5 +191,13 @@ struct fame_ctx {
     ~fame_ctx();
 };
 
+/* what fame_create takes from the environment; the children of a batch take their
+ * parent's, since they run with its plans and tiles                           */
+struct fame_settings {
+    int eng_forced = -1;
+    bool autotune = true, use_graphs = true;
+};
+fame_status fame_create_with(const fame_lattice* lat, int max_batch, int device, const fame_settings& set, fame_ctx** out);
+
 void fame_phases(const fame_lattice& L, const double* k, fame::ProbDev* p);
 unsigned fame_magic32(int d);

@@ -296,7 +296,11 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         if (freeb < need) return FAME_OK;
         for (int i = 0; i < G; ++i) {
             fame_ctx* k = nullptr;
-            const fame_status st = fame_create(&c->lat, kid_count(c->nk, G, i), c->device, &k);
+            /* the parent's settings, not today's environment: the tiles copied below
+             * name plans and plane tables that a child has only if it was built as
+             * the parent was                                                    */
+            const fame_settings set = {c->eng_forced, c->autotune, c->use_graphs};
+            const fame_status st = fame_create_with(&c->lat, kid_count(c->nk, G, i), c->device, set, &k);
             if (st != FAME_OK) {
                 for (fame_ctx* q : c->kids) (void)fame_destroy(q);
                 c->kids.clear();
@@ -337,11 +341,6 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         c->kids_k_ver = c->k_ver;
     }
     for (fame_ctx* k : c->kids) {
-        /* the parent's plans: a child built under another FAME_FFT setting may
-         * lack the matrix-core plan that the parent's tiles name */
-        k->eng_forced = c->eng_forced;
-        for (int a = 0; a < 3; ++a)
-            if (c->ax[a][1].n > 0 && k->ax[a][1].n == 0) CHK(k->ax[a][1].build(c->ax[a][1].n, FFT_ENGINE_MFMA));
         bool same = true;
         for (int pi = 0; pi < 2; ++pi)
             for (int a = 0; a < 3; ++a)
@@ -365,7 +364,6 @@ static fame_status sync_kids(fame_ctx* c, int G, int nstep, int nwant, bool* ok)
         k->groups = 1;
         k->gram_batch = c->nk;
         k->out_pmul = G;
-        k->use_graphs = c->use_graphs;
         k->ritz_sweeps = c->ritz_sweeps; k->ritz_tol = c->ritz_tol; k->ritz_maxit = c->ritz_maxit;
         k->refine_max_sweeps = c->refine_max_sweeps; k->refine_reltol = c->refine_reltol;
     }

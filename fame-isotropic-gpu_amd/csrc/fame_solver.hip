@@ -510,7 +510,22 @@ KLine fame_ctx::cg_line(int prec, int p0, bool contract, void* p, void* r, void*
     return k;
 }
 
+/* FAME_FFT=stockham|mfma restricts the line-transform engine (default: both
+ * are planned, the matrix cores are preferred for lengths 16..127 and the
+ * autotuner may change the choice); FAME_AUTOTUNE=0 disables tuning,
+ * FAME_GRAPH=0 the captured graphs */
 extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int device, fame_ctx** out) {
+    fame_settings s;
+    if (const char* e = std::getenv("FAME_FFT")) {
+        if (!std::strcmp(e, "stockham")) s.eng_forced = 0;
+        else if (!std::strcmp(e, "mfma")) s.eng_forced = 1;
+    }
+    if (const char* e = std::getenv("FAME_AUTOTUNE")) s.autotune = std::strcmp(e, "0") != 0;
+    if (const char* e = std::getenv("FAME_GRAPH")) s.use_graphs = std::strcmp(e, "0") != 0;
+    return fame_create_with(lat, max_batch, device, s, out);
+}
+
+fame_status fame_create_with(const fame_lattice* lat, int max_batch, int device, const fame_settings& set, fame_ctx** out) {
     if (!lat || !out || max_batch < 1) FAIL(FAME_ERR_ARG, "fame_create: null argument or max_batch < 1");
     for (int i = 0; i < 3; ++i) if (lat->grid_nums[i] < 1 || lat->grid_nums[i] > 1024) FAIL(FAME_ERR_ARG, "grid_nums out of range");
     int ndev = 0;
@@ -538,15 +553,7 @@ extern "C" fame_status fame_create(const fame_lattice* lat, int max_batch, int d
     g.m_nb = fame_magic32(g.nb);
     c->N = g.N;
     fame_status st;
-    /* FAME_FFT=stockham|mfma restricts the line-transform engine (default: both
-     * are planned, the matrix cores are preferred for lengths 16..127 and the
-     * autotuner may change the choice); FAME_AUTOTUNE=0 disables tuning */
-    if (const char* e = std::getenv("FAME_FFT")) {
-        if (!std::strcmp(e, "stockham")) c->eng_forced = 0;
-        else if (!std::strcmp(e, "mfma")) c->eng_forced = 1;
-    }
-    if (const char* e = std::getenv("FAME_AUTOTUNE")) c->autotune = std::strcmp(e, "0") != 0;
-    if (const char* e = std::getenv("FAME_GRAPH")) c->use_graphs = std::strcmp(e, "0") != 0;
+    c->eng_forced = set.eng_forced; c->autotune = set.autotune; c->use_graphs = set.use_graphs;
     const int len[3] = {g.na, g.nb, g.nc};
     for (int a = 0; a < 3; ++a) {
         if ((st = c->ax[a][0].build(len[a], FFT_ENGINE_STOCKHAM)) != FAME_OK) { delete c; return st; }
