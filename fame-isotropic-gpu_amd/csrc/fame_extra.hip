@@ -131,11 +131,18 @@ __global__ void __launch_bounds__(256) k_resid(const double2* F, const double2* 
     }
 }
 
-/* partials of sum eps |E|^2 of the fields of one wave vector (reference layout;
- * field i on blockIdx.y) */
-__global__ void __launch_bounds__(256) k_wnorm(const double2* E, const double* eps, double* partials, size_t n3) {
+/* the bands of a wave vector that one pass of the gradient takes: those whose
+ * coefficient -w lambda is not 0, in band order                              */
+constexpr int GRAD_CHUNK = 16;
+struct GradBands { double c[GRAD_CHUNK]; int b[GRAD_CHUNK]; };
+
+/* partials of sum eps |E|^2 of those bands' fields (reference layout; entry
+ * blockIdx.y of the list).  A field without weight is not read: a band-edge
+ * objective weighs one or two bands of many (one of 16, SC 128: 88 us, with
+ * every band's norm taken 652)                                               */
+__global__ void __launch_bounds__(256) k_wnorm(const double2* E, GradBands bands, const double* eps, double* partials, size_t n3) {
     double a = 0;
-    E += (size_t)blockIdx.y * n3;
+    E += (size_t)bands.b[blockIdx.y] * n3;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n3; i += (size_t)gridDim.x * 256) {
         double2 e = E[i];
         a += eps[i] * (e.x * e.x + e.y * e.y);
@@ -150,21 +157,18 @@ __global__ void __launch_bounds__(256) k_wnorm(const double2* E, const double* e
     if (threadIdx.x == 0) partials[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = ra[0];
 }
 
-constexpr int GRAD_CHUNK = 16;
-struct GradCoef { double c[GRAD_CHUNK]; };
-
-/* g (+)= sum_i c_i / s_i |E_i|^2 over the fields of one chunk of a wave vector's
- * bands whose c is not 0, in band order, the gradient held in a register: one pass
- * instead of one read-modify-write of g, and one launch, per field              */
-__global__ void __launch_bounds__(256) k_grad_acc(double* g, const double2* E, GradCoef coef, const double* s, int nf, size_t n3,
+/* g (+)= sum_i c_i / s_i |E_i|^2 over the listed bands, in band order, the gradient
+ * held in a register: one pass instead of one read-modify-write of g, and one
+ * launch, per field                                                          */
+__global__ void __launch_bounds__(256) k_grad_acc(double* g, const double2* E, GradBands bands, const double* s, int nf, size_t n3,
                                                   int first) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n3; i += (size_t)gridDim.x * 256) {
         double a = first ? 0.0 : g[i];
 #pragma unroll
         for (int f = 0; f < GRAD_CHUNK; ++f) {
-            if (f >= nf || coef.c[f] == 0.0) continue;
-            const double2 e = E[(size_t)f * n3 + i];
-            a += coef.c[f] / s[f] * (e.x * e.x + e.y * e.y);
+            if (f >= nf) continue;
+            const double2 e = E[(size_t)bands.b[f] * n3 + i];
+            a += bands.c[f] / s[f] * (e.x * e.x + e.y * e.y);
         }
         g[i] = a;
     }
@@ -474,7 +478,7 @@ extern "C" fame_status fame_eig_grad(fame_ctx* c, int nwant, const double* freq,
      * band: with the restoration before it, SC 64, 4 wave vectors x 6 bands,
      * 2.49 -> 0.75 ms                                                          */
     const int chunk = (int)std::min<size_t>(GRAD_CHUNK, std::max<size_t>(1, ((size_t)192 << 20) / (16 * N3)));
-    if (nk < 1) HIPCHK(hipMemsetAsync(grad_dev, 0, sizeof(double) * N3, c->stream));
+    bool first = true;
     for (int p = 0; p < nk; ++p) {
         const double* f = freq + (size_t)p * nwant;
         /* degenerate clusters: mean weight over bands whose lambda agree to 1e-8 relative */
@@ -489,19 +493,26 @@ extern "C" fame_status fame_eig_grad(fame_ctx* c, int nwant, const double* freq,
             for (int q = i; q < j; ++q) w[q] = m;
             i = j;
         }
-        for (int i0 = 0; i0 < nwant; i0 += chunk) {
-            const int n = std::min(chunk, nwant - i0);
-            GradCoef co = {};
-            for (int i = 0; i < n; ++i) co.c[i] = -w[i0 + i] * (f[i0 + i] * f[i0 + i]);
-            const double2* E = (const double2*)E_dev + ((size_t)p * nwant + i0) * N3;
-            hipLaunchKernelGGL(k_wnorm, dim3(NB, n), dim3(256), 0, c->stream, E, c->eps_ref, c->partials, N3);
+        const double2* E = (const double2*)E_dev + (size_t)p * nwant * N3;
+        for (int i = 0; i < nwant;) {
+            GradBands bd = {};
+            int n = 0;
+            for (; i < nwant && n < chunk; ++i) {
+                const double ci = -w[i] * (f[i] * f[i]);
+                if (ci == 0.0) continue;
+                bd.c[n] = ci;
+                bd.b[n++] = i;
+            }
+            if (n == 0) break;
+            hipLaunchKernelGGL(k_wnorm, dim3(NB, n), dim3(256), 0, c->stream, E, bd, c->eps_ref, c->partials, N3);
             HIPCHK(hipGetLastError());
             HIPCHK(fame_reduce_partials(c->partials, NB, 1, c->scal, n, c->stream));
-            hipLaunchKernelGGL(k_grad_acc, dim3(1024), dim3(256), 0, c->stream, (double*)grad_dev, E, co, c->scal, n, N3,
-                               p == 0 && i0 == 0 ? 1 : 0);
+            hipLaunchKernelGGL(k_grad_acc, dim3(1024), dim3(256), 0, c->stream, (double*)grad_dev, E, bd, c->scal, n, N3, first ? 1 : 0);
             HIPCHK(hipGetLastError());
+            first = false;
         }
     }
+    if (first) HIPCHK(hipMemsetAsync(grad_dev, 0, sizeof(double) * N3, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return FAME_OK;
 }
