@@ -1,0 +1,42 @@
+"""What fame_autotune chooses, against the alternatives timed at length."""
+import numpy as np
+import pytest
+
+import fame_amd as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(fl, nk, max_batch=None):
+    rng = np.random.default_rng(nk)
+    S = F.Solver(fl, max_batch=max_batch or nk)
+    S.set_eps(1.0 + 11.0 * rng.random(3 * S.N))
+    S.set_wave_vectors(rng.uniform(0.08, 0.42, (nk, 3)))
+    return S
+
+
+def test_fp64_path_of_a_large_batch(gpu):
+    """FCC 96 x 30 wave vectors, FP64: axis passes take 2.64 ms per CG iteration and the
+    planes 2.82; whichever the tuner takes must be within half of that difference of
+    the better one, every time it is asked, first of all on a new context."""
+    fl = F.to_fame_lattice(F.build_lattice("face_centered_cubic", 96))
+    chosen = []
+    for i in range(6):
+        S = _context(fl, 30)
+        chosen.append(S.autotune(8))
+        if i < 5:
+            S.close()
+    t = {}
+
+    def time(tiles):
+        key = str(tiles)
+        if key not in t:
+            S.set_tiles(8, tiles)
+            S.time_cg_passes(8, 5)
+            t[key] = min(float(S.time_cg_passes(8, 10)[7]) for _ in range(2))
+        return t[key]
+    best = min(time({"inner": (0, 6), "mid": (1, 16), "outer": (0, 16)}),
+               time({"inner": (0, 8), "mid": (2, 12), "outer": (3, 512)}))
+    for tiles in chosen:
+        assert time(tiles) < 1.035 * best, (tiles, t)
+    S.close()
