@@ -1125,6 +1125,10 @@ fame_status fame_ctx::tune(int prec) {
         axis_ms += best_ms;
     }
     if (axis_too && plane_ok[pi] && st == FAME_OK) {
+        /* before the first fame_set_eps: any positive constant, on which the
+         * iterations below do not stop                                         */
+        if (!have_eps && (hipMemsetAsync(eps_ref, 0x3c, sizeof(double) * 3 * (size_t)N, stream) != hipSuccess || spread_eps() != FAME_OK))
+            st = FAME_ERR_HIP;
         /* whole iterations against each other: the axis passes' inner kernels in
          * their CG forms too (tuned alone they look cheaper than they are: four
          * BCC 128 problems ran 532 us of axis passes for 455 of planes).  The first

