@@ -245,7 +245,10 @@ fame_status fame_autotune(fame_ctx* ctx, int prec, int* choice);
 /* Set the pass tiles of precision prec explicitly, in the format of
  * fame_autotune's choice (e.g. to reproduce a tuned configuration); marks the
  * precision as tuned.  FAME_ERR_ARG when an engine or line count is not
- * available for this grid.  No reference counterpart.                       */
+ * available for this grid.  A choice with engine 2 says nothing of the axis
+ * passes, by which Pr, Prs and fame_check_eigendecomp run on every grid: they
+ * keep the tiles they had (fame_autotune's, an earlier choice's, or the start
+ * values).  No reference counterpart.                                        */
 fame_status fame_set_tiles(fame_ctx* ctx, int prec, const int* choice);
 
 /* Stream used by all launches (a hipStream_t passed as void*; NULL = default). */

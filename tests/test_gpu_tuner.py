@@ -52,3 +52,32 @@ def test_path_chosen_before_the_permittivity(gpu):
         for _ in range(2):
             assert (S.autotune(8)["mid"][0] == 2) == planes, nk
         S.close()
+
+
+@pytest.mark.parametrize("lt,nx,tiles", [("simple_cubic", 64, {"inner": (0, 4), "mid": (0, 16), "outer": (0, 16)}),
+                                         ("body_centered_cubic", 48, {"inner": (0, 6), "mid": (0, 16), "outer": (0, 8)})])
+def test_operators_of_the_axis_passes_are_tuned(gpu, lt, nx, tiles):
+    """Pr and Prs run by axis passes on every grid: after fame_autotune they take no
+    longer than with fixed tiles that fit them (the start tiles take 20 to 35% longer)."""
+    import time
+    import torch
+    S = _context(F.to_fame_lattice(F.build_lattice(lt, nx)), 1)
+    x = torch.randn(2 * S.N, dtype=torch.complex128, device="cuda")
+    v = torch.randn(3 * S.N, dtype=torch.complex128, device="cuda")
+
+    def best():
+        t = []
+        for _ in range(40):
+            torch.cuda.synchronize()
+            a = time.perf_counter()
+            S.apply(F.OP_PR, 0, x)
+            S.apply(F.OP_PRS, 0, v)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - a)
+        return min(t)
+    S.autotune(8)
+    best()
+    tuned = best()
+    S.set_tiles(8, tiles)
+    assert tuned < 1.1 * best(), (tuned, best())
+    S.close()
