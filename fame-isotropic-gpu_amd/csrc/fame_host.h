@@ -49,6 +49,7 @@ struct fame_ctx {
     int nblk_in[2] = {0, 0};      /* blocks of the inner-axis kernels per problem */
     int eng_forced = -1;          /* FAME_FFT: -1 auto, else the only engine allowed */
     bool tuned[2] = {false, false};
+    bool axis_set = false;        /* the FP64 axis tiles are tuned or fixed, no start values */
     bool autotune = true;
     /* permittivity, kernel layout */
     double* invB64 = nullptr; float* invB32 = nullptr; double* eps_int = nullptr; double* eps_ref = nullptr;
@@ -145,6 +146,7 @@ struct fame_ctx {
     hipError_t launch_line(const KLine& k, int expand, int mode, int prec, int nprob);
     hipError_t launch_plane(const KPlane& k, int prec, int nprob);
     KSyn ksyn(int p0) const;
+    bool one_way_planes(bool analysis) const;
     /* eps_ref (device) into the kernels' layouts */
     fame_status spread_eps();
     int inner_blocks(int prec) const;

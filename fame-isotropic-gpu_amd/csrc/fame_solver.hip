@@ -487,6 +487,18 @@ KSyn fame_ctx::ksyn(int p0) const {
     a.ostride = 3 * (size_t)N;
     return a;
 }
+/* Qr (or Qrs: analysis) of one problem by planes or by axis passes.  A plane that
+ * fills its CU takes about the same time however few there are, the axis passes'
+ * time grows with the grid, so flat grids are left to them once their tiles fit
+ * (with the start tiles the planes win from 4 on).  Planes / tuned axis passes, us:
+ *   Simple  96x96: Qr 57/42 with 4 planes per component, 63/56 with 16, 70/64 with 24,
+ *           73/72 with 32; Qrs 50/42, 57/54, 63/61, 66/70; 84x84, 24: 59/59, 53/56
+ *   General 96x96: Qr 52/44 with 4, 54/47 with 8, 56/57 with 16; Qrs 44/42, 45/44, 48/54 */
+bool fame_ctx::one_way_planes(bool analysis) const {
+    if (!plane_ok[0]) return false;
+    if (!axis_set || fame_plane_lds(g.nb, g.nc, kpl[0].b.ntab + kpl[0].c.ntab, 8) <= FAME_LDS_HALF) return true;
+    return g.na > (g.general ? (analysis ? 6 : 10) : (analysis ? 20 : 24));
+}
 int fame_ctx::inner_blocks(int prec) const {
     const int pi = prec == 8 ? 0 : 1;
     return plane[pi] ? (g.nb * g.nc + ctile[pi].L - 1) / ctile[pi].L : nblk_in[pi];
@@ -904,7 +916,7 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
     auto unpack = [&]() { return same ? hipSuccess : fame_launch_pack(yout, y, N, Nd, -1, 8, c->stream); };
     switch (op) {
         case FAME_OP_QR:
-            if (c->plane_ok[0]) {
+            if (c->one_way_planes(false)) {
                 /* vector and field straight in the reference's layouts; a Simple
                  * grid's field needs the transpose                           */
                 KLine k = c->kline(8, ik, nullptr);
@@ -925,7 +937,7 @@ extern "C" fame_status fame_apply(fame_ctx* c, int op, int ik, const void* x, vo
             CHK(c->field_to_ref(c->F64 + (size_t)ik * 3 * N, y, 1, 3 * (size_t)N));
             break;
         case FAME_OP_QRS:
-            if (c->plane_ok[0]) {
+            if (c->one_way_planes(true)) {
                 KLine k = c->kline(8, ik, nullptr, true);
                 KSyn s = c->ksyn(ik);
                 if (c->g.general) s.in = (const double2*)x;
@@ -1171,6 +1183,7 @@ fame_status fame_ctx::tune(int prec) {
     if (st != FAME_OK) FAIL(st, std::string("autotune: HIP error: ") + hipGetErrorString(hipGetLastError()));
     nblk_in[pi] = (g.nb * g.nc + tile[AX_INNER][pi].L - 1) / tile[AX_INNER][pi].L;
     tuned[pi] = true;
+    if (prec == 8) axis_set = true;
     drop_graphs();            /* captured launches carry the old tiles */
     return FAME_OK;
 }
@@ -1204,6 +1217,7 @@ extern "C" fame_status fame_set_tiles(fame_ctx* c, int prec, const int* choice) 
         PassTile& t = c->tile[a][pi];
         t.eng = choice[2 * a]; t.L = choice[2 * a + 1]; t.P = c->ax[a][t.eng].M | 1;
     }
+    if (prec == 8) c->axis_set = true;
     c->plane[pi] = false;
     c->nblk_in[pi] = (c->g.nb * c->g.nc + c->tile[AX_INNER][pi].L - 1) / c->tile[AX_INNER][pi].L;
     c->tuned[pi] = true;

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import fame_amd as F
+import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -80,4 +81,49 @@ def test_operators_of_the_axis_passes_are_tuned(gpu, lt, nx, tiles):
     tuned = best()
     S.set_tiles(8, tiles)
     assert tuned < 1.1 * best(), (tuned, best())
+    S.close()
+
+
+def _flat(lt, n):
+    fl = F.to_fame_lattice(F.build_lattice(lt, 16))
+    for i in range(3):
+        fl.mesh_len[i] *= fl.grid_nums[i] / n[i]
+        fl.grid_nums[i] = n[i]
+    fl.m1 = fl.m2 = fl.m3 = fl.m4 = 0
+    return fl
+
+
+@pytest.mark.parametrize("lt,n", [("simple_cubic", (4, 96, 96)), ("simple_cubic", (16, 96, 96)), ("face_centered_cubic", (96, 96, 4))])
+def test_flat_grids_by_the_faster_operators(gpu, lt, n):
+    """A few planes that fill their CUs take longer than tuned axis passes: Qr (5 kernels
+    with a layout change, as Pr) no longer than Pr, which runs by axis passes on every
+    grid (planes: 20 to 35% longer).  The same values with start tiles and tuned."""
+    import time
+    import torch
+    fl = _flat(lt, n)
+    S = _context(fl, 1)
+    T = O.Tables(O.lattice_from(fl), S.k[0])
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    r = lambda m: torch.randn(m, dtype=torch.complex128, device="cuda", generator=gen)
+    x, v = r(2 * S.N), r(3 * S.N)
+    qr, qrs = T.qr(x.cpu().numpy()), T.qrs(v.cpu().numpy())
+
+    def check():
+        for got, ref in ((S.apply(F.OP_QR, 0, x), qr), (S.apply(F.OP_QRS, 0, v), qrs)):
+            assert np.abs(got.cpu().numpy() - ref).max() < 1e-11 * np.abs(ref).max()
+
+    def best(op):
+        t = []
+        for _ in range(40):
+            torch.cuda.synchronize()
+            a = time.perf_counter()
+            S.apply(op, 0, x)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - a)
+        return min(t)
+    check()
+    S.autotune(8)
+    check()
+    best(F.OP_PR)
+    assert best(F.OP_QR) < 1.08 * best(F.OP_PR)
     S.close()
