@@ -140,6 +140,7 @@ struct fame_ctx {
     fame_status cg_step_rc(int prec, void* p, void* r, void* x, int p0, int nprob, int npap);
 
     bool line_tile_ok(int prec, int eng, int L) const;
+    int start_threads(int pi) const;
     fame_status plane_setup();
     KLine kline(int prec, int p0, const int* act, bool contract = false) const;
     KPlane kplane(int prec, int p0, const int* act) const;

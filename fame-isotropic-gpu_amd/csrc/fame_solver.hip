@@ -366,6 +366,18 @@ static bool plane_axis(const AxisPlan& p, int eng, int pi, int nl, PlaneAxis* q,
     return true;
 }
 
+/* threads per block of the plane kernel before tuning.  The wide variant's 256
+ * registers leave a CU 512 threads, in two blocks of 256 where two planes fit and
+ * the wave vectors in use bring that many, else in one (60^3, one wave vector:
+ * QBQ 69 us with 512 threads, 73 with 256)                                   */
+int fame_ctx::start_threads(int pi) const {
+    const KPlane& k = kpl[pi];
+    const size_t lds = fame_plane_lds(g.nb, g.nc, k.b.ntab + k.c.ntab, pi == 0 ? 8 : 4);
+    if (lds > FAME_LDS_HALF) return pi == 0 ? 512 : 1024;
+    if (k.wide) return 3 * g.na * nk > 512 ? 256 : 512;
+    return lds > 24 * 1024 ? 512 : 256;
+}
+
 /* whether the grid has the plane path, per precision: no Bluestein axis (a
  * length with a prime factor above 13 takes the direct DFT), and a plane
  * within the LDS of a CU */
@@ -400,11 +412,9 @@ fame_status fame_ctx::plane_setup() {
          * plane fills the CU alone anyway, or the compound radices save a pass
          * (48^3: 21.6 -> 18.5 us, eight 72.2 -> 63.9; FCC 96: 54 -> 50, four 227
          * -> 188).  At equal passes the narrow one's 4 waves per SIMD are better
-         * (16 x 64^3: 170 against 193).  Many blocks: two of 256 threads per CU
-         * instead of one of 512                                               */
+         * (16 x 64^3: 170 against 193)                                        */
         k.wide = prec == 8 && (lds > FAME_LDS_HALF || wide_ax[0].nst + wide_ax[1].nst < k.b.nst + k.c.nst);
-        k.nt = lds > FAME_LDS_HALF ? (prec == 8 ? 512 : 1024) : lds > 24 * 1024 ? 512 : 256;
-        if (k.wide && lds <= FAME_LDS_HALF) k.nt = 3 * g.na * maxb > 512 ? 256 : 512;
+        k.nt = start_threads(pi);
         bool any = false;
         for (int e = 0; e < 2; ++e) {
             if (eng_forced >= 0 && e != eng_forced && !(eng_forced == 0 && ax[AX_INNER][0].blue)) { laxis[pi][e].n = 0; continue; }
@@ -735,6 +745,12 @@ extern "C" fame_status fame_set_wave_vectors(fame_ctx* c, int nk, const double* 
     if (nk > c->maxb) FAIL(FAME_ERR_ARG, "fame_set_wave_vectors: more wave vectors than max_batch");
     HIPCHK(hipSetDevice(c->device));
     c->nk = nk;
+    for (int pi = 0; pi < 2; ++pi) {
+        if (!c->plane_ok[pi] || c->tuned[pi]) continue;
+        const int nt = c->start_threads(pi);
+        if (nt != c->kpl[pi].nt) c->drop_graphs();     /* captured launches carry the old count */
+        c->kpl[pi].nt = nt;
+    }
     c->kvec.assign(k, k + 3 * (size_t)nk);
     c->prob_h.resize(nk);
     c->nd.resize(nk);

@@ -127,3 +127,19 @@ def test_flat_grids_by_the_faster_operators(gpu, lt, n):
     best(F.OP_PR)
     assert best(F.OP_QR) < 1.08 * best(F.OP_PR)
     S.close()
+
+
+@pytest.mark.parametrize("nx", [48, 60])
+def test_start_values_follow_the_wave_vectors_in_use(gpu, nx):
+    """One wave vector in a context made for 30 runs its FP64 plane kernel as in a
+    context made for one (with the launch that 30 take: 10 to 15% longer), also when
+    30 were set before."""
+    fl = F.to_fame_lattice(F.build_lattice("simple_cubic", nx))
+    us = {}
+    for max_batch in (1, 30):
+        S = _context(fl, max_batch)
+        S.set_wave_vectors(np.array([[0.21, -0.13, 0.07]]))
+        S.time_qbq_passes(8, 50)
+        us[max_batch] = min(float(S.time_qbq_passes(8, 50)[2]) for _ in range(5))
+        S.close()
+    assert us[30] < 1.05 * us[1], us
