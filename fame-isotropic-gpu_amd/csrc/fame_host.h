@@ -29,11 +29,12 @@ struct AxisPlan {
     std::vector<int> radices;
     fame::LinePlanDev lists[2][NLIST];   /* [0] FP64, [1] FP32; LIST_* stage lists */
     int cap[2] = {0, 0};                 /* elements a 256-thread block transforms at once */
-    std::vector<void*> bufs;
     const PlaneStage* pst[2] = {nullptr, nullptr};  /* passes of the plane kernels: nst, then nst reversed */
     const void* afrag[2] = {nullptr, nullptr};   /* direct DFT: A operand fragments of the plane kernels */
-    fame_status build(int n, int engine);
-    ~AxisPlan();
+    /* build appends the plan's tables to `tables` and leaves their places there
+     * (offset + 1) in the pointers; rebase makes them addresses in the device copy */
+    fame_status build(int n, int engine, std::vector<char>& tables);
+    void rebase(const char* device);
 };
 
 struct fame_ctx {

@@ -26,6 +26,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 using namespace fame;
@@ -93,8 +94,13 @@ unsigned fame_magic32(int d) {
 
 typedef std::complex<long double> cld;
 
-AxisPlan::~AxisPlan() {
-    for (void* p : bufs) if (p) (void)hipFree(p);
+void AxisPlan::rebase(const char* device) {
+    auto at = [&](auto& p) { if (p) p = (std::remove_reference_t<decltype(p)>)(device + ((uintptr_t)p - 1)); };
+    for (int pi = 0; pi < 2; ++pi) {
+        for (LinePlanDev& d : lists[pi]) { at(d.W); at(d.chirp); at(d.bm); at(d.bp); }
+        at(afrag[pi]);
+        at(pst[pi]);
+    }
 }
 
 /* append one transform of sign `sign` to a stage list */
@@ -134,7 +140,7 @@ static bool add_mid(LinePlanDev& d) {
     return true;
 }
 
-fame_status AxisPlan::build(int n_, int engine) {
+fame_status AxisPlan::build(int n_, int engine, std::vector<char>& tables) {
     n = n_;
     /* lengths 16..127: direct DFT on the matrix cores (any n, no Bluestein);
      * otherwise Stockham passes, or Bluestein when n has a prime factor > 13
@@ -181,23 +187,24 @@ fame_status AxisPlan::build(int n_, int engine) {
             bm[k] = s1; bp[k] = s2;
         }
     }
-    auto upload = [&](const std::vector<cld>& v, int prec, const void** dst) -> fame_status {
-        if (v.empty()) { *dst = nullptr; return FAME_OK; }
-        void* d = nullptr;
-        size_t bytes = v.size() * (prec == 8 ? 16 : 8);
-        HIPCHK(hipMalloc(&d, bytes));
-        bufs.push_back(d);
+    auto add = [&](const void* data, size_t bytes) -> uintptr_t {
+        const size_t o = (tables.size() + 255) & ~(size_t)255;
+        tables.resize(o + bytes);
+        std::memcpy(tables.data() + o, data, bytes);
+        return (uintptr_t)o + 1;
+    };
+    auto upload = [&](const std::vector<cld>& v, int prec, const void** dst) {
+        *dst = nullptr;
+        if (v.empty()) return;
         if (prec == 8) {
             std::vector<double> h(2 * v.size());
             for (size_t i = 0; i < v.size(); ++i) { h[2 * i] = (double)v[i].real(); h[2 * i + 1] = (double)v[i].imag(); }
-            HIPCHK(hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice));
+            *dst = (const void*)add(h.data(), 8 * h.size());
         } else {
             std::vector<float> h(2 * v.size());
             for (size_t i = 0; i < v.size(); ++i) { h[2 * i] = (float)v[i].real(); h[2 * i + 1] = (float)v[i].imag(); }
-            HIPCHK(hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice));
+            *dst = (const void*)add(h.data(), 4 * h.size());
         }
-        *dst = d;
-        return FAME_OK;
     };
     /* FP64 lists: the same length M factored without the compound radices */
     std::vector<int> rad64 = radices;
@@ -212,10 +219,10 @@ fame_status AxisPlan::build(int n_, int engine) {
         base.n = n; base.M = M; base.blue = blue;
         base.ntab = blue ? 4 * M : M;
         base.mM = fame_magic32(M); base.mN = fame_magic32(n);
-        CHK(upload(W, prec, &base.W));
-        CHK(upload(ch, prec, &base.chirp));
-        CHK(upload(bm, prec, &base.bm));
-        CHK(upload(bp, prec, &base.bp));
+        upload(W, prec, &base.W);
+        upload(ch, prec, &base.chirp);
+        upload(bm, prec, &base.bm);
+        upload(bp, prec, &base.bp);
         if (mfma) {
             /* lane l of K step ks, tile w: row q = 16 w + l % 16, t = 4 ks + l / 16 + 1 */
             const int m = (n - 1) / 2, Q = n / 2 + 1, nqt = (Q + 15) / 16, nks = std::max(1, (m + 3) / 4);
@@ -226,7 +233,7 @@ fame_status AxisPlan::build(int n_, int engine) {
                         const int q = 16 * w + l % 16, t = 4 * ks + l / 16 + 1;
                         if (q < Q && t <= m) af[((size_t)w * nks + ks) * 64 + l] = W[(size_t)q * t % n];
                     }
-            CHK(upload(af, prec, &afrag[pi]));
+            upload(af, prec, &afrag[pi]);
         }
         if (!mfma && !blue) {
             std::vector<PlaneStage> ps(2 * rads.size());
@@ -242,11 +249,7 @@ fame_status AxisPlan::build(int n_, int engine) {
                 fill(ps[i], Ri, Ns); Ns *= Ri;
                 fill(ps[rads.size() + i], rads[i], Nf); Nf *= rads[i];
             }
-            void* d = nullptr;
-            HIPCHK(hipMalloc(&d, sizeof(PlaneStage) * std::max<size_t>(ps.size(), 1)));
-            bufs.push_back(d);
-            HIPCHK(hipMemcpy(d, ps.data(), sizeof(PlaneStage) * ps.size(), hipMemcpyHostToDevice));
-            pst[pi] = (const PlaneStage*)d;
+            if (!ps.empty()) pst[pi] = (const PlaneStage*)add(ps.data(), sizeof(PlaneStage) * ps.size());
         }
         bool ok = true;
         for (int l = 0; l < NLIST && mfma; ++l) {
@@ -429,11 +432,13 @@ fame_status fame_ctx::plane_setup() {
         if (!line_tile_ok(prec, eng, L)) { plane_ok[pi] = false; continue; }
         ltile[pi].eng = eng; ltile[pi].L = L; ltile[pi].P = g.na | 1;
         ctile[pi] = ltile[pi];
-        if (prec == 8) {
-            syn_wide = k.wide;
-            HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+        if (prec == 8) syn_wide = k.wide;
+        /* leave to use more than 64 KiB of LDS (with the kernels' static LDS), which
+         * costs the host 10 us per kernel, only where a plane needs it          */
+        if (lds > 63 * 1024) {
+            if (prec == 8) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
+            HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng) : fame_prepare_plane32(k.b.eng, k.c.eng));
         }
-        HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng) : fame_prepare_plane32(k.b.eng, k.c.eng));
         /* before tuning: an FP64 plane that fills a CU alone pays where one
          * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
          * iteration in 112 us against 134 by axis passes; SC 96, 288 blocks: 193
@@ -577,10 +582,23 @@ fame_status fame_create_with(const fame_lattice* lat, int max_batch, int device,
     fame_status st;
     c->eng_forced = set.eng_forced; c->autotune = set.autotune; c->use_graphs = set.use_graphs;
     const int len[3] = {g.na, g.nb, g.nc};
+    /* the tables of all plans in one allocation and one copy (a context on a 16^3
+     * grid: 504 us with 24 of each and the LDS attributes that no kernel of its
+     * size needs, 159 without)                                                */
+    std::vector<char> tables;
     for (int a = 0; a < 3; ++a) {
-        if ((st = c->ax[a][0].build(len[a], FFT_ENGINE_STOCKHAM)) != FAME_OK) { delete c; return st; }
+        if ((st = c->ax[a][0].build(len[a], FFT_ENGINE_STOCKHAM, tables)) != FAME_OK) { delete c; return st; }
         if (c->eng_forced != 0 && len[a] >= 2 && len[a] <= 127 &&
-            (st = c->ax[a][1].build(len[a], FFT_ENGINE_MFMA)) != FAME_OK) { delete c; return st; }
+            (st = c->ax[a][1].build(len[a], FFT_ENGINE_MFMA, tables)) != FAME_OK) { delete c; return st; }
+    }
+    {
+        void* d = nullptr;
+        if ((st = dalloc(c, &d, tables.size())) != FAME_OK) { delete c; return st; }
+        if (hipMemcpy(d, tables.data(), tables.size(), hipMemcpyHostToDevice) != hipSuccess) {
+            delete c;
+            FAIL(FAME_ERR_HIP, "fame_create: copy of the transform tables failed");
+        }
+        for (auto& x : c->ax) for (AxisPlan& q : x) q.rebase((const char*)d);
     }
     for (int pi = 0; pi < 2; ++pi) {
         const int prec = pi == 0 ? 8 : 4;
