@@ -1130,22 +1130,25 @@ fame_status fame_ctx::tune(int prec) {
     const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF;
     plane[pi] = plane_ok[pi];
     /* Pr, Prs and the check of the factorisation run by FP64 axis passes on every
-     * grid, one problem at a time (Pr on SC 64: 83 us with the start tiles, 66 tuned) */
-    const int nt_prob = axis_too ? nk : 1;
+     * grid, one problem at a time (Pr on SC 64: 83 us with the start tiles, 60
+     * tuned).  Where nothing else does, only tiles that leave one problem many blocks
+     * are tried, twice each (32^3: 0.9 ms of tuning instead of 3.2)             */
+    const int nt_prob = axis_too ? nk : 1, reps = axis_too ? 3 : 2;
+    static const int candL_few[] = {2, 4, 6, 8, 16};
     for (int a = 0; a < 3 && st == FAME_OK && (axis_too || prec == 8); ++a) {
         PassTile best = tile[a][pi];
         float best_ms = 1e30f;
         for (int eng = 0; eng < 2; ++eng) {
             if (ax[a][eng].n == 0 || (eng_forced >= 0 && eng != eng_forced)) continue;
-            const int* cl = a == AX_INNER ? candL_inner : candL_axis;
-            const int ncl = a == AX_INNER ? 10 : 7;
+            const int* cl = axis_too ? (a == AX_INNER ? candL_inner : candL_axis) : candL_few + (a == AX_INNER ? 0 : 1);
+            const int ncl = axis_too ? (a == AX_INNER ? 10 : 7) : 4;
             for (int ci = 0; ci < ncl; ++ci) {
                 const int L = cl[ci];
                 if (!tile_ok(ax[a][eng], a, prec, L, g)) continue;
                 const PassTile save = tile[a][pi];
                 tile[a][pi].eng = eng; tile[a][pi].L = L; tile[a][pi].P = ax[a][eng].M | 1;
                 float ms = 0;
-                for (int rep = -1; rep < 3; ++rep) {
+                for (int rep = -1; rep < reps; ++rep) {
                     if (rep == 0 && hipEventRecord(e0, stream) != hipSuccess) { st = FAME_ERR_HIP; break; }
                     hipError_t e = hipSuccess;
                     if (a == AX_INNER) {
