@@ -7,6 +7,7 @@
 #include <vector>
 #include <hip/hip_runtime.h>
 #include "fame_hip.h"
+#include "fame_guess.h"
 #include "fame_kernels.h"
 
 /* contraction and expansion modes of the plane path (fame_plane.hpp) */
@@ -98,8 +99,7 @@ struct fame_ctx {
     std::vector<size_t> big_bytes;  /* their sizes (the shape they were allocated for) */
     /* tuning / state */
     /* iterations the next solve is expected to take, per precision and refinement sweep */
-    int cg_predict[2][4] = {{24}, {24}};   /* 0: not known, the sweep before's count */
-    int cg_last[2][4] = {};
+    CgGuess cg_guess[2][4];
     /* inverse-iteration sweeps applied by fame_eigs to the converged Ritz pairs
      * (fame_set_refinement; 0 = the reference's algorithm), their absolute CG
      * tolerance and iteration limit */

@@ -1322,11 +1322,12 @@ fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, do
     else HIPCHK(fame_cg_begin(x, r, p, b, partials, NBLK_VEC, n, st, nprob, prec, mask_dev, stream));
     HIPCHK(fame_cg_init_scal2(cgsc, partials, nbp, tol, reltol, maxit, nprob, active, mask_dev, stream));
     int done_it = 0;
-    /* the iterations expected: an iteration too many costs three launches that
-     * return at once (10 us), one too few a round trip to the host (40 us)     */
-    int& predict = cg_predict[pix(prec)][slot];
-    if (predict == 0) predict = cg_last[pix(prec)][slot - 1];
-    int chunk = std::max(1, std::min(maxit, predict));
+    /* the iterations expected; a sweep not seen yet: the sweep before's count */
+    CgGuess::Entry& guess = cg_guess[pix(prec)][slot].at(tol, maxit);
+    int expect = guess.predict;
+    if (expect == 0 && slot > 0) expect = cg_guess[pix(prec)][slot - 1].at(tol, maxit).last;
+    if (expect == 0) expect = 24;
+    int chunk = std::max(1, std::min(maxit, expect));
     while (true) {
         for (int it = 0; it < chunk;) {
             const int left = chunk - it;
@@ -1360,10 +1361,7 @@ fame_status fame_ctx::cg(int prec, const void* b, void* x, int p0, int nprob, do
         applied += sc_h[i].iters - 1;
     }
     if (prec == 8) cnt_qbq64 += applied; else cnt_qbq32 += applied;
-    int& last = cg_last[pix(prec)][slot];
-    const int its = std::max(1, mx - 1);
-    predict = std::max(its, std::min(last, its + 1));      /* counts that go up and down by one: the larger */
-    last = its;
+    CgGuess::took(guess, mx - 1);
     return FAME_OK;
 }
 
