@@ -142,6 +142,8 @@ struct fame_ctx {
 
     bool line_tile_ok(int prec, int eng, int L) const;
     int start_threads(int pi) const;
+    float small_plane_load(int pi) const;
+    bool start_plane(int pi) const;
     fame_status plane_setup();
     KLine kline(int prec, int p0, const int* act, bool contract = false) const;
     KPlane kplane(int prec, int p0, const int* act) const;

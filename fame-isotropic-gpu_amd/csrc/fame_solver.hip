@@ -382,6 +382,31 @@ int fame_ctx::start_threads(int pi) const {
     return lds > 24 * 1024 ? 512 : 256;
 }
 
+/* Small planes, many of them: a block of the plane kernel costs some 12 ns however
+ * small its plane, so a batch of long grids is faster by axis passes.  Iterations
+ * by tuned planes / axis passes, us, FP64 (FP32 alike): 200 x 6 x 6 one problem 38/43,
+ * five 63/47, 64 462/129; 100 x 10 x 10 sixteen 64/61, 64 198/135; 50 x 16 x 16 64
+ * 149/147; from planes of 24 x 24 on the planes win at every batch.
+ * The blocks of the batch in units of what the axis passes match with both tuned: */
+float fame_ctx::small_plane_load(int pi) const {
+    const int p = g.nb * g.nc;
+    if (p > 512) return 0.0f;
+    /* a block of four or more FP64 passes (6 x 6, 5 x 30) takes twice as long   */
+    const int blocks = 3 * g.na * (pi == 0 && kpl[0].b.nst + kpl[0].c.nst >= 4 ? 2 : 1);
+    return (float)blocks * nk / (1500.0f + 25.0f * p);
+}
+/* whether the solver takes the planes before tuning: an FP64 plane that fills a
+ * CU alone pays where one wave vector's blocks are all resident at once (FCC 96,
+ * 234 blocks: an iteration in 112 us against 134 by axis passes; SC 96, 288
+ * blocks: 193 against 180).  The axis passes' start tiles fit long lines better
+ * than short ones (200 x 8 x 8, 16 problems: planes 97 us, axis passes 74; 100 x 10
+ * x 10, 64 problems: 201 and 241; 100 x 8 x 8: 166 and 146)                    */
+bool fame_ctx::start_plane(int pi) const {
+    if (!plane_ok[pi] || small_plane_load(pi) > (g.na >= 128 ? 1.25f : 5.0f)) return false;
+    const KPlane& k = kpl[pi];
+    return pi == 1 || fame_plane_lds(g.nb, g.nc, k.b.ntab + k.c.ntab, 8) <= FAME_LDS_HALF || 3 * g.na <= 256;
+}
+
 /* whether the grid has the plane path, per precision: no Bluestein axis (a
  * length with a prime factor above 13 takes the direct DFT), and a plane
  * within the LDS of a CU */
@@ -440,11 +465,7 @@ fame_status fame_ctx::plane_setup() {
             if (prec == 8) HIPCHK(fame_prepare_syn(k.b.eng, k.c.eng));
             HIPCHK(prec == 8 ? fame_prepare_plane64(k.b.eng, k.c.eng) : fame_prepare_plane32(k.b.eng, k.c.eng));
         }
-        /* before tuning: an FP64 plane that fills a CU alone pays where one
-         * wave vector's blocks are all resident at once (FCC 96, 234 blocks: an
-         * iteration in 112 us against 134 by axis passes; SC 96, 288 blocks: 193
-         * against 180)                                                        */
-        plane[pi] = prec == 4 || lds <= FAME_LDS_HALF || 3 * g.na <= 256;
+        plane[pi] = start_plane(pi);
     }
     return FAME_OK;
 }
@@ -767,8 +788,10 @@ extern "C" fame_status fame_set_wave_vectors(fame_ctx* c, int nk, const double* 
     for (int pi = 0; pi < 2; ++pi) {
         if (!c->plane_ok[pi] || c->tuned[pi]) continue;
         const int nt = c->start_threads(pi);
-        if (nt != c->kpl[pi].nt) c->drop_graphs();     /* captured launches carry the old count */
+        const bool pl = c->start_plane(pi);
+        if (nt != c->kpl[pi].nt || pl != c->plane[pi]) c->drop_graphs();     /* captured launches carry the old ones */
         c->kpl[pi].nt = nt;
+        c->plane[pi] = pl;
     }
     c->kvec.assign(k, k + 3 * (size_t)nk);
     c->prob_h.resize(nk);
@@ -1124,10 +1147,10 @@ fame_status fame_ctx::tune(int prec) {
         plane_ms += best_ms;
     }
     /* a plane that leaves room for two blocks per CU beats the axis passes by 8% to
-     * 30% at every batch measured; one that fills the CU alone may not, so both
-     * are tuned and compared                                                  */
+     * 30% at every batch measured, many small ones apart; one that fills the CU
+     * alone may not, so there both are tuned and compared                     */
     const size_t plds = plane_ok[pi] ? fame_plane_lds(g.nb, g.nc, kpl[pi].b.ntab + kpl[pi].c.ntab, prec) : 0;
-    const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF;
+    const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF || small_plane_load(pi) > 0.25f;
     plane[pi] = plane_ok[pi];
     /* Pr, Prs and the check of the factorisation run by FP64 axis passes on every
      * grid, one problem at a time (Pr on SC 64: 83 us with the start tiles, 60

@@ -143,3 +143,24 @@ def test_start_values_follow_the_wave_vectors_in_use(gpu, nx):
         us[max_batch] = min(float(S.time_qbq_passes(8, 50)[2]) for _ in range(5))
         S.close()
     assert us[30] < 1.05 * us[1], us
+
+
+@pytest.mark.parametrize("n,nk", [((400, 6, 6), 16), ((200, 4, 4), 64), ((100, 10, 10), 64)])
+def test_many_small_planes(gpu, n, nk):
+    """A batch of long grids, whose planes are small and many, takes 1.5 to 3.4 times as
+    long by planes as by axis passes: the tuner's choice is well under the planes, and
+    for the longer ones so are the start values."""
+    S = _context(_flat("simple_cubic", n), nk)
+
+    def time(prec):
+        S.time_cg_passes(prec, 10)
+        return min(float(S.time_cg_passes(prec, 20)[7]) for _ in range(3))
+    for prec in (8, 4):
+        start = time(prec)
+        S.autotune(prec)
+        tuned = time(prec)
+        S.set_tiles(prec, {"inner": (0, 2), "mid": (2, 2), "outer": (2, 256)})
+        planes = time(prec)
+        assert tuned < 0.8 * planes, (prec, start, tuned, planes)
+        assert n[0] < 200 or start < 0.8 * planes, (prec, start, tuned, planes)
+    S.close()
