@@ -223,7 +223,7 @@ static fame_status residuals_chunk(fame_ctx* c, int nwant, const double* freq, c
  * in and compare tile by tile).  One read-back at the end.                   */
 static bool residuals_by_planes(const fame_ctx* c, int nwant) {
     /* two sums per plane in pap_part, 3 numbers per wave vector and band in partials2 */
-    return c->plane_ok[0] && c->nk > 0 && nwant <= 1024 && 2 * c->g.na <= xcd_round(c->g.na * c->g.nb);
+    return c->plane_ok[0] && c->nk > 0 && nwant <= 1024 && !c->long_lines(1000);
 }
 static fame_status residuals_planes(fame_ctx* c, int nwant, const double* freq, const void* E_dev, double* res) {
     const size_t N = c->N, N3 = 3 * N, pn = (size_t)c->g.nb * c->g.nc, es = (size_t)nwant * N3;

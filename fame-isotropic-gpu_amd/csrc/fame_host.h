@@ -151,6 +151,7 @@ struct fame_ctx {
     hipError_t launch_plane(const KPlane& k, int prec, int nprob);
     KSyn ksyn(int p0) const;
     bool one_way_planes(bool analysis) const;
+    bool long_lines(int r) const;
     /* eps_ref (device) into the kernels' layouts */
     fame_status spread_eps();
     int inner_blocks(int prec) const;

@@ -637,11 +637,12 @@ extern "C" fame_status fame_eigs_impl(fame_ctx* c, int precision, const fame_es*
 /* E_i = invB .* Qr(Sigma .* ev_i), times ||E_i|| (reference scaling), for band i
  * of every problem (FAME_Fast_Algorithms_Isotropic.cu:90-125).  ev: padded
  * reduced vectors of band i with per-problem stride ev_pstride.              */
+static bool restore_by_planes(const fame_ctx* c) { return c->plane_ok[0] && !c->long_lines(5000); }
 static fame_status restore_band(fame_ctx* c, int i, int nwant, const double2* ev, size_t ev_pstride, void* E_dev,
                                 bool ref = false) {
     const size_t N = c->N, n2 = 2 * N, N3 = 3 * N;
     const int nk = c->nk;
-    if (c->plane_ok[0]) {
+    if (restore_by_planes(c)) {
         /* four kernels and no host round trip: the expansion scales by Sigma as it
          * reads, the plane kernel applies 1/eps and sums |E|^2, the transpose to the
          * reference's layout applies the norm.  Against the separate passes
@@ -711,7 +712,7 @@ extern "C" fame_status fame_restore(fame_ctx* c, int nwant, const void* evr_dev,
     const size_t n2 = 2 * (size_t)c->N;
     double2* stage = (double2*)c->ref64[2];
     for (int i = 0; i < nwant; ++i) {
-        if (c->plane_ok[0]) {
+        if (restore_by_planes(c)) {
             CHK(restore_band(c, i, nwant, (const double2*)evr_dev + (size_t)i * n2, (size_t)nwant * n2, E_dev, true));
             continue;
         }

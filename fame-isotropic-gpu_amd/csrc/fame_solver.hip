@@ -536,6 +536,15 @@ bool fame_ctx::one_way_planes(bool analysis) const {
     if (!axis_set || fame_plane_lds(g.nb, g.nc, kpl[0].b.ntab + kpl[0].c.ntab, 8) <= FAME_LDS_HALF) return true;
     return g.na > (g.general ? (analysis ? 6 : 10) : (analysis ? 20 : 24));
 }
+/* a batch of long lines with small planes, r the line's square per plane: the
+ * one-way plane kernels of restoration and residuals take some 20 ns per plane, and
+ * behind lines of more than 256 points there are many.  Two bands by planes / axis
+ * passes, us: residuals 400 x 4 x 4 sixteen problems 730/450, 64 2540/1040; 400 x 12 x
+ * 12 sixteen 790/640, four 300/350; 200 x 6 x 6 64 1020/1180; restoration 400 x 4 x 4
+ * sixteen 450/420, 64 1570/1060; 400 x 6 x 6 sixteen 360/450                    */
+bool fame_ctx::long_lines(int r) const {
+    return g.na > 256 && g.na * g.na > r * g.nb * g.nc && 3 * g.na * nk > 12000;
+}
 int fame_ctx::inner_blocks(int prec) const {
     const int pi = prec == 8 ? 0 : 1;
     return plane[pi] ? (g.nb * g.nc + ctile[pi].L - 1) / ctile[pi].L : nblk_in[pi];
@@ -1150,7 +1159,7 @@ fame_status fame_ctx::tune(int prec) {
      * 30% at every batch measured, many small ones apart; one that fills the CU
      * alone may not, so there both are tuned and compared                     */
     const size_t plds = plane_ok[pi] ? fame_plane_lds(g.nb, g.nc, kpl[pi].b.ntab + kpl[pi].c.ntab, prec) : 0;
-    const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF || small_plane_load(pi) > 0.25f;
+    const bool axis_too = !plane_ok[pi] || plds > FAME_LDS_HALF || small_plane_load(pi) > 0.2f;
     plane[pi] = plane_ok[pi];
     /* Pr, Prs and the check of the factorisation run by FP64 axis passes on every
      * grid, one problem at a time (Pr on SC 64: 83 us with the start tiles, 60

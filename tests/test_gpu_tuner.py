@@ -164,3 +164,45 @@ def test_many_small_planes(gpu, n, nk):
         assert tuned < 0.8 * planes, (prec, start, tuned, planes)
         assert n[0] < 200 or start < 0.8 * planes, (prec, start, tuned, planes)
     S.close()
+
+
+def test_fields_and_residuals_of_long_lines(gpu):
+    """A batch of 400 x 4 x 4 grids takes the axis passes, one of its problems the
+    planes: the same fields and residuals to rounding, Gamma among them; and 64 cost
+    less than eight times 8, which is what they cost by planes (2.5 ms against 8 x 0.3)."""
+    import time
+    import torch
+    fl = _flat("simple_cubic", (400, 4, 4))
+    rng = np.random.default_rng(2)
+    nk, nw = 12, 3
+    ks = np.vstack([np.zeros((1, 3)), rng.uniform(0.08, 0.42, (nk - 1, 3))])
+    S = _context(fl, nk)
+    S.set_wave_vectors(ks)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    evr = torch.randn((nk, nw, 2 * S.N), dtype=torch.complex128, device="cuda", generator=gen)
+    freq = np.tile([0.4, 0.5, 0.9], (nk, 1))
+    E = S.restore(evr)
+    res = S.residuals(freq, E)
+    one = _context(fl, nk)          # the same permittivity
+    for p in (0, 1, nk - 1):
+        one.set_wave_vectors(ks[p:p + 1])
+        e = one.restore(evr[p:p + 1])
+        assert float((e - E[p:p + 1]).norm() / e.norm()) < 1e-12
+        r = one.residuals(freq[p:p + 1], E[p:p + 1])
+        assert np.max(np.abs(r - res[p:p + 1]) / r) < 1e-12
+    S.close()
+    one.close()
+
+    def cost(n):
+        S = _context(fl, n)
+        E = torch.randn((n, 2, 3 * S.N), dtype=torch.complex128, device="cuda", generator=gen)
+        f = np.full((n, 2), 0.5)
+        t = []
+        for _ in range(15):
+            torch.cuda.synchronize()
+            a = time.perf_counter()
+            S.residuals(f, E)
+            t.append(time.perf_counter() - a)
+        S.close()
+        return min(t)
+    assert cost(64) < 4.5 * cost(8)
