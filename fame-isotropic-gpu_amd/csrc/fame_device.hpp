@@ -777,6 +777,15 @@ __device__ __forceinline__ double rsq(double x) {
     return rsqrt(x);
 }
 
+/* 3 Lq - |S|^2 as |d|^2, d = (Lz - Ly, Lx - Lz, Ly - Lx): near L parallel to (1, 1, 1)
+ * the difference loses up to 6 digits (FCC 96), by other amounts in every
+ * kernel that sums in another order, and the basis has to be the same in all
+ * of them; the sum of squares is accurate to a few ulp in any order          */
+__device__ __forceinline__ double pi_d2_general(double2 lx, double2 ly, double2 lz) {
+    const double2 d1 = csub(lz, ly), d2 = csub(lx, lz), d3 = csub(ly, lx);
+    return d1.x * d1.x + d1.y * d1.y + d2.x * d2.x + d2.y * d2.y + d3.x * d3.x + d3.y * d3.y;
+}
+
 /* General gauge (FAME_Matrix_Lambdas.cu:441-461) with S = Lx + Ly + Lz:
  *   p1 = (Lq - L_i conj(S)) / sqrt(Lq (3 Lq - |S|^2)),  p2 = conj(Lz - Ly, Lx - Lz, Ly - Lx) / sqrt(3 Lq - |S|^2).
  * Its normalisers vanish (0/0) where L is parallel to (1, 1, 1), and lose
@@ -787,17 +796,9 @@ __device__ __forceinline__ double rsq(double x) {
  * both formed from d without cancellation, and a mode with |d|^2 <= 1e-30 Lq
  * takes the Simple gauge (w = (3, 5, 1)), which is well defined there.  Every
  * kernel evaluates the same form and branch from the same FP64 symbols, so the
- * basis is consistent; other grids keep the reference's arithmetic, whose
- * register footprint matters in the FP32 inner kernels.                     */
-/* 3 Lq - |S|^2 as |d|^2, d = (Lz - Ly, Lx - Lz, Ly - Lx): near L parallel to (1, 1, 1)
- * the difference loses up to 6 digits (FCC 96), by other amounts in every
- * kernel that sums in another order, and the basis has to be the same in all
- * of them; the sum of squares is accurate to a few ulp in any order          */
-__device__ __forceinline__ double pi_d2_general(double2 lx, double2 ly, double2 lz) {
-    const double2 d1 = csub(lz, ly), d2 = csub(lx, lz), d3 = csub(ly, lx);
-    return d1.x * d1.x + d1.y * d1.y + d2.x * d2.x + d2.y * d2.y + d3.x * d3.x + d3.y * d3.y;
-}
-
+ * basis is consistent; other grids keep the reference's numerators, whose
+ * register footprint matters in the FP32 inner kernels, over the normalisers
+ * |d| and |d| sqrt(Lq) (pi_d2_general).                                      */
 template <bool FAST = false, bool GUARD = false>
 __device__ __forceinline__ void pi_basis(const GridDev& g, double2 lx, double2 ly, double2 lz,
                                          double2 p1[3], double2 p2[3]) {

@@ -243,7 +243,7 @@ static fame_status residuals_planes(fame_ctx* c, int nwant, const double* freq, 
             HIPCHK(fame_launch_transpose(E, c->F64, (int)pn, c->g.na, c->g.na, c->PP, N, c->CS, 3, es, 3 * (size_t)c->CS, nullptr, nk,
                                          c->stream));
         HIPCHK(fame_launch_ana(s, nk, c->stream));
-        HIPCHK(fame_launch_curl(c->kline(8, 0, nullptr), 0, nk, c->stream));
+        HIPCHK(fame_launch_curl(c->kline(8, 0, nullptr), nk, c->stream));
         if (c->g.general) {
             HIPCHK(fame_launch_syn(s, SYN_RES, nk, c->stream));
             HIPCHK(fame_reduce_partials(c->pap_part, 3 * c->g.na, 2, sums + 2 * (size_t)i * nk, nk, c->stream));

@@ -154,10 +154,11 @@ struct fame_ctx {
     bool long_lines(int r) const;
     /* eps_ref (device) into the kernels' layouts */
     fame_status spread_eps();
+    /* blocks per problem whose sums the contracting pass leaves */
     int inner_blocks(int prec) const;
     /* the plane path's inner kernels form alpha and beta themselves */
     bool folds(int prec) const;
-    KLine cg_line(int prec, int p0, bool contract, void* p, void* r, void* x) const;   /* blocks per problem whose sums the contracting pass leaves */
+    KLine cg_line(int prec, int p0, bool contract, void* p, void* r, void* x) const;
     KInner kin(int prec, int p0, const int* act, int list) const;
     KAxis kmid(int prec, int p0, const int* act, int list) const;
     KAxis kout(int prec, int p0, const int* act, int list) const;

@@ -246,7 +246,7 @@ hipError_t fame_prepare_plane64(int eb, int ec);
 hipError_t fame_prepare_syn(int eb, int ec);
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s);
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s);
-hipError_t fame_launch_curl(const KLine& k, int step, int nprob, hipStream_t s);
+hipError_t fame_launch_curl(const KLine& k, int nprob, hipStream_t s);
 /* out = s in^T for `batch` matrices (rows x cols, pitch ip) of each problem, s the
  * square root of scale2[p] (null: 1) */
 hipError_t fame_launch_transpose(const double2* in, double2* out, int rows, int cols, int ip, int op, size_t ib, size_t ob,

@@ -61,9 +61,9 @@ template <> struct C2<float> { typedef float2 T2; };
 
 /* hook bits of a transform: multiply element m of line l, at [m ld + l],
  *   HK_TIN  by tw before the first pass,
- *   HK_EPS  by the real eps before the first pass (and sum <v, eps v>),
- *   HK_TOUT by conj(tw) after the last pass                                  */
-enum { HK_TIN = 1, HK_EPS = 2, HK_TOUT = 4 };
+ *   HK_TOUT by conj(tw) after the last pass
+ * (eps and pap serve the fused middle pass)                                  */
+enum { HK_TIN = 1, HK_TOUT = 2 };
 template <typename T, typename T2>
 struct Hook {
     const T2* tw;
@@ -296,12 +296,6 @@ __device__ __forceinline__ void line_passes(T2* S, int nl, int LS, int ES, CStag
         cur = next;
     }
 #undef LP
-}
-
-/* ordering of LDS accesses between the lanes of one wave */
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 /* Direct DFTs on the matrix cores, the products of dft_mfma (fame_device.hpp):

@@ -628,61 +628,56 @@ __global__ void __launch_bounds__(FFT_THREADS) k_contract(KLine k) {
     }
 }
 
-/* rows c0 .. c0 + nr - 1 of a plane between global memory (contiguous, from G)
- * and LDS (pitch Pb = nb | 1), by the nt threads tid < nt.  nb odd: the LDS rows
- * are as long as the plane's, a linear copy.  FP32: 16 bytes per access (the
- * last one of an odd count covers one element of padding or of the next rows,
- * so it is left out of partial copies with one 8-byte access instead).      */
+/* a plane of n = nb nc elements between global memory (contiguous, from G) and LDS
+ * (pitch Pb = nb | 1).  nb odd: the LDS rows are as long as the plane's, a linear
+ * copy.  FP32: 16 bytes per access, the last element of an odd count by itself */
 template <typename T, typename T2, int U>
-__device__ __forceinline__ void rows_in(T2* S, const T2* G, int nb, int Pb, unsigned mnb, int c0, int nr, int tid, int nt) {
-    const int n = nr * nb, o = c0 * nb;
+__device__ __forceinline__ void rows_in(T2* S, const T2* G, int nb, int Pb, unsigned mnb, int n) {
+    const int tid = threadIdx.x, nt = blockDim.x;
     if constexpr (sizeof(T) == 4) {
-        const int h = o & 1, np = (n - h) >> 1;     /* pairs start at an even offset (16-byte aligned) */
-        const float4* G4 = reinterpret_cast<const float4*>(G + o + h);
+        const int np = n >> 1;
+        const float4* G4 = reinterpret_cast<const float4*>(G);
         for (int i0 = tid; i0 < np; i0 += U * nt) {
             float4 v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) if (i0 + u * nt < np) v[u] = G4[i0 + u * nt];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int i = i0 + u * nt;
-                if (i < np) {
-                    const int e = o + h + 2 * i;
+                const int e = 2 * (i0 + u * nt);
+                if (e < 2 * np) {
                     if (Pb == nb) { *reinterpret_cast<float4*>(S + e) = v[u]; }
                     else { T2* d = S + e + udiv(e, mnb); d[0] = lo2(v[u]); d[1] = hi2(v[u]); }
                 }
             }
         }
-        if (tid == 0 && h) S[o + (Pb == nb ? 0 : udiv(o, mnb))] = G[o];
-        if (tid == 1 && ((n - h) & 1)) { const int e = o + n - 1; S[e + (Pb == nb ? 0 : udiv(e, mnb))] = G[e]; }
+        /* n odd: nb is odd too, and with it the copy linear */
+        if (tid == 0 && (n & 1)) S[n - 1] = G[n - 1];
     } else {
         for (int i0 = tid; i0 < n; i0 += U * nt) {
             T2 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) if (i0 + u * nt < n) v[u] = G[o + i0 + u * nt];
+            for (int u = 0; u < U; ++u) if (i0 + u * nt < n) v[u] = G[i0 + u * nt];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int e = o + i0 + u * nt;
-                if (e < o + n) S[Pb == nb ? e : e + udiv(e, mnb)] = v[u];
+                const int e = i0 + u * nt;
+                if (e < n) S[Pb == nb ? e : e + udiv(e, mnb)] = v[u];
             }
         }
     }
 }
 template <typename T, typename T2>
-__device__ __forceinline__ void rows_out(const T2* S, T2* G, int nb, int Pb, unsigned mnb, int c0, int nr, int tid, int nt) {
-    const int n = nr * nb, o = c0 * nb;
+__device__ __forceinline__ void rows_out(const T2* S, T2* G, int nb, int Pb, unsigned mnb, int n) {
+    const int tid = threadIdx.x, nt = blockDim.x;
     if constexpr (sizeof(T) == 4) {
-        const int h = o & 1, np = (n - h) >> 1;
-        float4* G4 = reinterpret_cast<float4*>(G + o + h);
-        for (int i = tid; i < np; i += nt) {
-            const int e = o + h + 2 * i;
+        float4* G4 = reinterpret_cast<float4*>(G);
+        for (int i = tid; i < n >> 1; i += nt) {
+            const int e = 2 * i;
             if (Pb == nb) G4[i] = *reinterpret_cast<const float4*>(S + e);
             else { const T2* d = S + e + udiv(e, mnb); G4[i] = make_float4(d[0].x, d[0].y, d[1].x, d[1].y); }
         }
-        if (tid == 0 && h) G[o] = S[o + (Pb == nb ? 0 : udiv(o, mnb))];
-        if (tid == 1 && ((n - h) & 1)) { const int e = o + n - 1; G[e] = S[e + (Pb == nb ? 0 : udiv(e, mnb))]; }
+        if (tid == 0 && (n & 1)) G[n - 1] = S[n - 1];
     } else {
-        for (int i = tid; i < n; i += nt) { const int e = o + i; G[e] = S[Pb == nb ? e : e + udiv(e, mnb)]; }
+        for (int i = tid; i < n; i += nt) G[i] = S[Pb == nb ? i : i + udiv(i, mnb)];
     }
 }
 
@@ -716,12 +711,12 @@ __global__ void __launch_bounds__(TB) k_plane(KPlane k) {
     hk.eps = reinterpret_cast<const T*>(k.invB) + po;
     hk.ld = nb;
     hk.pap = k.pap != nullptr;
-    rows_in<T, T2, 4>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
+    rows_in<T, T2, 4>(S, F, nb, Pb, k.mnb, plane);
     line_transform<T, T2, ENGB, true, MAXE>(S, nc, Pb, 1, k.b, Wb);
     double vw = column_round_trip<T, T2, ENGC, MAXE>(S, nb, Pb, k.c, Wc, hk);
     line_transform<T, T2, ENGB, false, MAXE>(S, nc, Pb, 1, k.b, Wb);
     __syncthreads();
-    rows_out<T, T2>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
+    rows_out<T, T2>(S, F, nb, Pb, k.mnb, plane);
     if (hk.pap) {
         __shared__ double red[16];
         for (int o = 32; o > 0; o >>= 1) vw += __shfl_xor(vw, o);

@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(TB) k_syn(KSyn a) {
     Hook<double, T2> hk;
     hk.tw = reinterpret_cast<const T2*>(k.tw) + (size_t)p * plane;
     hk.eps = nullptr; hk.ld = nb; hk.pap = false;
-    rows_in<double, T2, 4>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
+    rows_in<double, T2, 4>(S, F, nb, Pb, k.mnb, plane);
     line_transform<double, T2, ENGB, true, MAXE>(S, nc, Pb, 1, k.b, Wb);
     column_transform<double, T2, ENGC, true, MAXE>(S, nb, Pb, k.c, Wc, hk);
     __syncthreads();
@@ -190,14 +190,13 @@ __global__ void __launch_bounds__(TB) k_ana(KSyn a) {
     column_transform<double, T2, ENGC, false, MAXE>(S, nb, Pb, k.c, Wc, hk);
     line_transform<double, T2, ENGB, false, MAXE>(S, nc, Pb, 1, k.b, Wb);
     __syncthreads();
-    rows_out<double, T2>(S, F, nb, Pb, k.mnb, 0, nc, threadIdx.x, blockDim.x);
+    rows_out<double, T2>(S, F, nb, Pb, k.mnb, plane);
 }
 
 /* the inner axis of the curl-curl operator on the plane layout, in place:
- * conj twiddle, FFT_a, the step on every mode, IFFT_a, twiddle.
- * step 0: -conj(L) x (L x .); step 1: component c times Lambda_c              */
+ * conj twiddle, FFT_a, -conj(L) x (L x .) on every mode, IFFT_a, twiddle       */
 template <int ENG>
-__global__ void __launch_bounds__(FFT_THREADS) k_curl(KLine k, int step) {
+__global__ void __launch_bounds__(FFT_THREADS) k_curl(KLine k) {
     typedef double2 T2;
     const int p = blockIdx.y;
     const int nlines = k.g.nb * k.g.nc, na = k.g.na, L = k.L, P = k.P;
@@ -247,11 +246,6 @@ __global__ void __launch_bounds__(FFT_THREADS) k_curl(KLine k, int step) {
         double2 v[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) v[c] = S[(c * L + line) * P + a];
-        if (step) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) S[(c * L + line) * P + a] = cmul(l[c], v[c]);
-            continue;
-        }
         const double2 u[3] = {fmas2(cmul(l[1], v[2]), l[2], v[1]), fmas2(cmul(l[2], v[0]), l[0], v[2]),
                               fmas2(cmul(l[0], v[1]), l[1], v[0])};
         const double2 n[3] = {make_double2(-l[0].x, l[0].y), make_double2(-l[1].x, l[1].y), make_double2(-l[2].x, l[2].y)};
@@ -414,9 +408,9 @@ static hipError_t launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) 
 }
 hipError_t fame_launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) { return launch_syn(k, mode, nprob, s); }
 hipError_t fame_launch_ana(const KSyn& k, int nprob, hipStream_t s) { return launch_syn(k, 4, nprob, s); }
-hipError_t fame_launch_curl(const KLine& k, int step, int nprob, hipStream_t s) {
+hipError_t fame_launch_curl(const KLine& k, int nprob, hipStream_t s) {
     KLine q = k;
-    void* arg[] = {&q, &step};
+    void* arg[] = {&q};
     return hipLaunchKernel(k.a.eng == ENG_MFMA ? (const void*)k_curl<ENG_MFMA> : (const void*)k_curl<ENG_STOCKHAM>,
                            dim3(xcd_round((k.g.nb * k.g.nc + k.L - 1) / k.L), nprob), dim3(FFT_THREADS), arg,
                            fame_line_lds2(k.g.na, k.a.ntab, k.L, k.P, 8), s);

@@ -490,7 +490,6 @@ KLine fame_ctx::kline(int prec, int p0, const int* act, bool contract) const {
     const PassTile& t = contract ? ctile[pi] : ltile[pi];
     k.g = g; k.prob = prob_d + p0; k.active = act;
     k.a = laxis[pi][t.eng];
-    k.a.mnl = fame_magic32(3 * t.L);
     k.lt = ltab + nl * p0;
     k.tw = (char*)ltw[pi] + es * nl * inner_tw_per_line(g.na) * p0;
     k.ea = eatab;
