@@ -1163,16 +1163,16 @@ fame_status fame_ctx::tune(int prec) {
     /* Pr, Prs and the check of the factorisation run by FP64 axis passes on every
      * grid, one problem at a time (Pr on SC 64: 83 us with the start tiles, 60
      * tuned).  Where nothing else does, only tiles that leave one problem many blocks
-     * are tried, twice each (32^3: 0.9 ms of tuning instead of 3.2)             */
+     * are tried, twice each (32^3: 0.7 ms of tuning instead of 3.2)             */
     const int nt_prob = axis_too ? nk : 1, reps = axis_too ? 3 : 2;
-    static const int candL_few[] = {2, 4, 6, 8, 16};
+    static const int few_inner[] = {2, 4, 6}, few_axis[] = {4, 8, 16};
     for (int a = 0; a < 3 && st == FAME_OK && (axis_too || prec == 8); ++a) {
         PassTile best = tile[a][pi];
         float best_ms = 1e30f;
         for (int eng = 0; eng < 2; ++eng) {
             if (ax[a][eng].n == 0 || (eng_forced >= 0 && eng != eng_forced)) continue;
-            const int* cl = axis_too ? (a == AX_INNER ? candL_inner : candL_axis) : candL_few + (a == AX_INNER ? 0 : 1);
-            const int ncl = axis_too ? (a == AX_INNER ? 10 : 7) : 4;
+            const int* cl = a == AX_INNER ? (axis_too ? candL_inner : few_inner) : (axis_too ? candL_axis : few_axis);
+            const int ncl = axis_too ? (a == AX_INNER ? 10 : 7) : 3;
             for (int ci = 0; ci < ncl; ++ci) {
                 const int L = cl[ci];
                 if (!tile_ok(ax[a][eng], a, prec, L, g)) continue;
