@@ -419,10 +419,12 @@ fame_status fame_ctx::plane_setup() {
         KPlane& k = kpl[pi];
         std::memset(&k, 0, sizeof(k));
         /* 8 to 24 points: the direct DFT on the matrix cores: one step between
-         * barriers instead of two or three passes.  The plane kernel of a 16^3 grid,
-         * one wave vector, 11.3 -> 8.7 us in FP64 (10.7 -> 8.1 in FP32), 24^3 12.2
-         * -> 10.6 (12.5 -> 9.4), eight 24^3 16.9 -> 15.4; from 32^3 on the passes
-         * win (eight in FP64 20.8 against 29.1)                               */
+         * barriers instead of two or three passes.  Plane kernel of n^3 grids, us,
+         * direct / passes: FP64 one problem 16 7.1/9.5, 20 8.5/10.1, 24 9.2/10.7, eight
+         * 16 8.3/16.7, 20 10.3/12.0, 24 13.4/14.7; FP32 24 8.2/10.8, eight 9.7/13.0.
+         * Above: 25 9.1/10.3, 26 9.4/16.8, 28 10.4/11.5, 30 10.6/13.6, eight 16.8/28.5
+         * (one output tile still: the line could lie at 31); 32 11.7/11.6, eight
+         * 25.0/17.8, 36 16.0/14.7, eight 45.5/35.5                             */
         auto engine = [&](int axis) {
             return (ax[axis][0].blue || eng_forced == 1 || (eng_forced < 0 && ax[axis][1].n >= 8 && ax[axis][1].n <= 24)) ? ENG_MFMA : ENG_STOCKHAM;
         };
