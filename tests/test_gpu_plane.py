@@ -1,7 +1,8 @@
 """The plane path of the QBQ (the two outer axes in one pass over (b, c) planes in
 LDS) against the FP64 oracle, at the sizes where its kernels can go wrong: odd and
 even rows (linear or padded LDS rows), odd planes (padding of the plane pitch),
-one-, two- and three-pass axes, direct DFTs on the matrix cores along every axis,
+direct DFTs on the matrix cores along every axis (plane axes of 8 to 24 points and
+prime ones; the radix passes of longer composite axes are in test_gpu_plane_passes),
 line counts that leave the last block of the inner kernels ragged, Gamma, and every
 lines-per-block and thread count its rule accepts.  Both precisions hold the bars of
 the axis passes: 1e-11 of the oracle in FP64, 2e-6 in FP32, 1e-8 in lambda for an
@@ -17,9 +18,9 @@ pytestmark = pytest.mark.gpu
 
 O.set_threads(8)
 
-# grid sides (a, b, c) reached: 9^3 (one radix per axis), 16^3 (one FP32 pass), 17^3 (direct DFT on
-# all axes), 18^3, 26^3 (13 x 2), 34^3 (2 x 17: direct), FCC 22x19x18, 41x36x33 (c = 41 direct),
-# BCC 17x16x13, hexagonal 31x26x22 and 16x13x11
+# grid sides (a, b, c) reached: 9^3, 16^3, 17^3, 18^3 (direct DFTs along b and c), 26^3 (13 x 2 passes),
+# 34^3 (2 x 17: direct), FCC 22x19x18, 41x36x33 (c = 41 direct, b = 36 passes), BCC 17x16x13,
+# hexagonal 31x26x22 and 16x13x11
 GRIDS = [("simple_cubic", 9), ("simple_cubic", 16), ("simple_cubic", 17), ("simple_cubic", 18), ("simple_cubic", 26),
          ("simple_cubic", 34), ("face_centered_cubic", 22), ("face_centered_cubic", 41), ("body_centered_cubic", 17),
          ("hexagonal", 31), ("hexagonal", 16)]
