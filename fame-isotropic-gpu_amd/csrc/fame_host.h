@@ -125,6 +125,8 @@ struct fame_ctx {
     int kid_nk = 0;
     int eps_ver = 0, k_ver = 0, kids_eps_ver = -1, kids_k_ver = -1;
     int gram_batch = 0;
+    /* problems of the batch that this context solves, or a group of */
+    int whole_batch() const { return gram_batch > 0 ? gram_batch : nk; }
     int out_pmul = 1;
     long long cnt_qbq64 = 0, cnt_qbq32 = 0;
     int last_iters = 0;

@@ -187,6 +187,7 @@ struct KSyn {
     size_t ostride;              /* problem stride of in / out / E              */
     double* part;                /* SYN_EPS: |E|^2 per block; SYN_RES: |r|^2, |E|^2 per block */
     int w2step;
+    int batch;                   /* problems by which the block size is chosen: the sums' order (0: the launch's) */
 };
 
 struct KAxis {

@@ -76,7 +76,7 @@ fame_status lz_alloc(fame_ctx* c, LzBuffers& b, int nk, int nstep, int nwant) {
     b.n2 = 2 * (size_t)c->N; b.nk = nk; b.nstep = nstep; b.nwant = nwant;
     b.ls_time.assign(nk, 0.0);
     const size_t m = nstep + 1;
-    const size_t gp = std::max((size_t)GEMV_BLK_GS * 2 * m, (size_t)gram_blk(c->gram_batch > 0 ? c->gram_batch : nk) * 2 * m * m);
+    const size_t gp = std::max((size_t)GEMV_BLK_GS * 2 * m, (size_t)gram_blk(c->whole_batch()) * 2 * m * m);
     void** ptr[] = {(void**)&b.U, (void**)&b.W, (void**)&b.T0d, (void**)&b.T1d, (void**)&b.hdot, (void**)&b.h,
                     (void**)&b.hh, (void**)&b.nrm, (void**)&b.invb, (void**)&b.gpart, (void**)&b.G, (void**)&b.Q,
                     (void**)&b.mask, (void**)&b.mask2};
@@ -537,7 +537,7 @@ extern "C" fame_status fame_eigs_impl(fame_ctx* c, int precision, const fame_es*
         /* Gram matrices of the bases that restart */
         HIPCHK(hipMemcpyAsync(b.mask, rmask.data(), sizeof(int) * nk, hipMemcpyHostToDevice, c->stream));
         const size_t ps = b.n2 * m;
-        const int gblk = gram_blk(c->gram_batch > 0 ? c->gram_batch : nk);
+        const int gblk = gram_blk(c->whole_batch());
         HIPCHK(fame_gram(b.U, b.gpart, gblk, m, b.n2, b.n2, ps, nk, b.mask, c->stream));
         HIPCHK(fame_reduce_partials(b.gpart, gblk, 2 * m * m, b.G, nk, c->stream));
         HIPCHK(hipMemcpyAsync(G.data(), b.G, sizeof(double) * 2 * m * m * nk, hipMemcpyDeviceToHost, c->stream));
@@ -652,6 +652,7 @@ static fame_status restore_band(fame_ctx* c, int i, int nwant, const double2* ev
         HIPCHK(c->launch_line(k, 1, LINE_EX_PLAIN, 8, nk));
         KSyn s = c->ksyn(0);
         s.part = c->pap_part;
+        s.batch = c->whole_batch();
         HIPCHK(fame_launch_syn(s, SYN_EPS, nk, c->stream));
         HIPCHK(fame_reduce_partials(c->pap_part, 3 * c->g.na, 1, c->scal, nk, c->stream));
         const size_t os = (size_t)c->out_pmul * nwant * N3, pn = (size_t)c->g.nb * c->g.nc;

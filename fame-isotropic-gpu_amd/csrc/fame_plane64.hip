@@ -402,7 +402,7 @@ static hipError_t launch_syn(const KSyn& k, int mode, int nprob, hipStream_t s) 
     KSyn q = k;
     void* arg[] = {&q};
     const size_t lds = fame_plane_lds(k.k.b.n, k.k.c.n, k.k.b.ntab + k.k.c.ntab, 8);
-    const int nt = lds <= FAME_LDS_HALF && k.k.wide && 3 * k.k.g.na * nprob > 512 ? 256 : 512;
+    const int nt = lds <= FAME_LDS_HALF && k.k.wide && 3 * k.k.g.na * (k.batch ? k.batch : nprob) > 512 ? 256 : 512;
     return hipLaunchKernel(k.k.wide ? syn_fn<512>(k.k.b.eng, k.k.c.eng, mode) : syn_fn<1024>(k.k.b.eng, k.k.c.eng, mode),
                            dim3(xcd_round(3 * k.k.g.na), nprob), dim3(nt), arg, lds, s);
 }

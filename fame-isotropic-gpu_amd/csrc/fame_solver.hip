@@ -544,7 +544,7 @@ bool fame_ctx::one_way_planes(bool analysis) const {
  * 12 sixteen 790/640, four 300/350; 200 x 6 x 6 64 1020/1180; restoration 400 x 4 x 4
  * sixteen 450/420, 64 1570/1060; 400 x 6 x 6 sixteen 360/450                    */
 bool fame_ctx::long_lines(int r) const {
-    return g.na > 256 && g.na * g.na > r * g.nb * g.nc && 3 * g.na * nk > 12000;
+    return g.na > 256 && g.na * g.na > r * g.nb * g.nc && 3 * g.na * whole_batch() > 12000;
 }
 int fame_ctx::inner_blocks(int prec) const {
     const int pi = prec == 8 ? 0 : 1;
